@@ -12,17 +12,17 @@ A step is one complete 256-spp render into device-resident films (scene, BVH
 and films already in HBM; parse + BVH build + upload are reported separately as
 load_s).  value = width * height * spp * steps / timed wall time.
 
-The roofline object covers the dominant kernel (pt_extend, the closest-hit
-traversal): its algorithmic bytes per launch are the canonical per-ray bytes
-(64 B per BVH2 node visit + 48 B per triangle test, counted by the CPU
-oracle's binned-SAH BVH2 over 2^16 paths) plus the 52 B of queue/ray/hit
+The roofline object covers the dominant kernel (pt_trace, the traversal of
+extension and shadow rays): its algorithmic bytes per launch are the canonical
+per-ray bytes (64 B per BVH2 node visit + 48 B per triangle test, counted by
+the CPU oracle's binned-SAH BVH2 over 2^16 paths) plus the 48 B of ray and hit
 records each ray moves, times the rays one launch processes; divided by the
 launch's average duration from HIP events on the library's stream.
 
 cpu_baseline: the oracle (the project's C++ restatement of the reference path
 tracer) timed on the host on 48 passes (48 spp) of the same 1024x1024 workload.
 
-roofline.traffic: HBM bytes per pt_extend launch measured by rocprofv3
+roofline.traffic: HBM bytes per pt_trace launch measured by rocprofv3
 FETCH_SIZE and WRITE_SIZE runs, scaled by the factor the same counters read
 for a plain copy of known size (--copy-calibration); read from the committed
 summary in profiles/ when present.
@@ -46,8 +46,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "pt_extend_ggx_grid_1024_traffic.md")
-STATE_BYTES_PER_RAY = 52  # queue index 4 + ray origin/direction 32 + hit record 16
+TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "pt_trace_ggx_grid_1024_traffic.md")
+STATE_BYTES_PER_RAY = 48  # ray origin/direction 32 + hit record (or radiance to add) 16
 
 
 def log(msg):
@@ -162,7 +162,7 @@ def sppm_cpu_baseline(job_path, args):
 
 
 def measured_traffic():
-    """HBM bytes per pt_extend launch from the committed rocprofv3 summary
+    """HBM bytes per pt_trace launch from the committed rocprofv3 summary
     (line 'traffic_bytes_per_launch: N'), or None.  rocprofv3 counters need a
     run of their own, so this figure comes from the profiles/ summary of an
     earlier counter run of the same command, not from this run; the bench line
@@ -658,7 +658,7 @@ def main():
         render()
         log("warmup %d: %.3f s" % (i, time.perf_counter() - t))
 
-    # timed steps: HIP events around the extension launches only (the
+    # timed steps: HIP events around the traversal launches only (the
     # roofline's kernel), so that the events of the other launches add
     # nothing to the timed region
     scene.reset_stats()
@@ -696,13 +696,13 @@ def main():
         log("cpu baseline %.4g paths/s" % base["value"])
 
     roofline = None
-    launches, ext_ms = kstats_timed.get("pt_extend", (0, 0.0))
+    launches, trace_ms = kstats_timed.get("pt_trace", (0, 0.0))
     if canon and launches:
         b_ray = (64.0 * canon["node_visits"] + 48.0 * canon["tri_tests"]) / canon["rays"]
-        ext_rays_per_render = counters["extension_rays"]
-        rays_per_launch = ext_rays_per_render / (launches / args.steps)
+        rays_per_render = counters["extension_rays"] + counters["shadow_rays"]
+        rays_per_launch = rays_per_render / (launches / args.steps)
         bytes_per_launch = rays_per_launch * (b_ray + STATE_BYTES_PER_RAY)
-        avg_s = ext_ms / launches / 1e3
+        avg_s = trace_ms / launches / 1e3
         achieved = bytes_per_launch / avg_s / 1e9
         roofline = {
             "bound": "hbm",
@@ -712,8 +712,8 @@ def main():
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": measured_traffic(),
             "traffic_source": "rocprofv3 FETCH_SIZE/WRITE_SIZE of an earlier run of this command, read from "
-                              "profiles/pt_extend_ggx_grid_1024_traffic.md (not measured in this run)",
-            "kernel": "pt_extend",
+                              "profiles/pt_trace_ggx_grid_1024_traffic.md (not measured in this run)",
+            "kernel": "pt_trace",
             "bytes_per_ray_canonical": round(b_ray, 1),
             "rays_per_launch": round(rays_per_launch, 1),
             "avg_launch_ms": round(avg_s * 1e3, 4),
@@ -742,7 +742,7 @@ def main():
             "environment": "2048x1024 lat-long, importance sampled",
             "camera": "thin lens f/2.8, 8 blades",
             "launch": tuned,
-            # the timed steps record HIP events around the extension launches,
+            # the timed steps record HIP events around the traversal launches,
             # and a render with events launches eagerly (no hipGraph replay)
             "launch_timed": dict(tuned, use_graph=0),
             "parallelism": "single-gpu",

@@ -580,7 +580,7 @@ class Scene:
         _err(lib().hasty_trace_hits_device_noalloc(self._h, C.c_void_p(d_rays), n, C.c_void_p(d_hits)))
 
     def set_profiling(self, events=True, counters=False, extend_only=False):
-        """HIP-event timing of every launch (of the extension launches only
+        """HIP-event timing of every launch (of the traversal launches only
         with extend_only) and/or device counters."""
         _err(lib().hasty_set_profiling(self._h, (1 if events else 0) | (2 if counters else 0) |
                                        (4 if extend_only else 0)))

@@ -185,7 +185,9 @@ struct HastyScene {
   // path buffers
   hasty::PathBuffers pb{};
   std::vector<void*> pathAllocs;
-  uint32_t pathCapacity = 0;
+  uint32_t poolCapacity = 0, poolRing = 0;  // allocated paths and ring entries
+  uint32_t poolMost = 0xFFFFFFFFu, ringMost = 0xFFFFFFFFu;  // what an allocation failed above
+  static constexpr uint32_t kDefaultSlots = 1u << 24;
   uint32_t slotsWanted = 0;  // 0 = automatic
   uint32_t* dTileOrder = nullptr;
   uint32_t tileW = 0, tileH = 0;
@@ -216,12 +218,12 @@ struct HastyScene {
   float guidePhotonShare = 0.5f;   // their samples' weight sum / the camera samples'
   uint32_t guidePhotonPass = 0;    // light-path pass counter (random streams)
   uint32_t lastGuidePhotonSamples = 0;
-  float4* guideRaw = nullptr;
-  float4* guideRec = nullptr;
-  float* guideSel = nullptr;  // per slot: learned selection probability
+  DevBuf guideRaw;    // mixture tables of the paths alive
+  DevBuf guideSel;    // their learned selection probabilities
+  DevBuf guideRec;    // training records by path of a call
+  DevBuf guideEnded;  // paths that ended at a bounce with records
   float4* guideSamples = nullptr;
   uint32_t* guideCount = nullptr;
-  uint32_t guideSlots = 0;
   static constexpr uint32_t kGuideSampleCap = 1u << 21;
   static constexpr uint64_t kGuideTrainPaths = 1u << 20;  // paths per online training step
   float lastGuideLoss = 0.0f;
@@ -252,7 +254,8 @@ struct HastyScene {
   void freePath() {
     for (void* p : pathAllocs) (void)hipFree(p);
     pathAllocs.clear();
-    pathCapacity = 0;
+    pb = hasty::PathBuffers{};
+    poolCapacity = poolRing = 0;
   }
   ~HastyScene() {
     if (timer) timer->collect();
@@ -263,7 +266,7 @@ struct HastyScene {
     }
     for (void* p : sceneAllocs) (void)hipFree(p);
     if (dTileOrder) (void)hipFree(dTileOrder);
-    for (void* p : {(void*)guideRaw, (void*)guideRec, (void*)guideSel, (void*)guideSamples, (void*)guideCount})
+    for (void* p : {(void*)guideSamples, (void*)guideCount})
       if (p) (void)hipFree(p);
     if (dFilm) (void)hipFree(dFilm);
     if (traceOverflow) (void)hipFree(traceOverflow);
@@ -280,60 +283,88 @@ struct HastyScene {
     dev.height = st.height;
   }
 
-  // Path slots in flight (regenerated as paths end) and the results ring.
-  // Slots for a render of `paths` paths: the wanted pool (default 2^23), but
-  // no more than the render needs (at least 2^16).
-  uint32_t slotCount(uint64_t paths = 0) const {
-    if (paths == 0) paths = (uint64_t)dev.width * dev.height;
-    uint64_t want = slotsWanted ? slotsWanted : (1ull << 23);
+  // Paths in flight (a path that ends makes room for the next) of a render of
+  // `paths` paths: the wanted pool (default 2^24), but no more than the
+  // render needs (at least 2^16).  Larger pools spread a bounce's fixed costs
+  // (the tail of its longest rays) over more rays: 132 ms at 2^22, 129 at
+  // 2^23, 125 at 2^24, 122 at 2^25 for 128 samples of the 1024x1024 GGX grid.
+  uint32_t slotCount(uint64_t paths) const {
+    uint64_t want = slotsWanted ? slotsWanted : kDefaultSlots;
     return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(want, std::max<uint64_t>(paths, 1ull << 16)));
   }
-  uint32_t ringPathsWanted() const {
-    uint64_t P = (uint64_t)dev.width * dev.height;
-    uint64_t r = std::max<uint64_t>(P, (uint64_t)(1u << 26) / P * P);  // about 64M paths, whole samples
-    return (uint32_t)std::min<uint64_t>(r, 0x7FFFFFFFull / P * P);
+  // Results ring: the whole render if it is no more than about 2^27 paths
+  // (finished paths wait in the ring for the oldest one in flight, so a ring
+  // much longer than a pool x depth never holds a path's start up), else
+  // whole samples of this scene's film.
+  uint32_t ringPathsWanted(uint64_t paths) const {
+    const uint64_t P = (uint64_t)dev.width * dev.height, most = 1ull << 27;
+    if (paths <= std::max(P, most)) return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(paths, 1), 0x7FFFFFFFull);
+    return (uint32_t)std::min<uint64_t>(std::max(P, most / P * P), 0x7FFFFFFFull / P * P);
   }
 
-  void ensurePathBuffers(uint64_t paths = 0) {
-    uint32_t need = slotCount(paths);
-    uint32_t ring = ringPathsWanted();
-    uint32_t traceThreads = launch.traceBlocks * hasty::kBlock;
-    if (need == pathCapacity && ring == pb.ringPaths && pb.traceThreads == traceThreads) return;
+  // Buffers of a render call; grown when a call needs more, else kept (a call
+  // that needs less uses a part).  A pool or ring that does not fit the free
+  // memory is halved until it does.
+  void ensurePathBuffers(uint64_t paths, bool late, bool textured) {
+    const uint32_t need = std::min(slotCount(paths), poolMost);
+    const uint64_t P = (uint64_t)dev.width * dev.height;
+    const uint32_t ring = (uint32_t)std::min<uint64_t>(ringPathsWanted(paths), std::max<uint64_t>(ringMost, P));
+    const uint32_t traceThreads = launch.traceBlocks * hasty::kBlock;
+    const bool fits = need <= poolCapacity && ring <= poolRing && traceThreads <= pb.traceThreads &&
+                      (!late || pb.sh.lateQ) && (!textured || pb.set[0].mediaTx);
+    if (!fits) {
+      uint32_t n = std::max(need, poolCapacity), r = std::max(ring, poolRing);
+      late = late || pb.sh.lateQ;
+      textured = textured || pb.set[0].mediaTx;
+      const uint32_t tt = std::max(traceThreads, pb.traceThreads);
+      for (;;) {
+        try {
+          allocPool(n, r, tt, late, textured);
+          break;
+        } catch (const std::exception&) {
+          freePath();
+          (void)hipGetLastError();  // the failed allocation's
+          if (n <= (1u << 20) && r <= std::max<uint64_t>(P, 1u << 20)) throw;
+          if (n > (1u << 20)) poolMost = n = n / 2;
+          if (r > std::max<uint64_t>(P, 1u << 20)) ringMost = r = (uint32_t)std::max<uint64_t>(P, r / 2);
+        }
+      }
+    }
+    pb.capacity = std::min(need, poolCapacity);
+    pb.ringPaths = std::min(ring, poolRing);
+  }
+  void allocPool(uint32_t n, uint32_t r, uint32_t traceThreads, bool late, bool textured) {
     freePath();
-    size_t n = need;
-    pb.rayO = allocPath<float4>(n);
-    pb.rayD = allocPath<float4>(n);
+    for (hasty::PathSet& ps : pb.set) {
+      ps.rayO = allocPath<float4>(n);
+      ps.rayD = allocPath<float4>(n);
+      ps.beta = allocPath<float4>(n);
+      ps.L = allocPath<float4>(n);
+      ps.state = allocPath<uint4>(n);
+      ps.media = allocPath<uint4>(2 * (size_t)n);
+      if (textured) ps.mediaTx = allocPath<uint32_t>((size_t)hdev::kMaxMedia * n);
+    }
     pb.hit = allocPath<float4>(n);
-    pb.beta = allocPath<float4>(n);
-    pb.L = allocPath<float4>(n);
-    pb.state = allocPath<uint4>(n);
-    pb.media = allocPath<uint4>(2 * n);
-    pb.mediaTx = allocPath<uint32_t>((size_t)hdev::kMaxMedia * n);
-    pb.auxN = allocPath<float4>(n);
-    pb.auxA = allocPath<float4>(n);
-    pb.shO = allocPath<float4>(n);
-    pb.shD = allocPath<float4>(n);
-    pb.shFD = allocPath<float4>(n);
-    pb.shFC = allocPath<float4>(n);
-    pb.shThr = allocPath<float4>(n);
-    pb.shBeta = allocPath<float4>(n);
-    pb.shT = allocPath<float4>(n);
-    pb.qA = allocPath<uint32_t>(n);
-    pb.qB = allocPath<uint32_t>(n);
-    pb.qS = allocPath<uint32_t>(n);
-    pb.qR = allocPath<uint32_t>(n);
-    pb.mark = allocPath<uint32_t>(n);
+    pb.sh.q = allocPath<uint2>(n);
+    pb.sh.o = allocPath<float4>(n);
+    pb.sh.d = allocPath<float4>(n);
+    pb.sh.c = allocPath<float4>(n);
+    pb.sh.job = allocPath<uint32_t>(n);
+    if (late) {
+      for (float4** a : {&pb.sh.lateFD, &pb.sh.lateFC, &pb.sh.lateThr, &pb.sh.lateBeta, &pb.sh.lateT, &pb.sh.lateHit})
+        *a = allocPath<float4>(n);
+      pb.sh.lateQ = allocPath<uint2>(n);
+    }
     pb.counters = allocPath<uint32_t>(hasty::kNumCounters);
     pb.stats = allocPath<unsigned long long>(hasty::kNumStats);
     pb.stackOverflow = allocPath<uint2>((size_t)traceThreads * hasty::kStackOvf);
-    pb.ringL = allocPath<float4>(ring);
-    pb.ringN = allocPath<float4>(ring);
-    pb.ringA = allocPath<float4>(ring);
-    pb.ringPaths = ring;
+    pb.ringL = allocPath<float4>(r);
+    pb.ringN = allocPath<float4>(r);
+    pb.ringA = allocPath<float4>(r);
     pb.traceThreads = traceThreads;
-    pb.capacity = need;
-    pathCapacity = need;
     HIPCHECK(hipMemset(pb.stats, 0, sizeof(unsigned long long) * hasty::kNumStats));
+    poolCapacity = n;
+    poolRing = r;
   }
 
   void ensureTileOrder() {
@@ -424,9 +455,14 @@ static void renderBatch(HastyScene* owner, const BatchItem* items, uint32_t nIte
     return;
   }
   uint64_t allPaths = 0;
-  for (uint32_t i = 0; i < nItems; ++i)
-    allPaths += (uint64_t)items[i].n * items[i].scene->dev.width * items[i].scene->dev.height;
-  owner->ensurePathBuffers(allPaths);
+  bool late = false, textured = false;
+  for (uint32_t i = 0; i < nItems; ++i) {
+    const hdev::DevScene& d = items[i].scene->dev;
+    allPaths += (uint64_t)items[i].n * d.width * d.height;
+    late = late || (d.hasEnv && d.hasSurfaceLight);
+    textured = textured || d.texturedMedia;
+  }
+  owner->ensurePathBuffers(allPaths, late, textured);
   // Split every item into calls of < 2^31 paths and lay out all Halton
   // offsets in one upload to the owner's offset buffer.
   struct Piece {
@@ -533,44 +569,36 @@ struct HastySppm {
 // minibatches, and at least one step per sample index of the group.  Without
 // training: every index in one call.
 static void renderGuided(HastyScene* s, const BatchItem& it) {
-  s->ensurePathBuffers((uint64_t)it.n * s->dev.width * s->dev.height);
+  const uint64_t P = (uint64_t)s->dev.width * s->dev.height;
+  // Without training no radiance samples are recorded.
+  const bool training = s->guideLr > 0.0f;
+  const uint64_t groupPaths = training ? HastyScene::kGuideTrainPaths : 0x7FFFFFFFull;
+  const uint32_t perCall = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(it.n, groupPaths / P));
+  s->ensurePathBuffers(perCall * P, s->dev.hasEnv && s->dev.hasSurfaceLight, s->dev.texturedMedia != 0);
   s->ensureTileOrder();
-  uint32_t slots = s->pb.capacity;
-  if (s->guideSlots != slots) {
-    for (void* p : {(void*)s->guideRaw, (void*)s->guideRec, (void*)s->guideSel})
-      if (p) (void)hipFree(p);
-    s->guideRaw = nullptr, s->guideRec = nullptr, s->guideSel = nullptr;
-    s->guideSlots = 0;
-    HIPCHECK(hipMalloc(&s->guideRaw, sizeof(float4) * 10 * (size_t)slots));
-    HIPCHECK(hipMalloc(&s->guideRec, sizeof(float4) * 12 * (size_t)slots));
-    s->guideSlots = slots;
-  }
-  if (s->guide->g->learnedSelection() && !s->guideSel) {
-    HIPCHECK(hipMalloc(&s->guideSel, sizeof(float) * (size_t)slots));
-  }
+  const size_t slots = s->pb.capacity;
+  float4* raw = (float4*)s->guideRaw.ensure(sizeof(float4) * 10 * slots);
+  float* sel = s->guide->g->learnedSelection() ? (float*)s->guideSel.ensure(sizeof(float) * slots) : nullptr;
+  float4* rec = training ? (float4*)s->guideRec.ensure(sizeof(float4) * 12 * (size_t)perCall * P) : nullptr;
+  s->pb.ended = training ? (uint2*)s->guideEnded.ensure(sizeof(uint2) * slots) : nullptr;
   if (!s->guideSamples) {
     HIPCHECK(hipMalloc(&s->guideSamples, sizeof(float4) * 4 * (size_t)HastyScene::kGuideSampleCap));
     HIPCHECK(hipMalloc(&s->guideCount, sizeof(uint32_t)));
   }
   hasty::GuideRun gr;
   gr.net = s->guide->g->net();
-  gr.raw = s->guideRaw;
-  gr.rec = s->guideRec;
+  gr.raw = raw;
+  gr.rec = rec;
   gr.samples = s->guideSamples;
   gr.sampleCount = s->guideCount;
-  // Without training no radiance samples are recorded.
-  const bool training = s->guideLr > 0.0f;
   gr.sampleCap = training ? HastyScene::kGuideSampleCap : 0u;
   gr.fraction = s->guideFraction;
-  gr.sel = s->guide->g->learnedSelection() ? s->guideSel : nullptr;
+  gr.sel = sel;
   gr.maxDepth = s->guideMaxDepth;
   gr.maxThroughput = s->guideMaxThroughput;
   s->launch.countStats = s->counting;
   if (s->profiling && !s->timer) s->timer = std::make_unique<EventTimer>();
   hasty::KernelTimer* timer = s->profiling ? s->timer.get() : nullptr;
-  const uint64_t P = (uint64_t)s->dev.width * s->dev.height;
-  const uint64_t groupPaths = training ? HastyScene::kGuideTrainPaths : 0x7FFFFFFFull;
-  const uint32_t perCall = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(it.n, groupPaths / P));
   float2* dOff = (float2*)s->offsets.ensure(sizeof(float2) * perCall);
   for (uint32_t k = 0; k < it.n; k += perCall) {
     const uint32_t cnt = std::min(perCall, it.n - k);
@@ -1356,7 +1384,7 @@ int hasty_set_profiling(HastyScene* s, int flags) {
   s->counting = (flags & 2) != 0;
   if (s->profiling) {
     if (!s->timer) s->timer = std::make_unique<EventTimer>();
-    s->timer->only = (flags & 4) != 0 ? hasty::kKExtend : -1;
+    s->timer->only = (flags & 4) != 0 ? hasty::kKTrace : -1;
   }
   return 0;
 }
@@ -1417,7 +1445,7 @@ int hasty_get_launch(const HastyScene* s, HastyLaunch* out) {
     g_lastError = "null argument";
     return 1;
   }
-  out->path_slots = s->slotsWanted ? s->slotsWanted : (1u << 23);
+  out->path_slots = s->slotsWanted ? s->slotsWanted : HastyScene::kDefaultSlots;
   out->trace_blocks = s->launch.traceBlocks;
   out->shade_blocks = s->launch.shadeBlocks;
   out->chunk = s->launch.chunk;

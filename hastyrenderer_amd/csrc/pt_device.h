@@ -1110,18 +1110,25 @@ __device__ inline V3 envLookup(const DevScene& s, float u, float v) {
   if (col > (int)s.envW - 1) col = (int)s.envW - 1;
   return load3g(s.envRGB + ((size_t)row * s.envW + col) * 3);
 }
+// Environment coordinates of a direction: its radiance and its sampling
+// density share them (an acos and an atan2 in double precision).
+struct EnvUV {
+  float u, v, theta;
+};
+__device__ inline EnvUV envUV(V3 dir) {
+  float th, ph;
+  sphericalFromDir(dir, &th, &ph);
+  return EnvUV{ph * (float)(0.5 * kInvPi), 1.0f - th * (float)kInvPi, th};
+}
 __device__ inline V3 evalEnvironment(const DevScene& s, V3 dir) {  // Scene.cpp:482-485
   if (!s.hasEnv) return v3(s.bg[0], s.bg[1], s.bg[2]);
-  float th, ph;
-  sphericalFromDir(dir, &th, &ph);
-  return envLookup(s, ph * (float)(0.5 * kInvPi), 1.0f - th * (float)kInvPi);
+  const EnvUV e = envUV(dir);
+  return envLookup(s, e.u, e.v);
 }
 // ImageDistribution::evalDensity / EnvironmentTexture::evalSamplingDensity
-__device__ inline float envPdf(const DevScene& s, V3 dir) {
-  float th, ph;
-  sphericalFromDir(dir, &th, &ph);
-  float u = ph * (float)(0.5 * kInvPi), v = 1.0f - th * (float)kInvPi;
-  float sinT = hm::sinf(th);
+__device__ inline float envPdf(const DevScene& s, EnvUV e) {
+  float u = e.u, v = e.v;
+  float sinT = hm::sinf(e.theta);
   float W = (float)s.envW, H = (float)s.envH;
   if (u != u || v != v) return 0.0f / fmaxf(1e-7f, 2.0f * (float)(kPi * kPi) * sinT);
   float fx = u * s.envW, fy = (1.0f - v) * s.envH;
@@ -1130,6 +1137,7 @@ __device__ inline float envPdf(const DevScene& s, V3 dir) {
   float d = W * H * s.envPdf[(size_t)y * s.envW + x] / s.envValueSum;
   return d / fmaxf(1e-7f, 2.0f * (float)(kPi * kPi) * sinT);
 }
+__device__ inline float envPdf(const DevScene& s, V3 dir) { return envPdf(s, envUV(dir)); }
 // upper_bound over the environment CDF, narrowed by a guide table:
 // guide[g] = upper_bound(cdf, g / kEnvGuide), so for x in [g, g + 1) / kEnvGuide
 // the answer lies in [guide[g], guide[g + 1]] (upper_bound is monotone) and

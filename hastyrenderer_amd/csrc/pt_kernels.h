@@ -10,34 +10,54 @@
 
 namespace hasty {
 
-// Structure-of-arrays path state for `capacity` path slots.  Slots are
-// recycled: when a path ends its radiance goes to the results ring and the
-// slot starts the next path of the render (regeneration), so every stage
-// keeps a full queue until the last paths of a render drain.  Queues hold
-// slot indices.
-struct PathBuffers {
+// Path state, structure of arrays, of the paths alive at one bounce, packed
+// at [0, n).  There are two sets: a bounce reads one and writes the paths that
+// go on (and then the paths that start) to the other, so every access of
+// every stage is to consecutive records whatever ended in between.
+struct PathSet {
   float4* rayO;   // origin; w unused
   float4* rayD;   // direction; w = pdf of the BSDF sample that produced it
-  float4* hit;    // t, u, v, triangle (bits)
-  float4* beta;   // path throughput
-  float4* L;      // accumulated radiance
+  float4* beta;   // path throughput (not stored for paths that start)
+  float4* L;      // accumulated radiance (not stored for paths that start)
   uint4* state;   // x rng draws, y flags, z previous triangle, w path id
-  uint4* media;   // 2 x uint4 per slot (8 entries)
-  uint32_t* mediaTx;  // 8 per slot: albedo texel of each media entry
-  float4* auxN;   // depth-0 shading normal
-  float4* auxA;   // depth-0 albedo
-  float4* shO;    // shadow origin; w = BSDF pdf of the light direction
-  float4* shD;    // shadow direction; w = target triangle (bits, -1 = environment)
-  float4* shFD;   // f_diffuse; w = |cos| at the shading point
-  float4* shFC;   // f_concentrated; w = shading triangle (bits)
-  float4* shThr;  // local throughput (Beer / (1 - q))
-  float4* shBeta; // path throughput at the vertex
-  float4* shT;    // transmittance of the light-ray media copy
-  uint32_t* qA;   // extension queue of this bounce
-  uint32_t* qB;   // extension queue of the next bounce
-  uint32_t* qS;   // shadow queue
-  uint32_t* qR;   // paths that ended at this bounce
-  uint32_t* mark; // bounce (epoch) whose extension queue holds the slot
+  uint4* media;   // 2 x uint4 per path (8 entries), read when the flags say so
+  uint32_t* mediaTx;  // 8 per path: albedo texel of each media entry (or null)
+};
+
+// Shadow rays of one bounce: record i belongs to the vertex of path i, and q
+// lists the n that were cast.  Every factor of a light sample but its
+// visibility is known when it is drawn, so the record carries the radiance to
+// add if nothing is in the way, and q says where: to the path's L in the next
+// set, or, for a path that ended at the vertex, to the results ring
+// (kDestRing).
+struct ShadowRays {
+  uint2* q;      // record, destination
+  float4* o;     // origin; w = t of the target triangle (+inf: environment)
+  float4* d;     // direction; w = target triangle, kTargetSky or kTargetLate (bits)
+  float4* c;     // radiance to add
+  uint32_t* job; // job index (batches)
+  // Scenes with both an environment and emissive triangles (else null): an
+  // environment sample may meet a light instead of the sky, and its term is
+  // then computed from these (see kConnectLate).
+  float4* lateFD;   // f_diffuse; w = |cos| at the shading point
+  float4* lateFC;   // f_concentrated; w = shading triangle (bits)
+  float4* lateThr;  // local throughput (Beer / (1 - q)); w = BSDF pdf of the direction
+  float4* lateBeta; // path throughput at the vertex
+  float4* lateT;    // transmittance of the light-ray media copy
+  float4* lateHit;  // the light that was met: t, u, v, triangle (bits)
+  uint2* lateQ;     // entries of q whose ray met a light
+};
+constexpr int32_t kTargetSky = -1, kTargetLate = -2;
+constexpr uint32_t kDestRing = 0x80000000u;
+
+// Memory of a render: the path pool of `capacity` paths in flight (a path
+// that ends makes room for the next of the render), its shadow rays, and the
+// results ring.
+struct PathBuffers {
+  PathSet set[2];
+  float4* hit;    // closest hits of the paths alive: t, u, v, triangle (bits)
+  ShadowRays sh;
+  uint2* ended;   // training: path id and record count of the paths that ended
   uint32_t* counters;         // see CounterId
   unsigned long long* stats;  // see StatId
   uint2* stackOverflow;
@@ -49,16 +69,18 @@ struct PathBuffers {
   uint32_t traceThreads;  // threads of the traversal grids (overflow slices)
 };
 
+// Counters of a bounce; there are two sets, used in turn, so that the kernel
+// that closes a bounce can prepare the next one's while its own are read.
 enum CounterId {
-  kCntA = 0,      // live paths in qA
-  kCntB = 1,      // paths queued for the next bounce
-  kCntS = 2,      // shadow rays
-  kCntR = 3,      // paths that ended at this bounce
-  kCntNext = 4,   // next path id to start
-  kCntLimit = 5,  // path ids below this may start (results ring space)
-  kCntFill = 6,   // idle slots seen by kFill this bounce (its cursor)
-  kCntEpoch = 7,  // bounces advanced since the render started
-  kNumCounters = 8
+  kCntA = 0,     // paths that went on (packed at the front of the next set)
+  kCntS = 1,     // shadow rays (A and S are one 64-bit atomic)
+  kCntLive = 2,  // paths alive at this bounce
+  kCntNext = 3,  // next path id to start
+  kCntEnded = 4, // training: paths that ended with records
+  kCntLate = 5,  // shadow rays that met a light instead of the sky
+  kCntSet = 8,   // words per set
+  kCntLimit = 2 * kCntSet,  // path ids below this may start (results ring space)
+  kNumCounters = 3 * kCntSet
 };
 
 // One job of a render call: samples first .. first + paths / pixels - 1 of
@@ -76,21 +98,21 @@ struct PassInfo {
   const float2* offsets;      // per sample of the call
 };
 
-// Guided rendering (single job): per-slot raw guide outputs, per-slot
-// training records (2 x {position, normal, wo + the density wi was drawn
+// Guided rendering (single job): guide outputs of the paths alive, training
+// records by path id (2 x {position, normal, wo + the density wi was drawn
 // with, wi + the BSDF density of wi, throughput before the sample, radiance
 // before the continuation}) and the training samples harvested when paths
 // end (4 float4 each: position + weight, normal, wo + drawing density,
 // wi + BSDF density).
 struct GuideRun {
   guide::Net net;
-  float4* raw;      // 10 float4 per slot
-  float4* rec;      // 12 float4 per slot
+  float4* raw;      // 10 float4 per path alive
+  float4* rec;      // 12 float4 per path of the call (training)
   float4* samples;  // sampleCap x 4 float4
   uint32_t* sampleCount;
   uint32_t sampleCap;
   float fraction;   // probability of drawing the direction from the guide
-  float* sel;       // per slot: that probability as the guide learned it (or null: `fraction`)
+  float* sel;       // per path alive: that probability as the guide learned it (or null: `fraction`)
   uint32_t maxDepth;  // only vertices of depth below this are guided
   float maxThroughput;  // ... and only while every channel of the path throughput is at most this
 };
@@ -140,12 +162,11 @@ struct LaunchConfig {
 
 enum KernelId {
   kKGenerate = 0,
-  kKExtend,
+  kKTrace,
   kKShade,
   kKConnect,
   kKAccumulate,
   kKMisc,
-  kKRetire,
   kKGraph,
   kKGuideInfer,
   kKSppmRadii,

@@ -1,25 +1,32 @@
 // Wavefront path tracer for gfx950 with path regeneration:
-//   fill -> repeat { extend -> shade -> connect -> retire } -> accumulate.
+//   fill, trace, then repeat { shade -> fill -> trace }; accumulate.
 // A render call covers n samples of every pixel (n * pixels paths, numbered
-// sample-major, pixels in 8x8-tile order).  A fixed pool of path slots runs
-// them: `retire` writes a finished path's radiance into a results ring and
-// starts the next path id in the same slot, so the queues stay full until
-// the last paths drain.  Every path's random stream is keyed by (pixel,
-// sample), so the image does not depend on which slot ran which path, and
-// `accumulate` adds each pixel's samples in sample order.
+// sample-major, pixels in 8x8-tile order).  A pool of path records runs them:
+// `shade` takes every path alive one vertex further and packs those that go on
+// at the front of the other record set, `fill` appends the next paths of the
+// render behind them, and `trace` answers the rays of both kinds: the shadow
+// rays `shade` cast and the next extension rays.  A path that ends writes its
+// radiance into a results ring.  Every path's random stream is keyed by
+// (pixel, sample), so the image does not depend on which record ran which
+// path, and `accumulate` adds each pixel's samples in sample order.
 //
 // The recursion of estimateRadiance (core/src/PathTracing.cpp:21-95) becomes
 // one extension ray (BSDF strategy) plus one shadow ray (light strategy) per
-// vertex: `shade` runs a vertex up to both samples, `connect` finishes the
-// light strategy once its closest hit is known (visibility by triangle id,
-// Scene.cpp:558-559 / 572-577), and the BSDF strategy's MIS weight is applied
-// by the next `shade`, which is where the next hit is known.  Radiance is
-// accumulated forward along the path; every decision (roulette, lobe choice,
-// rejection, visibility) is made exactly as in the recursion.
+// vertex.  `shade` runs a vertex up to both samples and computes the light
+// sample's whole term, which is added once its ray is found clear (visibility
+// by triangle id, Scene.cpp:558-559 / 572-577); the BSDF strategy's MIS
+// weight is applied by the next `shade`, which is where the next hit is
+// known.  Radiance is accumulated forward along the path; every decision
+// (roulette, lobe choice, rejection, visibility) is made exactly as in the
+// recursion.
 //
-// Live paths are compacted after every vertex: each wave counts its survivors
-// with a ballot, the waves of a block combine their counts with a prefix sum
-// in LDS, and the block reserves its range with one atomic.
+// Records are packed by moving them: a vertex rewrites nearly all of a path's
+// state anyway, so writing it to its place in the next bounce's order costs
+// nothing extra, and every stage then reads consecutive records with all 64
+// lanes live, secondary rays first and the (coherent) camera rays after them.
+// Each wave counts its survivors with a ballot, the waves of a block combine
+// their counts with a prefix sum in LDS, and the block reserves its ranges of
+// paths and shadow rays with one 64-bit atomic.
 #include "pt_kernels.h"
 
 #include <algorithm>
@@ -33,11 +40,10 @@ using namespace hdev;
 const char* kernelName(int id) {
   switch (id) {
     case kKGenerate: return "pt_generate";
-    case kKExtend: return "pt_extend";
+    case kKTrace: return "pt_trace";
     case kKShade: return "pt_shade";
-    case kKConnect: return "pt_connect";
+    case kKConnect: return "pt_connect_late";
     case kKAccumulate: return "pt_accumulate";
-    case kKRetire: return "pt_retire";
     case kKGraph: return "pt_graph_chunk";
     case kKGuideInfer: return "guide_infer";
     case kKSppmRadii: return "sppm_init_radii";
@@ -52,29 +58,33 @@ const char* kernelName(int id) {
 
 namespace {
 
-// Block-wide append: returns this lane's index in the output queue (valid
-// only where `pred`).  Must be reached by every thread of the block.
-__device__ inline uint32_t blockAppend(uint32_t* counter, bool pred, uint32_t* ldsWave, uint32_t* ldsBase) {
-  uint64_t mask = __ballot(pred);
-  uint32_t lane = threadIdx.x & 63u;
-  uint32_t wave = threadIdx.x >> 6;
-  uint32_t prefix = (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
-  if (lane == 0) ldsWave[wave] = (uint32_t)__popcll(mask);
+// Block-wide append of two kinds at once: this lane's index among the paths
+// that go on (valid where `go`) and among the shadow rays (where `cast`).
+// `counter` holds both counts, paths in the low word.  Must be reached by
+// every thread of the block.
+__device__ inline void blockAppend2(unsigned long long* counter, bool go, bool cast, uint2* ldsWave,
+                                    unsigned long long* ldsBase, uint32_t* idxGo, uint32_t* idxCast) {
+  const uint64_t mg = __ballot(go), mc = __ballot(cast);
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const uint64_t below = (1ull << lane) - 1ull;
+  if (lane == 0) ldsWave[wave] = make_uint2((uint32_t)__popcll(mg), (uint32_t)__popcll(mc));
   __syncthreads();
   if (threadIdx.x == 0) {
-    uint32_t acc = 0;
-    uint32_t nw = blockDim.x >> 6;
-    for (uint32_t w = 0; w < nw; ++w) {
-      uint32_t c = ldsWave[w];
+    uint2 acc = make_uint2(0u, 0u);
+    for (uint32_t w = 0; w < (blockDim.x >> 6); ++w) {
+      const uint2 c = ldsWave[w];
       ldsWave[w] = acc;
-      acc += c;
+      acc.x += c.x, acc.y += c.y;
     }
-    *ldsBase = acc ? atomicAdd(counter, acc) : 0u;
+    const unsigned long long both = (unsigned long long)acc.x | ((unsigned long long)acc.y << 32);
+    *ldsBase = both ? atomicAdd(counter, both) : 0ull;
   }
   __syncthreads();
-  uint32_t r = *ldsBase + ldsWave[wave] + prefix;
+  const unsigned long long base = *ldsBase;
+  const uint2 before = ldsWave[wave];
+  *idxGo = (uint32_t)base + before.x + (uint32_t)__popcll(mg & below);
+  *idxCast = (uint32_t)(base >> 32) + before.y + (uint32_t)__popcll(mc & below);
   __syncthreads();
-  return r;
 }
 
 // Workgroups are dealt round-robin to the 8 XCDs; renumber them so that
@@ -94,24 +104,23 @@ __device__ inline void waveAddStat(unsigned long long* c, uint32_t v) {
 
 // Entries beyond md.n are never read, so an empty stack is neither loaded
 // nor stored.
-__device__ inline void loadMedia(const PathBuffers& pb, uint32_t slot, uint32_t flags, const uint32_t* txs,
-                                 Media& md) {
+__device__ inline void loadMedia(const PathSet& ps, uint32_t i, uint32_t flags, const uint32_t* txs, Media& md) {
   md.n = (int)((flags >> 12) & 0xFu);
   md.overflow = (flags >> 16) & 1u;
   md.tx0 = 0u;
   if (md.n == 0) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) md.e[i] = 0u;
+    for (int k = 0; k < 8; ++k) md.e[k] = 0u;
     return;
   }
-  uint4 a = pb.media[(size_t)slot * 2], b = pb.media[(size_t)slot * 2 + 1];
+  uint4 a = ps.media[(size_t)i * 2], b = ps.media[(size_t)i * 2 + 1];
   md.e[0] = a.x, md.e[1] = a.y, md.e[2] = a.z, md.e[3] = a.w;
   md.e[4] = b.x, md.e[5] = b.y, md.e[6] = b.z, md.e[7] = b.w;
   if (txs) md.tx0 = txs[0];
 }
-__device__ inline void storeMedia(const PathBuffers& pb, uint32_t slot, const Media& md) {
-  pb.media[(size_t)slot * 2] = make_uint4(md.e[0], md.e[1], md.e[2], md.e[3]);
-  pb.media[(size_t)slot * 2 + 1] = make_uint4(md.e[4], md.e[5], md.e[6], md.e[7]);
+__device__ inline void storeMedia(const PathSet& ps, uint32_t i, const Media& md) {
+  ps.media[(size_t)i * 2] = make_uint4(md.e[0], md.e[1], md.e[2], md.e[3]);
+  ps.media[(size_t)i * 2 + 1] = make_uint4(md.e[4], md.e[5], md.e[6], md.e[7]);
 }
 __device__ inline uint32_t packFlags(int depth, int wavelength, const Media& md) {
   return (uint32_t)depth | ((uint32_t)(wavelength + 1) << 8) | ((uint32_t)md.n << 12) |
@@ -205,231 +214,149 @@ __device__ inline void pathPixel(const PassInfo& pi, uint32_t pid, uint32_t* pix
 
 // ------------------------------------------------------------ path start ----
 // Camera ray of path `pid` (Camera.cpp:41-81 with the sample's offset,
-// RenderJob.h:53-60) into `slot`.
-__device__ inline void startPath(const DevScene& s, const PathBuffers& pb, const PassInfo& pi, uint32_t slot,
-                                 uint32_t pid, uint32_t flags) {
+// RenderJob.h:53-60) into record i.
+__device__ inline void startPath(const DevScene& s, const PathSet& ps, const PassInfo& pi, uint32_t i, uint32_t pid,
+                                 uint32_t flags) {
   uint32_t k, pixel;
   pathPixel(pi, pid, &pixel, &k);
-  uint32_t i = pixel % s.width, j = pixel / s.width;
+  uint32_t x = pixel % s.width, y = pixel / s.width;
   hrng::Stream rng = hrng::make_stream(s.seed, pixel, pi.first + k, hrng::kDomainPath);
   float2 off = pi.offsets[k];
   V3 o, d;
-  cameraRay(s, rng, (float)i + off.x, (float)j + off.y, &o, &d);
-  // throughput, radiance and the depth-0 normal / albedo are not stored
-  // here: kShade starts every path from throughput 1 and radiance 0 and
-  // writes the aux values at its first vertex
-  pb.rayO[slot] = f4(o, 0.0f);
-  pb.rayD[slot] = f4(d, 0.0f);
-  pb.state[slot] = make_uint4(rng.counter, flags, 0xFFFFFFFFu, pid);
+  cameraRay(s, rng, (float)x + off.x, (float)y + off.y, &o, &d);
+  // throughput and radiance are not stored here: kShade starts every path
+  // from throughput 1 and radiance 0
+  ps.rayO[i] = f4(o, 0.0f);
+  ps.rayD[i] = f4(d, 0.0f);
+  ps.state[i] = make_uint4(rng.counter, flags, 0xFFFFFFFFu, pid);
 }
 
-// Every slot idle, no path started.
-// Occupancy targets (waves per SIMD) of the three ray-bound stages: the
-// register budget each may use is 512 / waves VGPRs.  0 leaves it to the
-// compiler.  Extend at 8 waves (64 VGPRs) is ~7% faster than at the
-// compiler's 7; shade at 3 keeps the guided variant (which would take 190
-// VGPRs) at the plain one's occupancy without spills (4 and 5 lose); connect
-// at 5 (96 VGPRs, 28 B of spills) is ~1% faster than the compiler's 4, at 6
-// slower.
-#ifndef HASTY_EXTEND_WAVES
-#define HASTY_EXTEND_WAVES 8
+// Occupancy targets (waves per SIMD) of the ray-bound stages: the register
+// budget each may use is 512 / waves VGPRs.  0 leaves it to the compiler.
+// Shade at 3 waves spills 64 B per lane; at 2 (no spills) the GGX grid takes
+// 131 ms, at 4 128 ms, at 3 125 ms.
+#ifndef HASTY_TRACE_WAVES
+#define HASTY_TRACE_WAVES 8
 #endif
 #ifndef HASTY_SHADE_WAVES
 #define HASTY_SHADE_WAVES 3
 #endif
-#ifndef HASTY_CONNECT_WAVES
-#define HASTY_CONNECT_WAVES 5
-#endif
 #define HASTY_WAVES_ATTR_(n) __attribute__((amdgpu_waves_per_eu(n)))
-#if HASTY_EXTEND_WAVES > 0
-#define HASTY_EXTEND_ATTR HASTY_WAVES_ATTR_(HASTY_EXTEND_WAVES)
+#if HASTY_TRACE_WAVES > 0
+#define HASTY_TRACE_ATTR HASTY_WAVES_ATTR_(HASTY_TRACE_WAVES)
 #else
-#define HASTY_EXTEND_ATTR
+#define HASTY_TRACE_ATTR
 #endif
 #if HASTY_SHADE_WAVES > 0
 #define HASTY_SHADE_ATTR HASTY_WAVES_ATTR_(HASTY_SHADE_WAVES)
 #else
 #define HASTY_SHADE_ATTR
 #endif
-#if HASTY_CONNECT_WAVES > 0
-#define HASTY_CONNECT_ATTR HASTY_WAVES_ATTR_(HASTY_CONNECT_WAVES)
-#else
-#define HASTY_CONNECT_ATTR
-#endif
 
-// The paths to extend and shade this bounce: while they fill more than half
-// the pool they are visited in slot order (entry q is slot q, taken if its
-// mark is this bounce), so that neighbouring lanes read neighbouring path
-// records; otherwise through the queue qA.  Either way every path is visited
-// once, and the image does not depend on the order.
-struct ExtSet {
-  bool dense;
-  uint32_t total, epoch;
-  __device__ bool member(const PathBuffers& pb, uint32_t q, uint32_t* slot) const {
-    if (!dense) {
-      *slot = pb.qA[q];
-      return true;
-    }
-    *slot = q;
-    return pb.mark[q] == epoch;
-  }
-};
-__device__ inline ExtSet extensionSet(const PathBuffers& pb) {
-  ExtSet e;
-  const uint32_t n = pb.counters[kCntA];
-  e.dense = 2ull * n > (unsigned long long)pb.capacity;
-  e.total = e.dense ? pb.capacity : n;
-  e.epoch = pb.counters[kCntEpoch];
-  return e;
-}
-
-__global__ void __launch_bounds__(kBlock) kInitRender(PathBuffers pb, uint32_t limit) {
-  uint32_t stride = gridDim.x * blockDim.x;
-  for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < pb.capacity; k += stride) pb.mark[k] = 0xFFFFFFFFu;
-  if (blockIdx.x == 0 && threadIdx.x < kNumCounters) {
-    uint32_t v = 0u;
-    if (threadIdx.x == kCntLimit) v = limit;
-    pb.counters[threadIdx.x] = v;
-  }
-}
-
-// A slot is idle when its mark is not this bounce's (its path ended, or it
-// never had one).  kFill visits the slots in order: idle slots draw offsets
-// from the fill cursor (one atomic per block), those below the ring-space
-// limit start the paths next + offset and join qA; kFillCommit advances
-// next by the number started and resets the cursor.  Paths are started in
-// slot order, so their records are written in whole cache lines where idle
-// slots are adjacent.
-__device__ inline uint32_t fillAvail(const uint32_t* c) {
-  const uint32_t next = c[kCntNext], lim = c[kCntLimit];
-  return lim > next ? lim - next : 0u;
-}
-// Block-wide sum of v (every thread of the block calls it).
-__device__ inline uint32_t blockSum(uint32_t v, uint32_t* ldsWave) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  if ((threadIdx.x & 63u) == 0) ldsWave[threadIdx.x >> 6] = v;
-  __syncthreads();
-  uint32_t sum = 0;
-  for (uint32_t w = 0; w < (blockDim.x >> 6); ++w) sum += ldsWave[w];
-  __syncthreads();
-  return sum;
-}
-// Exclusive prefix count of pred in thread order over the block, and the
-// block's count in *total (every thread of the block calls it).
-__device__ inline uint32_t blockPrefix(bool pred, uint32_t* ldsWave, uint32_t* total) {
-  const uint64_t mask = __ballot(pred);
-  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  const uint32_t prefix = (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
-  if (lane == 0) ldsWave[wave] = (uint32_t)__popcll(mask);
-  __syncthreads();
-  uint32_t before = 0, sum = 0;
-  for (uint32_t w = 0; w < (blockDim.x >> 6); ++w) {
-    const uint32_t c = ldsWave[w];
-    before += w < wave ? c : 0u;
-    sum += c;
-  }
-  __syncthreads();
-  *total = sum;
-  return before + prefix;
-}
-// Each block owns a contiguous range of slots: it counts the range's idle
-// slots, takes offsets for all of them with one atomic on the fill cursor
-// and a qA range for those it can start with one more, then starts them in
-// slot order.  (Two atomics per block, instead of two per 256 slots: same-
-// address atomics from every block were what bounded this kernel.)  8192
-// blocks (1024 slots each at 2^23 slots) measured fastest: 2048 and 4096
-// leave too few waves to hide the mark reads, 16384 and more pay for the
-// atomics again.
-constexpr uint32_t kFillBlocks = 8192;
-template <bool MULTI>
-__global__ void __launch_bounds__(kBlock) kFill(JobSet js, PathBuffers pb) {
-  __shared__ uint32_t ldsWave[kBlock / 64];
-  __shared__ uint32_t ldsBase[3];
-  __shared__ uint32_t ldsIdle[2 * kBlock];  // idle slots waiting for a path, in slot order
-  const uint32_t avail = fillAvail(pb.counters);
-  if (avail == 0u) return;  // the same for every thread
-  const uint32_t next = pb.counters[kCntNext], epoch = pb.counters[kCntEpoch];
-  const uint32_t per = (pb.capacity + gridDim.x * kBlock - 1) / (gridDim.x * kBlock) * kBlock;
-  const uint32_t lo = min(blockIdx.x * per, pb.capacity), hi = min(lo + per, pb.capacity);
-  uint32_t mine = 0;
-  for (uint32_t slot = lo + threadIdx.x; slot < hi; slot += kBlock) mine += pb.mark[slot] != epoch ? 1u : 0u;
-  const uint32_t idleTotal = blockSum(mine, ldsWave);
-  if (threadIdx.x == 0) {
-    const uint32_t b = idleTotal ? atomicAdd(&pb.counters[kCntFill], idleTotal) : 0u;
-    const uint32_t live = b < avail ? min(idleTotal, avail - b) : 0u;
-    ldsBase[0] = b;
-    ldsBase[1] = live;
-    ldsBase[2] = live ? atomicAdd(&pb.counters[kCntA], live) : 0u;
-  }
-  __syncthreads();
-  const uint32_t b = ldsBase[0], live = ldsBase[1], qa = ldsBase[2];
-  // The r-th idle slot of the range starts path next + b + r.  The idle
-  // slots are queued in LDS and their paths started a block at a time, one
-  // per thread, so that the camera-ray code runs on full waves.
-  auto start = [&](uint32_t r, uint32_t slot) {
-    const uint32_t pid = next + b + r;
-    const uint32_t j = findJob<MULTI>(js, pid);
-    const uint32_t flags = MULTI ? jobBits(js, j) : 0u;
-    pb.mark[slot] = epoch;
-    forJob<MULTI>(js, j, [&](const DevScene& sc, const PassInfo& pi) { startPath(sc, pb, pi, slot, pid, flags); });
-    pb.qA[qa + r] = slot;
-  };
-  uint32_t rankBase = 0, done = 0;  // idle slots seen / started (uniform)
-  for (uint32_t base = lo; base < hi && rankBase < live; base += kBlock) {  // uniform bounds
-    const uint32_t slot = base + threadIdx.x;
-    const bool idle = slot < hi && pb.mark[slot] != epoch;
-    uint32_t count;
-    const uint32_t r = rankBase + blockPrefix(idle, ldsWave, &count);
-    if (idle && r < live) ldsIdle[r - done] = slot;  // fewer than kBlock were queued before
-    rankBase += count;
-    const uint32_t queued = min(rankBase, live) - done;
-    if (queued >= kBlock) {
-      __syncthreads();
-      start(done + threadIdx.x, ldsIdle[threadIdx.x]);
-      const uint32_t rest = threadIdx.x < queued - kBlock ? ldsIdle[kBlock + threadIdx.x] : 0u;
-      __syncthreads();
-      if (threadIdx.x < queued - kBlock) ldsIdle[threadIdx.x] = rest;
-      done += kBlock;
-    }
-  }
-  __syncthreads();
-  const uint32_t queued = min(rankBase, live) - done;
-  if (threadIdx.x < queued) start(done + threadIdx.x, ldsIdle[threadIdx.x]);
-}
-__global__ void kFillCommit(uint32_t* c) {
-  if (threadIdx.x == 0) {
-    const uint32_t avail = fillAvail(c), idle = c[kCntFill];
-    c[kCntNext] += idle < avail ? idle : avail;
-    c[kCntFill] = 0u;
-  }
+// No path started, nothing alive.
+__global__ void kInitRender(uint32_t* c, uint32_t limit) {
+  if (threadIdx.x < kNumCounters) c[threadIdx.x] = threadIdx.x == kCntLimit ? limit : 0u;
 }
 __global__ void kSetLimit(uint32_t* c, uint32_t limit) {
   if (threadIdx.x == 0) c[kCntLimit] = limit;
 }
 
-// --------------------------------------------------------------- extend ----
+// Paths that start at the end of bounce p: the pool's free places behind the
+// paths that went on, up to the ring-space limit.
+__device__ inline uint32_t startCount(const PathBuffers& pb, const uint32_t* c) {
+  const uint32_t limit = pb.counters[kCntLimit], next = c[kCntNext];
+  const uint32_t left = limit > next ? limit - next : 0u;
+  return min(pb.capacity - c[kCntA], left);
+}
+template <bool MULTI>
+__global__ void __launch_bounds__(kBlock) kFill(JobSet js, PathBuffers pb, PathSet out, uint32_t p) {
+  const uint32_t* c = pb.counters + p * kCntSet;
+  const uint32_t n = startCount(pb, c), base = c[kCntA], next = c[kCntNext];
+  for (uint32_t r = blockIdx.x * kBlock + threadIdx.x; r < n; r += gridDim.x * kBlock) {
+    const uint32_t pid = next + r, j = findJob<MULTI>(js, pid);
+    const uint32_t flags = MULTI ? jobBits(js, j) : 0u;
+    forJob<MULTI>(js, j, [&](const DevScene& sc, const PassInfo& pi) { startPath(sc, out, pi, base + r, pid, flags); });
+  }
+}
+
+// ---------------------------------------------------------------- trace ----
+// The rays of a bounce in one launch: the shadow rays, then the extension
+// rays of the paths alive.  One launch for both kinds because a launch ends
+// with a tail of its longest rays (a few hundred dependent node fetches)
+// during which the chip is nearly idle; together they have one tail instead
+// of two.  Shadow records carry the term to add, so both kinds fit the 64
+// registers of 8 waves per SIMD (7 waves: 14% slower on the 1024x1024 GGX
+// grid; grids other than the 2048 resident blocks lose 10% and more).
+// Bound by the latency of dependent node fetches and by divergence; against
+// separate launches over half-filled waves the 128-sample render of that grid
+// went from 170 to 125 ms, one sample of a 1283x721 film from 6.1 to 4.1 ms.
 // COUNT: add rays, node visits and triangle tests to the statistics (the
-// counting is compiled out otherwise).
+// counting is compiled out otherwise).  LATE: some shadow rays look for the
+// closest hit (kTargetLate).
 // W: node width of the single job's scene (4 or 8), 0 = each job's own.
-template <bool MULTI, bool COUNT, int W>
-__global__ void __launch_bounds__(kBlock) HASTY_EXTEND_ATTR kExtend(JobSet js, PathBuffers pb) {
+template <bool MULTI, bool COUNT, int W, bool LATE>
+__global__ void __launch_bounds__(kBlock) HASTY_TRACE_ATTR kTrace(JobSet js, PathBuffers pb, PathSet ps, uint32_t p) {
   __shared__ uint2 stack[kStackLds * kBlock];
-  const ExtSet es = extensionSet(pb);
-  uint32_t gtid = xcdBlock() * blockDim.x + threadIdx.x;
-  uint32_t stride = gridDim.x * blockDim.x;
+  const uint32_t gtid = xcdBlock() * blockDim.x + threadIdx.x;
+  const uint32_t stride = gridDim.x * blockDim.x;
+  uint2* lds = stack + threadIdx.x;
   uint2* ovf = pb.stackOverflow + (size_t)gtid * kStackOvf;
+  const uint32_t* c = pb.counters + p * kCntSet;
+  const uint32_t nS = c[kCntS];
   uint32_t nodes = 0, tris = 0, rays = 0;
-  for (uint32_t q = gtid; q < es.total; q += stride) {
-    uint32_t slot;
-    if (!es.member(pb, q, &slot)) continue;
-    float4 o = pb.rayO[slot], d = pb.rayD[slot];
-    const uint32_t job = MULTI ? jobOf<MULTI>(js, pb.state[slot]) : 0u;
-    Hit h;
-    forJob<MULTI>(js, job, [&](const DevScene& sc, const PassInfo&) {
-      h = traceClosest<kStackLds, kStackOvf, W>(sc, f4xyz(o), f4xyz(d), stack + threadIdx.x, kBlock, ovf, &nodes,
-                                                &tris);
+  for (uint32_t k = gtid; k < nS; k += stride) {
+    const uint2 ray = pb.sh.q[k];
+    const uint32_t i = ray.x, dest = ray.y;
+    const float4 o = pb.sh.o[i], d = pb.sh.d[i];
+    const int32_t target = __float_as_int(d.w);
+    bool clear = false;
+    forJob<MULTI>(js, MULTI ? pb.sh.job[i] : 0u, [&](const DevScene& sc, const PassInfo&) {
+      if (!LATE || target != kTargetLate) {
+        // closest hit == target  <=>  no other triangle is hit before it (or
+        // at its t with a smaller index); sky visible  <=>  nothing is hit
+        clear = findBlocker<kStackLds, kStackOvf, W>(sc, prepareRay(f4xyz(o), f4xyz(d)), o.w,
+                                                     target >= 0 ? target : 0x7FFFFFFF, lds, kBlock, ovf, &nodes,
+                                                     &tris) < 0;
+      } else {
+        const Hit h = traceClosest<kStackLds, kStackOvf, W>(sc, f4xyz(o), f4xyz(d), lds, kBlock, ovf, &nodes, &tris);
+        if (h.tri < 0) {
+          clear = true;
+        } else if (ldg(&sc.mats[ldg(sc.triMat + h.tri)].isLight)) {
+          pb.sh.lateHit[i] = make_float4(h.t, h.u, h.v, __int_as_float(h.tri));
+          pb.sh.lateQ[atomicAdd(&pb.counters[p * kCntSet + kCntLate], 1u)] = ray;
+        }
+      }
     });
-    pb.hit[slot] = make_float4(h.t, h.u, h.v, __int_as_float(h.tri));
+    if (clear) {
+      const float4 t = pb.sh.c[i];
+      float4* at = (dest & kDestRing) ? pb.ringL + (dest & ~kDestRing) : ps.L + dest;
+      const float4 L = *at;
+      *at = f4(f4xyz(L) + f4xyz(t), 0.0f);
+    }
+    rays++;
+  }
+  if (COUNT) {
+    waveAddStat(&pb.stats[kStatShadowRays], rays);
+    waveAddStat(&pb.stats[kStatShadowNodes], nodes);
+    waveAddStat(&pb.stats[kStatShadowTris], tris);
+    nodes = tris = rays = 0;
+  }
+  const uint32_t begin = startCount(pb, c), live = c[kCntA] + begin;
+  if (gtid == 0) {  // the next bounce's counters
+    uint32_t* d = pb.counters + (p ^ 1u) * kCntSet;
+    d[kCntA] = 0u, d[kCntS] = 0u, d[kCntEnded] = 0u, d[kCntLate] = 0u;
+    d[kCntLive] = live;
+    d[kCntNext] = c[kCntNext] + begin;
+  }
+  // the threads that got no shadow ray in the last sweep take the first
+  // extension rays
+  const uint32_t skip = nS % stride;
+  for (uint32_t i = gtid >= skip ? gtid - skip : gtid + (stride - skip); i < live; i += stride) {
+    const float4 o = ps.rayO[i], d = ps.rayD[i];
+    forJob<MULTI>(js, MULTI ? jobOf<MULTI>(js, ps.state[i]) : 0u, [&](const DevScene& sc, const PassInfo&) {
+      const Hit h = traceClosest<kStackLds, kStackOvf, W>(sc, f4xyz(o), f4xyz(d), lds, kBlock, ovf, &nodes, &tris);
+      pb.hit[i] = make_float4(h.t, h.u, h.v, __int_as_float(h.tri));
+    });
     rays++;
   }
   if (COUNT) {
@@ -458,396 +385,400 @@ __device__ inline bool guideThroughputOk(const GuideRun& g, V3 beta) {
   return fmaxf(beta.x, fmaxf(beta.y, beta.z)) <= g.maxThroughput;
 }
 
+// What a vertex leaves: the path's state where it goes on (o, d, pdf, beta,
+// flags, md, with L up to the vertex's own emission) and its light sample.
+struct Vertex {
+  V3 o, d;
+  float pdf;
+  V3 beta, L;
+  uint32_t draws, flags;
+  int32_t tri;
+  Media md;
+  bool go;  // the path goes on with the ray (o, d)
+  bool cast;  // its light sample needs a shadow ray (record i of pb.sh)
+};
+
+// The term of a light sample that nothing blocks, t2 = thr (fD + fC) cos / pL
+// weighted against the BSDF's density pB, times the incident radiance
+// (Scene.cpp:560-586, MIS.cpp:32-54); false where it adds nothing.
+__device__ inline bool lightTerm(V3 fD, V3 fC, float cosX, V3 thr, float pL, float pB, V3* t2) {
+  if (pL == 0.0f) return false;
+  const float mm = cosX / pL;
+  const V3 tD = fD * mm, tC = fC * mm;
+  *t2 = mul(thr, tD + tC);
+  if (isZero(*t2)) return false;
+  float sum = 0.0f;
+  sum += powci<2>(pL);
+  sum += powci<2>(pB);
+  const float w = powci<2>(pL) / sum;
+  *t2 = *t2 * w;
+  return true;
+}
+// Radiance of light triangle `tri` (point hx, normal hn) along -sd, through
+// the media of the light ray.
+__device__ inline V3 lightRadiance(const DevScene& s, int32_t tri, V3 hx, V3 hn, V3 so, V3 sd, V3 Tc) {
+  const DevMaterial lm = ldgStruct(s.mats + ldg(s.triMat + tri));
+  const V3 Tb = beersLaw(Tc, norm(hx - so));
+  const V3 Le = dot(hn, -sd) <= 0.0f ? v3(0.0f, 0.0f, 0.0f)
+                                      : v3(lm.emission[0], lm.emission[1], lm.emission[2]) * (float)kInvPi;
+  return mul(Tb, Le);
+}
+
+// One vertex of path i of the set `in`, whose ray met h4.
+template <bool GUIDED>
+__device__ inline void shadeVertex(const DevScene& s, const PassInfo& pi, const GuideRun& g, const PathBuffers& pb,
+                                   const PathSet& in, uint32_t i, const uint4 st, Vertex& vx) {
+  const bool twoStrategies = s.hasLight && s.useMIS;
+  int depth = (int)(st.y & 0xFFu);
+  int wavelength = (int)((st.y >> 8) & 0x3u) - 1;
+  // per-entry albedo texels of the media stack (albedo-textured scenes)
+  uint32_t* txs = s.texturedMedia ? in.mediaTx + (size_t)i * kMaxMedia : nullptr;
+  Media& md = vx.md;
+  loadMedia(in, i, st.y, txs, md);
+  int32_t prevTri = (int32_t)st.z;
+  const float4 ro4 = in.rayO[i], rd4 = in.rayD[i], h4 = pb.hit[i];
+  V3 ro = f4xyz(ro4), rd = f4xyz(rd4);
+  const int32_t tri = __float_as_int(h4.w);
+  // a path's first vertex starts from throughput 1 and radiance 0 (not
+  // stored by kFill)
+  const V3 b0 = depth == 0 ? v3(1.0f, 1.0f, 1.0f) : f4xyz(in.beta[i]);
+  V3 beta = b0;
+  const float4 L4 = depth == 0 ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : in.L[i];
+  V3& L = vx.L;
+  L = f4xyz(L4);
+  vx.go = vx.cast = false;
+  uint32_t nrec = GUIDED ? (st.y >> kRecShift) & 3u : 0u;
+  if (GUIDED && depth > 0 && nrec > 0 && ((st.y >> (kRecShift + 2)) & 1u)) {
+    // radiance before the continuation of the last recorded vertex
+    g.rec[(size_t)st.w * 12 + 6 * (nrec - 1) + 5] = L4;
+  }
+  hrng::Stream rng;
+  {
+    uint32_t k, pixel;
+    pathPixel(pi, st.w, &pixel, &k);
+    rng = hrng::make_stream(s.seed, pixel, pi.first + k, hrng::kDomainPath);
+    rng.counter = st.x;
+  }
+  const EnvUV sky = tri < 0 && s.hasEnv ? envUV(rd) : EnvUV{0.0f, 0.0f, 0.0f};
+  const float pSurf = !s.hasEnv ? 1.0f : (s.hasSurfaceLight ? 0.5f : 0.0f);
+  // The BSDF sample that produced this ray: self-intersection, then MIS.
+  if (depth > 0) {
+    if (tri == prevTri) return;
+    float pB = rd4.w;
+    float sum = 0.0f;
+    if (twoStrategies) {
+      float pL;
+      if (tri >= 0) {
+        V3 hx, hn;
+        hitPointNormal(s, tri, h4.y, h4.z, &hx, &hn);
+        pL = lightDensity(s, ro, rd, tri, hx, hn);
+      } else {
+        pL = s.hasEnv ? (1.0f - pSurf) * envPdf(s, sky) : 0.0f;
+      }
+      sum += powci<2>(pL);
+    }
+    sum += powci<2>(pB);
+    float w = powci<2>(pB) / sum;
+    beta = beta * w;
+  }
+  const uint32_t ri = depth == 0 ? st.w % pb.ringPaths : 0u;
+  if (tri < 0) {
+    V3 T = beersLaw(mediaTransmittance(s, md), 1e6f);
+    V3 Lc = mul(T, s.hasEnv ? envLookup(s, sky.u, sky.v) : v3(s.bg[0], s.bg[1], s.bg[2]));
+    L = L + mul(beta, Lc);
+    if (depth == 0) {
+      pb.ringN[ri] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      pb.ringA[ri] = f4(Lc, 0.0f);
+    }
+    return;
+  }
+  Interaction it = makeInteraction(s, tri, h4.y, h4.z);
+  DevMaterial m = ldgStruct(s.mats + it.mat);
+  // guided vertex: rough reflection (no delta lobe, and not so glossy
+  // that broad vMF lobes could only waste samples); decided on the
+  // material before its textures and on the stored throughput
+  // before this vertex's MIS weight, exactly as kGuideInfer decides
+  // it, so that every guided vertex has its mixture table
+  const bool guided = GUIDED && guideEligible(m) && (uint32_t)depth < g.maxDepth &&
+                      (depth == 0 || guideThroughputOk(g, b0));
+  if (depth == 0) pb.ringN[ri] = f4(it.ns, 0.0f);  // the default shading normal
+  uint32_t texel = 0u;
+  if (m.textured) applyTextures(s, m, it, 1.0f - h4.y - h4.z, h4.y, h4.z, &texel);
+  if (depth == 0) pb.ringA[ri] = make_float4(m.albedo[0], m.albedo[1], m.albedo[2], 0.0f);
+  V3 Tb = beersLaw(mediaTransmittance(s, md), norm(it.x - ro));
+  V3 wo = -rd;
+  if (m.isLight) {
+    V3 Le = dot(it.ng, wo) <= 0.0f ? v3(0.0f, 0.0f, 0.0f)
+                                    : v3(m.emission[0], m.emission[1], m.emission[2]) * (float)kInvPi;
+    L = L + mul(beta, mul(Tb, Le));
+    return;
+  }
+  float rrQ = depth >= s.rrStart ? s.rrQ : 0.0f;
+  if (rng.uniform01f() < rrQ) return;
+  V3 thr = Tb / (1.0f - rrQ);
+  if (depth + 1 >= s.maxDepth) return;  // every deeper estimate is zero
+  // the vertex's mixture table, written by kGuideInfer
+  const float4* gm = GUIDED ? g.raw + (size_t)i * 10 : nullptr;
+  // kGuideInfer wrote the learned probability of guided vertices
+  const float gf = GUIDED ? (g.sel && guided ? g.sel[i] : g.fraction) : 0.0f;
+  if (twoStrategies) {
+    // ---- light strategy (MIS.cpp:32-54, Scene.cpp:538-586)
+    float xi = rng.uniform01f();
+    V3 so, sd;
+    int32_t target = kTargetSky;
+    float tT = __builtin_inff();
+    V3 hx = v3(0.0f, 0.0f, 0.0f), hn = v3(0.0f, 0.0f, 0.0f);  // the target's point and normal
+    bool lit = true;  // the sampled light point emits toward so and its ray meets it
+    if (xi < pSurf) {
+      uint32_t li = lightCdfSearch(s, rng.canonical_double());
+      target = (int32_t)ldg(s.lightTris + li);
+      const float* p = s.triPos + (size_t)target * 9;
+      V3 p0 = load3g(p), p1 = load3g(p + 3), p2 = load3g(p + 6);
+      float su = rng.uniform01f();
+      float tt = hm::fsqrt(rng.uniform01f());
+      float b1 = 1.0f - tt;
+      float b3 = tt * su;
+      float b2 = fmaxf(0.0f, 1.0f - b1 - b3);
+      V3 x2 = p0 * b1 + p1 * b2 + p2 * b3;
+      V3 diff = x2 - it.x;
+      so = offsetOrigin(it, dot(it.ng, diff) >= 0.0f);
+      sd = normalize(x2 - so);
+      hn = normalize(cross(p1 - p0, p2 - p0));
+      lit = !(dot(hn, -sd) <= 0.0f);  // a one-sided light seen from behind gives zero
+      if (lit) {
+        float uT, vT;
+        lit = intersectTri(prepareRay(so, sd), f4(p0, 0.0f), f4(p1, 0.0f), f4(p2, 0.0f), 1e-6f, &tT, &uT, &vT);
+        hx = p0 * (1.0f - uT - vT) + p1 * uT + p2 * vT;
+      }
+    } else {
+      float dens;
+      sd = envSample(s, rng, &dens);
+      so = offsetOrigin(it, dot(it.ng, sd) >= 0.0f);
+    }
+    BsdfEval ev = bsdfEvaluate(m, it, wo, sd);
+    // A light sample the BSDF gives nothing (e.g. below the surface), that
+    // sees a light from behind or whose term is zero adds exactly zero
+    // whatever its shadow ray meets, so no ray is cast; about a quarter of
+    // the samples on the GGX grid.
+    if (lit && !isZero(ev.fD + ev.fC)) {
+      float pB = bsdfPdf(m, it, wo, sd, mediaOutsideIOR(s, md, it, wo, wavelength));
+      if (GUIDED && guided) pB = gf * guide::mixturePdfTable(gm, sd) + (1.0f - gf) * pB;
+      const V3 Tc = mediaTransmittanceAfter(s, md, it, wo, sd, texel, txs);
+      const float cosX = __builtin_fabsf(dot(sd, it.ng));
+      V3 t2, Lt = v3(0.0f, 0.0f, 0.0f);  // the term if nothing is in the way
+      if (target >= 0) {
+        if (target != tri && lightTerm(ev.fD, ev.fC, cosX, thr, lightDensity(s, so, sd, target, hx, hn), pB, &t2)) {
+          Lt = mul(beta, mul(lightRadiance(s, target, hx, hn, so, sd, Tc), t2));
+          vx.cast = true;
+        }
+      } else {
+        const EnvUV e = envUV(sd);
+        if (lightTerm(ev.fD, ev.fC, cosX, thr, (1.0f - pSurf) * envPdf(s, e), pB, &t2)) {
+          Lt = mul(beta, mul(mul(beersLaw(Tc, 1e6f), envLookup(s, e.u, e.v)), t2));
+          vx.cast = true;
+        }
+        if (pSurf > 0.0f) {  // the ray may meet a light instead (kConnectLate)
+          vx.cast = true;
+          target = kTargetLate;
+          pb.sh.lateFD[i] = f4(ev.fD, cosX);
+          pb.sh.lateFC[i] = f4(ev.fC, __int_as_float(tri));
+          pb.sh.lateThr[i] = f4(thr, pB);
+          pb.sh.lateBeta[i] = f4(beta, 0.0f);
+          pb.sh.lateT[i] = f4(Tc, 0.0f);
+        }
+      }
+      if (vx.cast) {
+        pb.sh.o[i] = f4(so, tT);
+        pb.sh.d[i] = f4(sd, __int_as_float(target));
+        pb.sh.c[i] = f4(Lt, 0.0f);
+      }
+    }
+  }
+  // ---- BSDF strategy (MIS.cpp:6-26, Scene.cpp:328-338)
+  float sampleProbability = 1.0f;
+  if (wavelength == -1 && m.varyIOR) {
+    float p0 = 1.0f / 3.0f;
+    float xi = rng.uniform01f();
+    if (xi < p0) wavelength = 0;
+    else if (xi < p0 + p0) wavelength = 1;
+    else wavelength = 2;
+    sampleProbability = p0;
+  }
+  float outsideIOR = mediaOutsideIOR(s, md, it, wo, wavelength);
+  BsdfSample bs;
+  float pBsdf = 0.0f;  // the BSDF's density of the direction (training records)
+  if (GUIDED && guided) {
+    // one-sample MIS of guide and BSDF: p = f pG + (1 - f) pB
+    if (rng.uniform01f() < gf) {
+      float x0 = rng.uniform01f(), x1 = rng.uniform01f(), x2 = rng.uniform01f();
+      bs.dir = guide::mixtureSampleTable(gm, x0, x1, x2);
+      bs.outside = dot(it.ng, wo) >= 0.0f;
+      BsdfEval ev = bsdfEvaluate(m, it, wo, bs.dir);
+      float pB = bsdfPdf(m, it, wo, bs.dir, outsideIOR);
+      pBsdf = pB;
+      bs.pdf = gf * guide::mixturePdfTable(gm, bs.dir) + (1.0f - gf) * pB;
+      float mm = bs.pdf > 0.0f ? __builtin_fabsf(dot(bs.dir, it.ng)) / bs.pdf : 0.0f;
+      bs.tD = ev.fD * mm;
+      bs.tC = ev.fC * mm;
+      if (!(bs.pdf > 0.0f)) bs.pdf = 0.0f;
+    } else {
+      bs = bsdfSample(m, rng, it, wo, wavelength, outsideIOR, false, 3);
+      pBsdf = bs.pdf;
+      if (bs.pdf != 0.0f) {
+        float pMix = gf * guide::mixturePdfTable(gm, bs.dir) + (1.0f - gf) * bs.pdf;
+        float sc = bs.pdf / pMix;
+        bs.tD = bs.tD * sc;
+        bs.tC = bs.tC * sc;
+        bs.pdf = pMix;
+      }
+    }
+  } else {
+    bs = bsdfSample(m, rng, it, wo, wavelength, outsideIOR, false, 3);
+  }
+  bs.tD = bs.tD / sampleProbability;
+  bs.tC = bs.tC / sampleProbability;
+  if (bs.pdf == 0.0f) return;
+  V3 t2 = mul(thr, bs.tD + bs.tC);
+  if (isZero(t2)) return;
+  mediaUpdate(md, it, wo, bs.dir, texel, txs);
+  vx.go = true;
+  vx.o = offsetOrigin(it, bs.outside);
+  vx.d = bs.dir;
+  vx.pdf = bs.pdf;
+  vx.beta = mul(beta, t2);
+  vx.draws = rng.counter;
+  vx.tri = tri;
+  uint32_t recBits = 0u;
+  if (GUIDED) {
+    if (guided && nrec < 2u && g.sampleCap > 0u) {  // records only when training
+      float4* rr = g.rec + (size_t)st.w * 12 + 6 * nrec;
+      V3 nf = dot(it.ng, wo) >= 0.0f ? it.ng : -it.ng;
+      rr[0] = f4(it.x, 0.0f);
+      rr[1] = f4(nf, 0.0f);
+      rr[2] = f4(wo, bs.pdf);
+      rr[3] = f4(bs.dir, pBsdf);
+      rr[4] = f4(beta, 0.0f);
+      nrec += 1u;
+      recBits = (nrec << kRecShift) | (1u << (kRecShift + 2));
+    } else {
+      recBits = nrec << kRecShift;
+    }
+  }
+  vx.flags = packFlags(depth + 1, wavelength, md) | recBits | (st.y & ~((1u << kJobShift) - 1u));
+}
+
+// Bounce p: every path alive in `in` one vertex further, those that go on
+// packed into `out`, light samples into the shadow rays, and the radiance of
+// those that end into the results ring (to which a last light sample is still
+// added by kTrace).  With `count`, ended paths whose media stack overflowed
+// are counted.
 template <bool MULTI, bool GUIDED>
-__global__ void __launch_bounds__(kBlock) HASTY_SHADE_ATTR kShade(JobSet js, PathBuffers pb) {
-  __shared__ uint32_t ldsWave[kBlock / 64];
-  __shared__ uint32_t ldsBase;
-  const ExtSet es = extensionSet(pb);
-  uint32_t stride = gridDim.x * blockDim.x;
-  for (uint32_t base = blockIdx.x * blockDim.x; base < es.total; base += stride) {
-    uint32_t q = base + threadIdx.x;
-    bool pushNext = false, pushShadow = false, live = false;
-    uint32_t slot = 0;
-    if (q < es.total && es.member(pb, q, &slot)) {
-      live = true;
-      const uint4 st = pb.state[slot];
-      forJob<MULTI>(js, jobOf<MULTI>(js, st), [&](const DevScene& s, const PassInfo& pi) {
-      const bool twoStrategies = s.hasLight && s.useMIS;
-      int depth = (int)(st.y & 0xFFu);
-      int wavelength = (int)((st.y >> 8) & 0x3u) - 1;
-      // per-entry albedo texels of the media stack (albedo-textured scenes)
-      uint32_t* txs = s.texturedMedia ? pb.mediaTx + (size_t)slot * kMaxMedia : nullptr;
-      Media md;
-      loadMedia(pb, slot, st.y, txs, md);
-      int32_t prevTri = (int32_t)st.z;
-      float4 ro4 = pb.rayO[slot], rd4 = pb.rayD[slot], h4 = pb.hit[slot];
-      V3 ro = f4xyz(ro4), rd = f4xyz(rd4);
-      int32_t tri = __float_as_int(h4.w);
-      // a path's first vertex starts from throughput 1 and radiance 0 (not
-      // stored by kFill)
-      const float4 b4 = depth == 0 ? make_float4(1.0f, 1.0f, 1.0f, 0.0f) : pb.beta[slot];
-      V3 beta = f4xyz(b4);
-      const float4 L4 = depth == 0 ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : pb.L[slot];
-      V3 L = f4xyz(L4);
-      uint32_t nrec = GUIDED ? (st.y >> kRecShift) & 3u : 0u;
-      if (GUIDED && depth > 0 && nrec > 0 && ((st.y >> (kRecShift + 2)) & 1u)) {
-        // radiance before the continuation of the last recorded vertex
-        js.g.rec[(size_t)slot * 12 + 6 * (nrec - 1) + 5] = L4;
-      }
-      hrng::Stream rng;
-      {
-        uint32_t k, pixel;
-        pathPixel(pi, st.w, &pixel, &k);
-        rng = hrng::make_stream(s.seed, pixel, pi.first + k, hrng::kDomainPath);
-        rng.counter = st.x;
-      }
-      bool alive = true;
-      // The BSDF sample that produced this ray: self-intersection, then MIS.
-      if (depth > 0) {
-        if (tri == prevTri) {
-          alive = false;
-        } else {
-          float pB = rd4.w;
-          float w;
-          if (twoStrategies) {
-            V3 hx = v3(0.0f, 0.0f, 0.0f), hn = v3(0.0f, 0.0f, 0.0f);
-            if (tri >= 0) hitPointNormal(s, tri, h4.y, h4.z, &hx, &hn);
-            float pL = lightDensity(s, ro, rd, tri, hx, hn);
-            float sum = 0.0f;
-            sum += powci<2>(pL);
-            sum += powci<2>(pB);
-            w = powci<2>(pB) / sum;
-          } else {
-            float sum = 0.0f;
-            sum += powci<2>(pB);
-            w = powci<2>(pB) / sum;
-          }
-          beta = beta * w;
-        }
-      }
-      if (alive) {
-        float4 aux = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (tri < 0) {
-          V3 T = beersLaw(mediaTransmittance(s, md), 1e6f);
-          V3 Lc = mul(T, evalEnvironment(s, rd));
-          L = L + mul(beta, Lc);
-          if (depth == 0) {
-            pb.auxN[slot] = aux;
-            pb.auxA[slot] = f4(Lc, 0.0f);
-          }
-          alive = false;
-        } else {
-          Interaction it = makeInteraction(s, tri, h4.y, h4.z);
-          DevMaterial m = ldgStruct(s.mats + it.mat);
-          // guided vertex: rough reflection (no delta lobe, and not so glossy
-          // that broad vMF lobes could only waste samples); decided on the
-          // material before its textures and on the stored throughput
-          // before this vertex's MIS weight, exactly as kGuideInfer decides
-          // it, so that every guided vertex has its mixture table
-          const bool guided = GUIDED && guideEligible(m) && (uint32_t)depth < js.g.maxDepth &&
-                              (depth == 0 || guideThroughputOk(js.g, f4xyz(b4)));
-          if (depth == 0) pb.auxN[slot] = f4(it.ns, 0.0f);  // the default shading normal
-          uint32_t texel = 0u;
-          if (m.textured) applyTextures(s, m, it, 1.0f - h4.y - h4.z, h4.y, h4.z, &texel);
-          if (depth == 0) pb.auxA[slot] = make_float4(m.albedo[0], m.albedo[1], m.albedo[2], 0.0f);
-          V3 Tb = beersLaw(mediaTransmittance(s, md), norm(it.x - ro));
-          V3 wo = -rd;
-          if (m.isLight) {
-            V3 Le = dot(it.ng, wo) <= 0.0f ? v3(0.0f, 0.0f, 0.0f)
-                                            : v3(m.emission[0], m.emission[1], m.emission[2]) * (float)kInvPi;
-            L = L + mul(beta, mul(Tb, Le));
-            alive = false;
-          } else {
-            float rrQ = depth >= s.rrStart ? s.rrQ : 0.0f;
-            if (rng.uniform01f() < rrQ) {
-              alive = false;
-            } else {
-              V3 thr = Tb / (1.0f - rrQ);
-              if (depth + 1 >= s.maxDepth) {
-                alive = false;  // every deeper estimate is zero
-              } else {
-                // the vertex's mixture table, written by kGuideInfer
-                const float4* gm = GUIDED ? js.g.raw + (size_t)slot * 10 : nullptr;
-                // kGuideInfer wrote the learned probability of guided vertices
-                const float gf = GUIDED ? (js.g.sel && guided ? js.g.sel[slot] : js.g.fraction) : 0.0f;
-                if (twoStrategies) {
-                  // ---- light strategy (MIS.cpp:32-54, Scene.cpp:538-586)
-                  float pSurf = !s.hasEnv ? 1.0f : (s.hasSurfaceLight ? 0.5f : 0.0f);
-                  float xi = rng.uniform01f();
-                  V3 so, sd;
-                  int32_t target = -1;
-                  bool lit = true;  // the sampled light point emits toward so
-                  if (xi < pSurf) {
-                    uint32_t li = lightCdfSearch(s, rng.canonical_double());
-                    target = (int32_t)ldg(s.lightTris + li);
-                    const float* p = s.triPos + (size_t)target * 9;
-                    V3 p0 = load3g(p), p1 = load3g(p + 3), p2 = load3g(p + 6);
-                    float su = rng.uniform01f();
-                    float tt = hm::fsqrt(rng.uniform01f());
-                    float b1 = 1.0f - tt;
-                    float b3 = tt * su;
-                    float b2 = fmaxf(0.0f, 1.0f - b1 - b3);
-                    V3 x2 = p0 * b1 + p1 * b2 + p2 * b3;
-                    V3 diff = x2 - it.x;
-                    so = offsetOrigin(it, dot(it.ng, diff) >= 0.0f);
-                    sd = normalize(x2 - so);
-                    // kConnect's emission test on the target (hitPointNormal's
-                    // normal): a one-sided light seen from behind gives zero
-                    lit = !(dot(normalize(cross(p1 - p0, p2 - p0)), -sd) <= 0.0f);
-                  } else {
-                    float dens;
-                    sd = envSample(s, rng, &dens);
-                    so = offsetOrigin(it, dot(it.ng, sd) >= 0.0f);
-                  }
-                  BsdfEval ev = bsdfEvaluate(m, it, wo, sd);
-                  // A light sample the BSDF gives nothing (e.g. below the
-                  // surface; kConnect's t2 = thr (fD + fC) |cos| / pL) or
-                  // that sees a light from behind adds exactly zero whatever
-                  // its shadow ray meets, so no ray is cast; about a quarter
-                  // of the samples on the GGX grid.
-                  if (lit && !isZero(ev.fD + ev.fC)) {
-                    float outsideIOR = mediaOutsideIOR(s, md, it, wo, wavelength);
-                    float pB = bsdfPdf(m, it, wo, sd, outsideIOR);
-                    if (GUIDED && guided) pB = gf * guide::mixturePdfTable(gm, sd) + (1.0f - gf) * pB;
-                    V3 Tc = mediaTransmittanceAfter(s, md, it, wo, sd, texel, txs);
-                    pb.shO[slot] = f4(so, pB);
-                    pb.shD[slot] = f4(sd, __int_as_float(target));
-                    pb.shFD[slot] = f4(ev.fD, __builtin_fabsf(dot(sd, it.ng)));
-                    pb.shFC[slot] = f4(ev.fC, __int_as_float(tri));
-                    pb.shThr[slot] = f4(thr, 0.0f);
-                    pb.shBeta[slot] = f4(beta, 0.0f);
-                    pb.shT[slot] = f4(Tc, 0.0f);
-                    pushShadow = true;
-                  }
-                }
-                // ---- BSDF strategy (MIS.cpp:6-26, Scene.cpp:328-338)
-                float sampleProbability = 1.0f;
-                if (wavelength == -1 && m.varyIOR) {
-                  float p0 = 1.0f / 3.0f;
-                  float xi = rng.uniform01f();
-                  if (xi < p0) wavelength = 0;
-                  else if (xi < p0 + p0) wavelength = 1;
-                  else wavelength = 2;
-                  sampleProbability = p0;
-                }
-                float outsideIOR = mediaOutsideIOR(s, md, it, wo, wavelength);
-                BsdfSample bs;
-                float pBsdf = 0.0f;  // the BSDF's density of the direction (training records)
-                if (GUIDED && guided) {
-                  // one-sample MIS of guide and BSDF: p = f pG + (1 - f) pB
-                  if (rng.uniform01f() < gf) {
-                    float x0 = rng.uniform01f(), x1 = rng.uniform01f(), x2 = rng.uniform01f();
-                    bs.dir = guide::mixtureSampleTable(gm, x0, x1, x2);
-                    bs.outside = dot(it.ng, wo) >= 0.0f;
-                    BsdfEval ev = bsdfEvaluate(m, it, wo, bs.dir);
-                    float pB = bsdfPdf(m, it, wo, bs.dir, outsideIOR);
-                    pBsdf = pB;
-                    bs.pdf = gf * guide::mixturePdfTable(gm, bs.dir) + (1.0f - gf) * pB;
-                    float mm = bs.pdf > 0.0f ? __builtin_fabsf(dot(bs.dir, it.ng)) / bs.pdf : 0.0f;
-                    bs.tD = ev.fD * mm;
-                    bs.tC = ev.fC * mm;
-                    if (!(bs.pdf > 0.0f)) bs.pdf = 0.0f;
-                  } else {
-                    bs = bsdfSample(m, rng, it, wo, wavelength, outsideIOR, false, 3);
-                    pBsdf = bs.pdf;
-                    if (bs.pdf != 0.0f) {
-                      float pMix = gf * guide::mixturePdfTable(gm, bs.dir) + (1.0f - gf) * bs.pdf;
-                      float sc = bs.pdf / pMix;
-                      bs.tD = bs.tD * sc;
-                      bs.tC = bs.tC * sc;
-                      bs.pdf = pMix;
-                    }
-                  }
-                } else {
-                  bs = bsdfSample(m, rng, it, wo, wavelength, outsideIOR, false, 3);
-                }
-                bs.tD = bs.tD / sampleProbability;
-                bs.tC = bs.tC / sampleProbability;
-                if (bs.pdf != 0.0f) {
-                  V3 t2 = mul(thr, bs.tD + bs.tC);
-                  if (!isZero(t2)) {
-                    V3 no = offsetOrigin(it, bs.outside);
-                    mediaUpdate(md, it, wo, bs.dir, texel, txs);
-                    pb.rayO[slot] = f4(no, 0.0f);
-                    pb.rayD[slot] = f4(bs.dir, bs.pdf);
-                    pb.beta[slot] = f4(mul(beta, t2), 0.0f);
-                    pushNext = true;
-                  }
-                }
-                alive = false;
-                if (pushNext) {
-                  uint32_t recBits = 0u;
-                  if (GUIDED) {
-                    if (guided && nrec < 2u && js.g.sampleCap > 0u) {  // records only when training
-                      float4* rr = js.g.rec + (size_t)slot * 12 + 6 * nrec;
-                      V3 nf = dot(it.ng, wo) >= 0.0f ? it.ng : -it.ng;
-                      rr[0] = f4(it.x, 0.0f);
-                      rr[1] = f4(nf, 0.0f);
-                      rr[2] = f4(wo, bs.pdf);
-                      rr[3] = f4(bs.dir, pBsdf);
-                      rr[4] = f4(beta, 0.0f);
-                      nrec += 1u;
-                      recBits = (nrec << kRecShift) | (1u << (kRecShift + 2));
-                    } else {
-                      recBits = nrec << kRecShift;
-                    }
-                  }
-                  pb.mark[slot] = es.epoch + 1u;
-                  pb.state[slot] =
-                      make_uint4(rng.counter,
-                                 packFlags(depth + 1, wavelength, md) | recBits | (st.y & ~((1u << kJobShift) - 1u)),
-                                 (uint32_t)tri, st.w);
-                  if (md.n > 0) storeMedia(pb, slot, md);
-                }
-              }
-            }
-          }
-        }
-      }
-      pb.L[slot] = f4(L, 0.0f);
+__global__ void __launch_bounds__(kBlock) HASTY_SHADE_ATTR kShade(JobSet js, PathBuffers pb, PathSet in, PathSet out,
+                                                                 uint32_t p, uint32_t count) {
+  __shared__ uint2 ldsWave[kBlock / 64];
+  __shared__ unsigned long long ldsBase;
+  uint32_t* c = pb.counters + p * kCntSet;
+  const uint32_t n = c[kCntLive];
+  uint32_t overflowed = 0;
+  for (uint32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
+    const uint32_t i = base + threadIdx.x;
+    Vertex vx;
+    vx.go = vx.cast = false;
+    uint4 st = make_uint4(0u, 0u, 0u, 0u);
+    uint32_t job = 0u;
+    if (i < n) {
+      st = in.state[i];
+      job = jobOf<MULTI>(js, st);
+      forJob<MULTI>(js, job, [&](const DevScene& s, const PassInfo& pi) {
+        shadeVertex<GUIDED>(s, pi, js.g, pb, in, i, st, vx);
       });
     }
-    uint32_t idxN = blockAppend(&pb.counters[kCntB], pushNext, ldsWave, &ldsBase);
-    if (pushNext) pb.qB[idxN] = slot;
-    uint32_t idxS = blockAppend(&pb.counters[kCntS], pushShadow, ldsWave, &ldsBase);
-    if (pushShadow) pb.qS[idxS] = slot;
-    bool retire = live && !pushNext;  // the path ends here (after its shadow ray, if any)
-    uint32_t idxR = blockAppend(&pb.counters[kCntR], retire, ldsWave, &ldsBase);
-    if (retire) pb.qR[idxR] = slot;
+    uint32_t idxN, idxS;
+    blockAppend2((unsigned long long*)(c + kCntA), vx.go, vx.cast, ldsWave, &ldsBase, &idxN, &idxS);
+    uint32_t dest = idxN;
+    if (vx.go) {
+      out.rayO[idxN] = f4(vx.o, 0.0f);
+      out.rayD[idxN] = f4(vx.d, vx.pdf);
+      out.beta[idxN] = f4(vx.beta, 0.0f);
+      out.L[idxN] = f4(vx.L, 0.0f);
+      out.state[idxN] = make_uint4(vx.draws, vx.flags, (uint32_t)vx.tri, st.w);
+      if (vx.md.n > 0) {
+        storeMedia(out, idxN, vx.md);
+        if (in.mediaTx)
+          for (int k = 0; k < vx.md.n; ++k)
+            out.mediaTx[(size_t)idxN * kMaxMedia + k] = in.mediaTx[(size_t)i * kMaxMedia + k];
+      }
+    } else if (i < n) {  // the path ends here (but for its shadow ray, if any)
+      const uint32_t ri = st.w % pb.ringPaths;
+      dest = ri | kDestRing;
+      pb.ringL[ri] = f4(vx.L, 0.0f);
+      overflowed += (st.y >> 16) & 1u;
+      const uint32_t nrec = GUIDED ? (st.y >> kRecShift) & 3u : 0u;
+      if (GUIDED && nrec > 0u) pb.ended[atomicAdd(c + kCntEnded, 1u)] = make_uint2(st.w, nrec);
+    }
+    if (vx.cast) {
+      pb.sh.q[idxS] = make_uint2(i, dest);
+      if (MULTI) pb.sh.job[i] = job;
+    }
   }
+  if (count) waveAddStat(&pb.stats[kStatMediaOverflow], overflowed);
 }
 
 // -------------------------------------------------------------- connect ----
-template <bool MULTI, bool COUNT, int W>
-__global__ void __launch_bounds__(kBlock) HASTY_CONNECT_ATTR kConnect(JobSet js, PathBuffers pb) {
-  __shared__ uint2 stack[kStackLds * kBlock];
-  uint32_t n = pb.counters[kCntS];
-  uint32_t gtid = xcdBlock() * blockDim.x + threadIdx.x;
-  uint32_t stride = gridDim.x * blockDim.x;
-  uint2* ovf = pb.stackOverflow + (size_t)gtid * kStackOvf;
-  uint32_t nodes = 0, tris = 0, rays = 0;
-  for (uint32_t q = gtid; q < n; q += stride) {
-    uint32_t slot = pb.qS[q];
-    const uint32_t job = MULTI ? jobOf<MULTI>(js, pb.state[slot]) : 0u;
+// Environment samples of bounce p whose ray met a light (scenes with both
+// kinds of lights): the light strategy's term for the light (Scene.cpp:560-586).
+template <bool MULTI>
+__global__ void __launch_bounds__(kBlock) kConnectLate(JobSet js, PathBuffers pb, PathSet ps, uint32_t p) {
+  const uint32_t n = pb.counters[p * kCntSet + kCntLate];
+  for (uint32_t q = blockIdx.x * kBlock + threadIdx.x; q < n; q += gridDim.x * kBlock) {
+    const uint32_t i = pb.sh.lateQ[q].x, dest = pb.sh.lateQ[q].y;
+    const uint32_t job = MULTI ? pb.sh.job[i] : 0u;
     forJob<MULTI>(js, job, [&](const DevScene& s, const PassInfo&) {
-    float4 o4 = pb.shO[slot], d4 = pb.shD[slot];
-    V3 so = f4xyz(o4), sd = f4xyz(d4);
-    int32_t target = __float_as_int(d4.w);
-    RayPre rp = prepareRay(so, sd);
-    rays++;
-    // Visibility exactly as the closest-hit test of Scene.cpp:558-559 / 572-577,
-    // answered with an early-exit search wherever that is equivalent.
-    Hit h;
-    bool visible;
-    if (target >= 0) {
-      // closest hit == target  <=>  the target is hit at (tT, target) and no
-      // other triangle hits before it (or at tT with a smaller index)
-      const float* p = s.triPos + (size_t)target * 9;
-      float4 p0 = make_float4(ldg(p), ldg(p + 1), ldg(p + 2), 0.0f),
-             p1 = make_float4(ldg(p + 3), ldg(p + 4), ldg(p + 5), 0.0f),
-             p2 = make_float4(ldg(p + 6), ldg(p + 7), ldg(p + 8), 0.0f);
-      float tT, uT, vT;
-      visible = intersectTri(rp, p0, p1, p2, 1e-6f, &tT, &uT, &vT);
-      if (visible) {
-        visible = findBlocker<kStackLds, kStackOvf, W>(s, rp, tT, target, stack + threadIdx.x, kBlock, ovf,
-                                                    &nodes, &tris) < 0;
-        h.t = tT, h.u = uT, h.v = vT, h.tri = target;
-      }
-    } else if (!s.hasSurfaceLight) {
-      // no emissive triangle: visible <=> nothing is hit at all
-      visible = findBlocker<kStackLds, kStackOvf, W>(s, rp, __builtin_inff(), 0x7FFFFFFF, stack + threadIdx.x, kBlock,
-                                                  ovf, &nodes,
-                                                  &tris) < 0;
-      h.t = __builtin_inff(), h.u = h.v = 0.0f, h.tri = -1;
-    } else {
-      h = traceClosest<kStackLds, kStackOvf, W>(s, so, sd, stack + threadIdx.x, kBlock, ovf,
-                                             &nodes, &tris);
-      bool hitLight = h.tri >= 0 && ldg(&s.mats[ldg(s.triMat + h.tri)].isLight);
-      visible = h.tri < 0 || hitLight;
-    }
-    if (!visible) return;
-    V3 hx = v3(0.0f, 0.0f, 0.0f), hn = v3(0.0f, 0.0f, 0.0f);
-    if (h.tri >= 0) hitPointNormal(s, h.tri, h.u, h.v, &hx, &hn);
-    float pL = lightDensity(s, so, sd, h.tri, hx, hn);
-    if (pL == 0.0f) return;
-    float4 fd4 = pb.shFD[slot], fc4 = pb.shFC[slot];
-    float mm = fd4.w / pL;
-    V3 tD = f4xyz(fd4) * mm, tC = f4xyz(fc4) * mm;
-    V3 thr = f4xyz(pb.shThr[slot]);
-    V3 t2 = mul(thr, tD + tC);
-    if (isZero(t2) || h.tri == __float_as_int(fc4.w)) return;
-    float pB = o4.w;
-    float sum = 0.0f;
-    sum += powci<2>(pL);
-    sum += powci<2>(pB);
-    float w = powci<2>(pL) / sum;
-    t2 = t2 * w;
-    V3 Tc = f4xyz(pb.shT[slot]);
-    V3 Li;
-    if (h.tri < 0) {
-      Li = mul(beersLaw(Tc, 1e6f), evalEnvironment(s, sd));
-    } else {
-      const DevMaterial lm = ldgStruct(s.mats + ldg(s.triMat + h.tri));
-      V3 Tb = beersLaw(Tc, norm(hx - so));
-      V3 Le = dot(hn, -sd) <= 0.0f ? v3(0.0f, 0.0f, 0.0f)
-                                    : v3(lm.emission[0], lm.emission[1], lm.emission[2]) * (float)kInvPi;
-      Li = mul(Tb, Le);
-    }
-    V3 beta = f4xyz(pb.shBeta[slot]);
-    float4 L4 = pb.L[slot];
-    pb.L[slot] = f4(f4xyz(L4) + mul(beta, mul(Li, t2)), 0.0f);
+      const V3 so = f4xyz(pb.sh.o[i]), sd = f4xyz(pb.sh.d[i]);
+      const float4 h = pb.sh.lateHit[i];
+      const int32_t tri = __float_as_int(h.w);
+      V3 hx, hn;
+      hitPointNormal(s, tri, h.y, h.z, &hx, &hn);
+      const float4 fd = pb.sh.lateFD[i], fc = pb.sh.lateFC[i], thr = pb.sh.lateThr[i];
+      V3 t2;
+      if (tri == __float_as_int(fc.w) ||
+          !lightTerm(f4xyz(fd), f4xyz(fc), fd.w, f4xyz(thr), lightDensity(s, so, sd, tri, hx, hn), thr.w, &t2))
+        return;
+      const V3 Li = lightRadiance(s, tri, hx, hn, so, sd, f4xyz(pb.sh.lateT[i]));
+      float4* L = (dest & kDestRing) ? pb.ringL + (dest & ~kDestRing) : ps.L + dest;
+      *L = f4(f4xyz(*L) + mul(f4xyz(pb.sh.lateBeta[i]), mul(Li, t2)), 0.0f);
     });
-  }
-  if (COUNT) {
-    waveAddStat(&pb.stats[kStatShadowRays], rays);
-    waveAddStat(&pb.stats[kStatShadowNodes], nodes);
-    waveAddStat(&pb.stats[kStatShadowTris], tris);
   }
 }
 
-// --------------------------------------------------------------- retire ----
-// Finished paths: results into the ring; the slot is idle from the next
-// bounce on (its mark is not renewed) and kFill gives it a new path id.
-// With `count`, paths whose media stack overflowed are counted.
-template <bool GUIDED>
-__global__ void __launch_bounds__(kBlock) kRetire(JobSet js, PathBuffers pb, uint32_t count) {
-  uint32_t n = pb.counters[kCntR];
-  uint32_t stride = gridDim.x * blockDim.x;
-  uint32_t overflowed = 0;
-  for (uint32_t q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += stride) {
-    const uint32_t slot = pb.qR[q];
-    uint4 st = pb.state[slot];
-    overflowed += (st.y >> 16) & 1u;
-    uint32_t ri = st.w % pb.ringPaths;
-    float4 Lf = pb.L[slot];
-    pb.ringL[ri] = Lf;
-    if (GUIDED) {
-      // training samples: weight = luminance of the radiance the
-      // continuation brought, over the throughput before the sample
-      uint32_t nrec = (st.y >> kRecShift) & 3u;
-      for (uint32_t r = 0; r < nrec; ++r) {
-        const float4* rr = js.g.rec + (size_t)slot * 12 + 6 * r;
-        float4 b = rr[4], ls = rr[5];
-        float cx = b.x > 0.0f ? (Lf.x - ls.x) / b.x : 0.0f;
-        float cy = b.y > 0.0f ? (Lf.y - ls.y) / b.y : 0.0f;
-        float cz = b.z > 0.0f ? (Lf.z - ls.z) / b.z : 0.0f;
-        float F = 0.2126f * cx + 0.7152f * cy + 0.0722f * cz;
-        if (F > 0.0f && F < 3.0e38f) {
-          uint32_t k = atomicAdd(js.g.sampleCount, 1u);
-          if (k < js.g.sampleCap) {
-            float4 x = rr[0];
-            js.g.samples[4 * (size_t)k] = make_float4(x.x, x.y, x.z, F);
-            js.g.samples[4 * (size_t)k + 1] = rr[1];
-            js.g.samples[4 * (size_t)k + 2] = rr[2];
-            js.g.samples[4 * (size_t)k + 3] = rr[3];
-          }
+// -------------------------------------------------------------- harvest ----
+// Training samples of the paths that ended at bounce p: weight = luminance
+// of the radiance the continuation brought, over the throughput before the
+// sample.
+__global__ void __launch_bounds__(kBlock) kHarvest(GuideRun g, PathBuffers pb, uint32_t p) {
+  const uint32_t n = pb.counters[p * kCntSet + kCntEnded];
+  for (uint32_t q = blockIdx.x * kBlock + threadIdx.x; q < n; q += gridDim.x * kBlock) {
+    const uint2 e = pb.ended[q];
+    const float4 Lf = pb.ringL[e.x % pb.ringPaths];
+    for (uint32_t r = 0; r < e.y; ++r) {
+      const float4* rr = g.rec + (size_t)e.x * 12 + 6 * r;
+      float4 b = rr[4], ls = rr[5];
+      float cx = b.x > 0.0f ? (Lf.x - ls.x) / b.x : 0.0f;
+      float cy = b.y > 0.0f ? (Lf.y - ls.y) / b.y : 0.0f;
+      float cz = b.z > 0.0f ? (Lf.z - ls.z) / b.z : 0.0f;
+      float F = 0.2126f * cx + 0.7152f * cy + 0.0722f * cz;
+      if (F > 0.0f && F < 3.0e38f) {
+        uint32_t k = atomicAdd(g.sampleCount, 1u);
+        if (k < g.sampleCap) {
+          float4 x = rr[0];
+          g.samples[4 * (size_t)k] = make_float4(x.x, x.y, x.z, F);
+          g.samples[4 * (size_t)k + 1] = rr[1];
+          g.samples[4 * (size_t)k + 2] = rr[2];
+          g.samples[4 * (size_t)k + 3] = rr[3];
         }
       }
     }
-    pb.ringN[ri] = pb.auxN[slot];
-    pb.ringA[ri] = pb.auxA[slot];
   }
-  if (count) waveAddStat(&pb.stats[kStatMediaOverflow], overflowed);
 }
 
 // ----------------------------------------------------------- accumulate ----
@@ -878,7 +809,7 @@ __global__ void __launch_bounds__(kBlock) kAccumulate(PathBuffers pb, PassInfo p
 }
 
 // ------------------------------------------------------------ guide infer ----
-// Raw guide outputs for every path in qA that hit a guided surface: inputs
+// Mixture tables of the paths alive that hit a guided surface: inputs
 // are the hit point, the geometric normal facing wo, and wo.  A wave takes 64
 // paths, one per lane, for the gathers (hit, material, triangle, ray), then
 // runs the network on its four 16-path tiles in turn; the tile's lanes fetch
@@ -889,32 +820,30 @@ __global__ void __launch_bounds__(kBlock) kAccumulate(PathBuffers pb, PassInfo p
 #endif
 constexpr uint32_t kGuideInferThreads = 512, kGuideInferBlocks = 256 * 3;
 __global__ void __launch_bounds__(kGuideInferThreads) HASTY_WAVES_ATTR_(HASTY_GUIDE_INFER_WAVES)
-    kGuideInfer(JobSet js, PathBuffers pb) {
+    kGuideInfer(JobSet js, PathBuffers pb, PathSet ps, uint32_t p) {
   __shared__ guide::LdsNet ldsNet;
   guide::stageNet(js.g.net, &ldsNet, true);
   const DevScene& s = js.s;
-  const uint32_t n = pb.counters[kCntA];
+  const uint32_t n = pb.counters[p * kCntSet + kCntLive];
   const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
   const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const uint32_t waves = (gridDim.x * blockDim.x) >> 6;
   for (uint32_t g = wave; g * 64 < n; g += waves) {
     const uint32_t e = g * 64 + lane;
-    uint32_t slot = 0u;
     bool want = false;
     V3 x = v3(0.0f, 0.0f, 0.0f), ng = v3(0.0f, 0.0f, 1.0f), wo = v3(0.0f, 0.0f, 1.0f);
     if (e < n) {
-      slot = pb.qA[e];
-      const float4 h4 = pb.hit[slot];
+      const float4 h4 = pb.hit[e];
       const int32_t tri = __float_as_int(h4.w);
       if (tri >= 0) {
         // only hits on guided materials read the outputs
         const DevMaterial m = ldgStruct(s.mats + ldg(s.triMat + tri));
-        const uint32_t depth = pb.state[slot].y & 0xFFu;
+        const uint32_t depth = ps.state[e].y & 0xFFu;
         want = guideEligible(m) && depth < js.g.maxDepth;
-        if (want && depth > 0) want = guideThroughputOk(js.g, f4xyz(pb.beta[slot]));
+        if (want && depth > 0) want = guideThroughputOk(js.g, f4xyz(ps.beta[e]));
         if (want) {
           hitPointNormal(s, tri, h4.y, h4.z, &x, &ng);
-          wo = -f4xyz(pb.rayD[slot]);
+          wo = -f4xyz(ps.rayD[e]);
           if (dot(ng, wo) < 0.0f) ng = -ng;
           x = guide::normPos(js.g.net, x);
         }
@@ -929,7 +858,7 @@ __global__ void __launch_bounds__(kGuideInferThreads) HASTY_WAVES_ATTR_(HASTY_GU
       const V3 xq = v3(__shfl(x.x, src), __shfl(x.y, src), __shfl(x.z, src));
       const V3 nq = v3(__shfl(ng.x, src), __shfl(ng.y, src), __shfl(ng.z, src));
       const V3 wq = v3(__shfl(wo.x, src), __shfl(wo.y, src), __shfl(wo.z, src));
-      const uint32_t sq = __shfl(slot, src);
+      const uint32_t sq = g * 64 + src;
       // lane group q holds lobes 2q and 2q + 1 of the path's mixture
       float r10[10], w0, w1, logit;
       guide::tileOutputs(&ldsNet, xq, nq, wq, r10, &w0, &w1, &logit);
@@ -941,17 +870,6 @@ __global__ void __launch_bounds__(kGuideInferThreads) HASTY_WAVES_ATTR_(HASTY_GU
         if (js.g.sel && q == 0) js.g.sel[sq] = guide::selectionOf(js.g.net, logit);
       }
     }
-  }
-}
-
-// Next bounce: qB becomes the input queue (the host swaps the pointers).
-__global__ void kAdvance(uint32_t* c) {
-  if (threadIdx.x == 0) {
-    c[kCntEpoch] += 1u;
-    c[kCntA] = c[kCntB];
-    c[kCntB] = 0u;
-    c[kCntS] = 0u;
-    c[kCntR] = 0u;
   }
 }
 
@@ -1123,64 +1041,74 @@ void hipOk(hipError_t e, const char* what) {
   if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
 }
 
-// The bounces of one chunk: fill, extend, shade, connect, retire, advance.
-// `chunk` is even, so the queue pointers are back in place afterwards and
-// every chunk issues identical launches (what a captured graph replays).
+// Launches of one render's bounces.  Bounce p (0 or 1, in turn) reads the
+// paths of set p and leaves the next bounce's in the other one.
 template <bool MULTI, bool GUIDED, int W>
-void launchChunk(const JobSet& js, const PathBuffers& pbIn, const LaunchConfig& cfg, uint32_t chunk,
-                 hipStream_t stream, KernelTimer* timer) {
-  PathBuffers pb = pbIn;
-  auto t0 = [&](int k) {
-    if (timer) timer->begin(k, stream);
-  };
-  auto t1 = [&](int k) {
-    if (timer) timer->end(k, stream);
-  };
-  const int countStats = cfg.countStats ? 1 : 0;
-  for (uint32_t it = 0; it < chunk; ++it) {
-    t0(kKGenerate);
-    kFill<MULTI><<<kFillBlocks, kBlock, 0, stream>>>(js, pb);
-    t1(kKGenerate);
-    t0(kKMisc);
-    kFillCommit<<<1, 64, 0, stream>>>(pb.counters);
-    t1(kKMisc);
-    t0(kKExtend);
-    if (countStats) kExtend<MULTI, true, W><<<cfg.traceBlocks, kBlock, 0, stream>>>(js, pb);
-    else kExtend<MULTI, false, W><<<cfg.traceBlocks, kBlock, 0, stream>>>(js, pb);
-    t1(kKExtend);
-    if (GUIDED) {
-      t0(kKGuideInfer);
-      kGuideInfer<<<kGuideInferBlocks, kGuideInferThreads, 0, stream>>>(js, pb);
-      t1(kKGuideInfer);
-    }
-    t0(kKShade);
-    kShade<MULTI, GUIDED><<<cfg.shadeBlocks, kBlock, 0, stream>>>(js, pb);
-    t1(kKShade);
-    t0(kKConnect);
-    if (countStats) kConnect<MULTI, true, W><<<cfg.traceBlocks, kBlock, 0, stream>>>(js, pb);
-    else kConnect<MULTI, false, W><<<cfg.traceBlocks, kBlock, 0, stream>>>(js, pb);
-    t1(kKConnect);
-    t0(kKRetire);
-    kRetire<GUIDED><<<cfg.shadeBlocks, kBlock, 0, stream>>>(js, pb, countStats ? 1u : 0u);
-    t1(kKRetire);
-    t0(kKMisc);
-    kAdvance<<<1, 64, 0, stream>>>(pb.counters);
-    t1(kKMisc);
-    uint32_t* tmp = pb.qA;
-    pb.qA = pb.qB;
-    pb.qB = tmp;
-  }
-}
+struct Bounces {
+  const JobSet& js;
+  const PathBuffers& pb;
+  const LaunchConfig& cfg;
+  hipStream_t stream;
+  KernelTimer* timer;
+  bool late;  // some job has both an environment and emissive triangles
 
-// The chunk's kernels for a batch (each job's node width read by the
-// kernels) or for one job (its width compiled in).
-void launchChunkAny(const JobSet& js, const PathBuffers& pb, const LaunchConfig& cfg, uint32_t chunk,
-                    hipStream_t stream, KernelTimer* timer, bool multi, bool guided) {
-  if (multi) launchChunk<true, false, 0>(js, pb, cfg, chunk, stream, timer);
-  else if (guided && js.s.bvhWidth == 8) launchChunk<false, true, 8>(js, pb, cfg, chunk, stream, timer);
-  else if (guided) launchChunk<false, true, 4>(js, pb, cfg, chunk, stream, timer);
-  else if (js.s.bvhWidth == 8) launchChunk<false, false, 8>(js, pb, cfg, chunk, stream, timer);
-  else launchChunk<false, false, 4>(js, pb, cfg, chunk, stream, timer);
+  template <class F>
+  void timed(int id, F&& launch) const {
+    if (timer) timer->begin(id, stream);
+    launch();
+    if (timer) timer->end(id, stream);
+  }
+  // No more blocks than the pool has work for (an idle block still costs its
+  // dispatch); whole rounds of the 8 XCDs.
+  uint32_t blocks(uint32_t most, uint64_t items) const {
+    const uint64_t need = ((items + kBlock - 1) / kBlock + 7) & ~7ull;
+    return (uint32_t)std::min<uint64_t>(most, need);
+  }
+  void fillTrace(uint32_t p, bool fill) const {
+    const PathSet& out = pb.set[p ^ 1u];
+    if (fill)
+      timed(kKGenerate, [&] {
+        kFill<MULTI><<<blocks(8192, pb.capacity), kBlock, 0, stream>>>(js, pb, out, p);
+      });
+    timed(kKTrace, [&] {
+      const uint32_t n = std::min(blocks(cfg.traceBlocks, 2ull * pb.capacity), pb.traceThreads / kBlock);
+      if (cfg.countStats && late) kTrace<MULTI, true, W, true><<<n, kBlock, 0, stream>>>(js, pb, out, p);
+      else if (cfg.countStats) kTrace<MULTI, true, W, false><<<n, kBlock, 0, stream>>>(js, pb, out, p);
+      else if (late) kTrace<MULTI, false, W, true><<<n, kBlock, 0, stream>>>(js, pb, out, p);
+      else kTrace<MULTI, false, W, false><<<n, kBlock, 0, stream>>>(js, pb, out, p);
+    });
+    if (late) timed(kKConnect, [&] { kConnectLate<MULTI><<<blocks(2048, pb.capacity), kBlock, 0, stream>>>(js, pb, out, p); });
+    if (GUIDED && js.g.sampleCap > 0u)
+      timed(kKMisc, [&] { kHarvest<<<blocks(2048, pb.capacity), kBlock, 0, stream>>>(js.g, pb, p); });
+  }
+  // `chunk` bounces (even, so every chunk issues identical launches, which is
+  // what a captured graph replays); without `fill` no path starts.
+  void chunk(uint32_t n, bool fill) const {
+    for (uint32_t it = 0; it < n; ++it) {
+      const uint32_t p = (it & 1u) ^ 1u;
+      if (GUIDED)
+        timed(kKGuideInfer, [&] {
+          kGuideInfer<<<kGuideInferBlocks, kGuideInferThreads, 0, stream>>>(js, pb, pb.set[p], p);
+        });
+      timed(kKShade, [&] {
+        kShade<MULTI, GUIDED><<<blocks(cfg.shadeBlocks, pb.capacity), kBlock, 0, stream>>>(
+            js, pb, pb.set[p], pb.set[p ^ 1u], p, cfg.countStats ? 1u : 0u);
+      });
+      fillTrace(p, fill);
+    }
+  }
+};
+
+// f(bounces) with the kernels of a batch (each job's node width read by the
+// kernels) or of one job (its width compiled in).
+template <class F>
+void withBounces(const JobSet& js, const PathBuffers& pb, const LaunchConfig& cfg, hipStream_t stream,
+                 KernelTimer* timer, bool late, bool guided, F&& f) {
+  if (js.nJobs > 1) f(Bounces<true, false, 0>{js, pb, cfg, stream, timer, late});
+  else if (guided && js.s.bvhWidth == 8) f(Bounces<false, true, 8>{js, pb, cfg, stream, timer, late});
+  else if (guided) f(Bounces<false, true, 4>{js, pb, cfg, stream, timer, late});
+  else if (js.s.bvhWidth == 8) f(Bounces<false, false, 8>{js, pb, cfg, stream, timer, late});
+  else f(Bounces<false, false, 4>{js, pb, cfg, stream, timer, late});
 }
 
 }  // namespace
@@ -1197,7 +1125,8 @@ void renderJobs(const std::vector<RenderJobDesc>& jobs, const PathBuffers& pb, c
   std::vector<DevScene> scenes(nJobs);
   std::vector<PassInfo> passes(nJobs);
   uint64_t total = 0;
-  int maxDepth = 0;
+  int maxDepth = 1;
+  bool late = false;
   for (uint32_t j = 0; j < nJobs; ++j) {
     const RenderJobDesc& d = jobs[j];
     scenes[j] = d.scene;
@@ -1212,6 +1141,7 @@ void renderJobs(const std::vector<RenderJobDesc>& jobs, const PathBuffers& pb, c
     if (pi.pixels > pb.ringPaths) throw std::runtime_error("renderJobs: results ring smaller than one sample");
     total += (uint64_t)d.n * pi.pixels;
     maxDepth = std::max(maxDepth, d.scene.maxDepth);
+    late = late || (d.scene.hasEnv && d.scene.hasSurfaceLight);
   }
   if (total >= (1ull << 31)) throw std::runtime_error("renderJobs: more than 2^31 paths in one call");
   JobSet js{};
@@ -1234,6 +1164,7 @@ void renderJobs(const std::vector<RenderJobDesc>& jobs, const PathBuffers& pb, c
     js.passes = (const PassInfo*)dPasses;
   }
   if (total == 0) return;
+  if (late && !pb.sh.lateQ) throw std::runtime_error("renderJobs: no buffers for late light samples");
   auto t0 = [&](int k) {
     if (timer) timer->begin(k, stream);
   };
@@ -1241,8 +1172,8 @@ void renderJobs(const std::vector<RenderJobDesc>& jobs, const PathBuffers& pb, c
     if (timer) timer->end(k, stream);
   };
   const uint32_t chunk = std::max<uint32_t>(2, (cfg.chunk + 1) & ~1u);
-  // Paths started during chunk c have finished `lag` chunks later: a path
-  // has at most maxDepth vertices, one per bounce.
+  // Paths started by the end of chunk c have finished `lag` chunks later: a
+  // path has at most maxDepth vertices, one per bounce.
   const uint32_t lag = ((uint32_t)maxDepth + chunk - 1) / chunk;
   std::vector<uint32_t> acc(nJobs, 0);  // samples of each job added to its films
   uint32_t front = 0;                    // first job not completely added
@@ -1251,8 +1182,10 @@ void renderJobs(const std::vector<RenderJobDesc>& jobs, const PathBuffers& pb, c
   };
   uint32_t limit = (uint32_t)std::min<uint64_t>(total, accPid() + pb.ringPaths);
   t0(kKMisc);
-  kInitRender<<<256, kBlock, 0, stream>>>(pb, limit);
+  kInitRender<<<1, 64, 0, stream>>>(pb.counters, limit);
   t1(kKMisc);
+  auto bounces = [&](KernelTimer* t, auto&& f) { withBounces(js, pb, cfg, stream, t, late, guide != nullptr, f); };
+  bounces(timer, [&](const auto& b) { b.fillTrace(0u, true); });
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   struct GraphFree {
@@ -1268,24 +1201,27 @@ void renderJobs(const std::vector<RenderJobDesc>& jobs, const PathBuffers& pb, c
   // replay graphs.
   if (cfg.useGraph && !timer) {
     hipOk(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
-    launchChunkAny(js, pb, cfg, chunk, stream, nullptr, nJobs > 1, guide != nullptr);
+    bounces(nullptr, [&](const auto& b) { b.chunk(chunk, true); });
     hipOk(hipStreamEndCapture(stream, &graph), "hipStreamEndCapture");
     hipOk(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "hipGraphInstantiate");
   }
   std::vector<uint32_t> startedBy;
+  uint64_t next = std::min<uint64_t>(limit, pb.capacity);  // paths started so far
   for (uint32_t c = 0;; ++c) {
     if (exec) {
       t0(kKGraph);
       hipOk(hipGraphLaunch(exec, stream), "hipGraphLaunch");
       t1(kKGraph);
     } else {
-      launchChunkAny(js, pb, cfg, chunk, stream, timer, nJobs > 1, guide != nullptr);
+      bounces(timer, [&](const auto& b) { b.chunk(chunk, next < total); });
     }
     uint32_t cnt[kNumCounters];
     hipOk(hipMemcpyAsync(cnt, pb.counters, sizeof(cnt), hipMemcpyDeviceToHost, stream), "counter readback");
     hipOk(hipStreamSynchronize(stream), "hipStreamSynchronize");
-    uint32_t live = cnt[kCntA], next = cnt[kCntNext];
-    startedBy.push_back(next);
+    // the chunk's last bounce (p = 0) left the next one's counters in set 1
+    const uint32_t live = cnt[kCntSet + kCntLive];
+    next = cnt[kCntSet + kCntNext];
+    startedBy.push_back((uint32_t)next);
     uint64_t done = live == 0 ? next : (c >= lag ? startedBy[c - lag] : 0u);
     for (uint32_t j = front; j < nJobs && passes[j].pidBase < done; ++j) {
       const PassInfo& pi = passes[j];

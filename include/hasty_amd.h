@@ -230,7 +230,7 @@ int hasty_trace_hits_device(HastyScene* scene, const HastyRay* d_rays, uint32_t 
 int hasty_trace_hits_device_noalloc(HastyScene* scene, const HastyRay* d_rays, uint32_t n, HastyHit* d_hits);
 
 /* Per-kernel timing with HIP events on the scene's stream (flags bit 0;
- * with bit 2 only the closest-hit extension launches are timed, which keeps
+ * with bit 2 only the traversal launches (pt_trace) are timed, which keeps
  * the events' own cost out of a timed render) and device counters (flags
  * bit 1, see hasty_counters). */
 typedef struct HastyKernelStat {
@@ -252,7 +252,7 @@ int hasty_counters(HastyScene* scene, uint64_t* out5);
 int hasty_counters_ex(HastyScene* scene, uint64_t* out, uint32_t n);
 
 /* Launch-shape knobs: path slots in flight (paths are regenerated into
- * freed slots; default 2^23, at least 2^16 unless the film is smaller) and
+ * freed slots; default 2^24, at least 2^16 unless the film is smaller) and
  * the grid sizes of the traversal and shading kernels.  0 keeps the current
  * value.  Images do not depend on these. */
 int hasty_set_launch(HastyScene* scene, uint32_t path_slots, uint32_t trace_blocks, uint32_t shade_blocks);
