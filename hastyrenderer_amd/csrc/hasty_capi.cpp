@@ -198,8 +198,7 @@ struct HastyScene {
   size_t filmFloats = 0;
 
   // trace entry point
-  uint2* traceOverflow = nullptr;
-  uint32_t traceOverflowThreads = 0;
+  DevBuf traceOverflow;
   DevBuf traceIO;  // rays in, hits out of the host-pointer trace call
 
   // Halton offsets of a render call and the job tables of a batch
@@ -269,7 +268,6 @@ struct HastyScene {
     for (void* p : {(void*)guideSamples, (void*)guideCount})
       if (p) (void)hipFree(p);
     if (dFilm) (void)hipFree(dFilm);
-    if (traceOverflow) (void)hipFree(traceOverflow);
     if (stream) (void)hipStreamDestroy(stream);
   }
 
@@ -921,13 +919,12 @@ static void uploadScene(HastyScene& S) {
   S.applySettings();
 }
 
-// The scene's traversal stack overflow buffer (256 blocks of threads).
-static void ensureTraceOverflow(HastyScene* s) {
-  if (!s->traceOverflow) {
-    const uint32_t threads = 256 * hasty::kBlock;
-    HIPCHECK(hipMalloc(&s->traceOverflow, sizeof(uint2) * threads * hasty::kStackOvf));
-    s->traceOverflowThreads = threads;
-  }
+// Overflow entries for a query of n rays on the scene's current BVH: a slice
+// per thread of its grid.
+static uint2* traceOverflow(HastyScene* s, uint32_t n, size_t* entries, uint32_t* slice) {
+  *slice = hasty::overflowSlice(s->bvh().width, s->bvh().depth);
+  *entries = (size_t)hasty::queryBlocks(n) * hasty::kBlock * *slice;
+  return (uint2*)s->traceOverflow.ensure(*entries * sizeof(uint2));
 }
 
 namespace hasty {
@@ -1305,14 +1302,16 @@ int hasty_trace_closest(HastyScene* s, const float* rays, uint32_t n, uint32_t* 
   if (n == 0) return 0;
   try {
     HIPCHECK(hipSetDevice(s->device));
-    ensureTraceOverflow(s);
+    size_t entries;
+    uint32_t slice;
+    uint2* ovf = traceOverflow(s, n, &entries, &slice);
     // rays, triangle ids and (t, u, v) share the scene's trace buffer
     char* io = (char*)s->traceIO.ensure((sizeof(float) * 6 + sizeof(int32_t) + sizeof(float) * 3) * (size_t)n);
     float* dRays = (float*)io;
     int32_t* dTri = (int32_t*)(io + sizeof(float) * 6 * (size_t)n);
     float* dTuv = (float*)(io + (sizeof(float) * 6 + sizeof(int32_t)) * (size_t)n);
     HIPCHECK(hipMemcpy(dRays, rays, sizeof(float) * 6 * n, hipMemcpyHostToDevice));
-    hasty::launchTraceClosest(s->dev, dRays, n, dTri, dTuv, s->traceOverflow, s->traceOverflowThreads, s->stream);
+    hasty::launchTraceClosest(s->dev, dRays, n, dTri, dTuv, ovf, entries, slice, s->stream);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(s->stream));
     HIPCHECK(hipMemcpy(tri, dTri, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
@@ -1346,9 +1345,10 @@ int hasty_trace_hits_device(HastyScene* s, const HastyRay* dRays, uint32_t n, Ha
   if (n == 0) return 0;
   try {
     HIPCHECK(hipSetDevice(s->device));
-    ensureTraceOverflow(s);
-    hasty::launchTraceHits(s->dev, (const float*)dRays, n, (hasty::HitRecord*)dHits, s->traceOverflow,
-                           s->traceOverflowThreads, s->stream);
+    size_t entries;
+    uint32_t slice;
+    uint2* ovf = traceOverflow(s, n, &entries, &slice);
+    hasty::launchTraceHits(s->dev, (const float*)dRays, n, (hasty::HitRecord*)dHits, ovf, entries, slice, s->stream);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(s->stream));
     return 0;

@@ -224,22 +224,33 @@ struct HitRecord {
 };
 static_assert(sizeof(HitRecord) == 32, "HitRecord is 32 bytes");
 
-// Closest-hit records for n rays (6 floats each).  `overflow` holds
-// kStackOvf stack entries for each of the overflowThreads threads the grid
-// may use (a multiple of kBlock).
+// Stack entries per lane that a traversal of a BVH of this width and depth
+// can need beyond the kStackLds in LDS: at most width - 1 per inner level,
+// and the root.
+constexpr uint32_t overflowSlice(int width, int depth) {
+  const int need = (width - 1) * depth + 1;
+  return need > kStackLds ? (uint32_t)(need - kStackLds) : 0u;
+}
+// Blocks of a query of n rays: the chip's 8 blocks per CU at most.
+constexpr uint32_t kQueryBlocks = 2048;
+uint32_t queryBlocks(uint32_t n);
+
+// Closest-hit records for n rays (6 floats each).  `overflow` holds `entries`
+// stack entries, `slice` (overflowSlice of the scene's BVH) for each thread;
+// the grid is cut to what they allow.
 void launchTraceHits(const hdev::DevScene& scene, const float* dRays, uint32_t n, HitRecord* dHits, uint2* dOverflow,
-                     uint32_t overflowThreads, hipStream_t stream);
+                     size_t entries, uint32_t slice, hipStream_t stream);
 
 // Caustic photons as guide training samples (4 float4 each, appended at
 // atomicAdd(sampleCount) below cap) from `count` light paths of pass `pass`;
-// `overflow` as for launchTraceHits.  Nothing without surface lights.
+// `overflow`: kStackOvf entries for each of the overflowThreads threads (a
+// multiple of kBlock).  Nothing without surface lights.
 void launchGuidePhotons(const hdev::DevScene& scene, uint32_t pass, uint32_t count, uint2* dOverflow,
                         uint32_t overflowThreads, float4* samples, uint32_t* sampleCount, uint32_t cap,
                         hipStream_t stream);
 
 // Closest hit for n rays (6 floats each): tri, t, u, v.
 void launchTraceClosest(const hdev::DevScene& scene, const float* dRays, uint32_t n, int32_t* dTri, float* dTuv,
-                        uint2* dOverflow, uint32_t overflowThreads, hipStream_t stream);
-
+                        uint2* dOverflow, size_t entries, uint32_t slice, hipStream_t stream);
 
 }  // namespace hasty

@@ -873,16 +873,24 @@ __global__ void __launch_bounds__(kGuideInferThreads) HASTY_WAVES_ATTR_(HASTY_GU
   }
 }
 
-__global__ void __launch_bounds__(kBlock) kTraceRays(DevScene s, const float* rays, uint32_t n, int32_t* tri,
-                                                     float* tuv, uint2* overflow) {
+// Batched closest-hit queries, grid-stride over the rays.  Bound, as kTrace,
+// by dependent node fetches: the time falls with the waves in flight, so the
+// registers are held to 8 waves per SIMD and the grid fills the chip (the
+// caller's overflow slices allowing).  `slice`: overflow entries per thread.
+// 4.2M incoherent rays of the GGX grid: 4.54 ms with 256 blocks (one wave per
+// SIMD), 1.14 ms with 2048.
+template <int W>
+__global__ void __launch_bounds__(kBlock) HASTY_TRACE_ATTR kTraceRays(DevScene s, const float* rays, uint32_t n,
+                                                                     int32_t* tri, float* tuv, uint2* overflow,
+                                                                     uint32_t slice) {
   __shared__ uint2 stack[kStackLds * kBlock];
   uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
   uint32_t stride = gridDim.x * blockDim.x;
-  uint2* ovf = overflow + (size_t)gtid * kStackOvf;
+  uint2* ovf = overflow + (size_t)gtid * slice;
   for (uint32_t q = gtid; q < n; q += stride) {
     const float* r = rays + (size_t)q * 6;
-    Hit h = traceClosest<kStackLds, kStackOvf>(s, v3(r[0], r[1], r[2]), v3(r[3], r[4], r[5]), stack + threadIdx.x, kBlock, ovf,
-                                    nullptr, nullptr);
+    Hit h = traceClosest<kStackLds, kStackOvf, W>(s, v3(r[0], r[1], r[2]), v3(r[3], r[4], r[5]), stack + threadIdx.x,
+                                                  kBlock, ovf, nullptr, nullptr);
     tri[q] = h.tri;
     tuv[(size_t)q * 3] = h.t;
     tuv[(size_t)q * 3 + 1] = h.u;
@@ -890,17 +898,19 @@ __global__ void __launch_bounds__(kBlock) kTraceRays(DevScene s, const float* ra
   }
 }
 
-// Closest-hit records (HitRecord) of n rays, grid-stride over the rays.
-__global__ void __launch_bounds__(kBlock) kTraceHits(DevScene s, const float* rays, uint32_t n, HitRecord* hits,
-                                                     uint2* overflow) {
+// The same with closest-hit records (HitRecord).
+template <int W>
+__global__ void __launch_bounds__(kBlock) HASTY_TRACE_ATTR kTraceHits(DevScene s, const float* rays, uint32_t n,
+                                                                     HitRecord* hits, uint2* overflow,
+                                                                     uint32_t slice) {
   __shared__ uint2 stack[kStackLds * kBlock];
   uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
   uint32_t stride = gridDim.x * blockDim.x;
-  uint2* ovf = overflow + (size_t)gtid * kStackOvf;
+  uint2* ovf = overflow + (size_t)gtid * slice;
   for (uint32_t q = gtid; q < n; q += stride) {
     const float* r = rays + (size_t)q * 6;
-    Hit h = traceClosest<kStackLds, kStackOvf>(s, v3(r[0], r[1], r[2]), v3(r[3], r[4], r[5]), stack + threadIdx.x,
-                                                kBlock, ovf, nullptr, nullptr);
+    Hit h = traceClosest<kStackLds, kStackOvf, W>(s, v3(r[0], r[1], r[2]), v3(r[3], r[4], r[5]), stack + threadIdx.x,
+                                                  kBlock, ovf, nullptr, nullptr);
     HitRecord rec;
     if (h.tri < 0) {
       rec.geomID = rec.primID = 0xFFFFFFFFu;
@@ -1250,15 +1260,36 @@ void renderJobs(const std::vector<RenderJobDesc>& jobs, const PathBuffers& pb, c
   if (front != nJobs) throw std::runtime_error("renderJobs: not every sample was accumulated");
 }
 
-void launchTraceHits(const DevScene& s, const float* dRays, uint32_t n, HitRecord* dHits, uint2* dOverflow,
-                     uint32_t overflowThreads, hipStream_t stream) {
+uint32_t queryBlocks(uint32_t n) {
+  return std::min<uint32_t>((n + kBlock - 1) / kBlock, kQueryBlocks);
+}
+
+namespace {
+// Blocks of a query on an overflow array of `entries`, `slice` per thread.
+uint32_t queryGrid(uint32_t n, size_t entries, uint32_t slice) {
   // the grid-stride index q + stride stays below 2^32
   if (n >= 0x80000000u) throw std::runtime_error("more than 2^31 - 1 rays in one query");
-  uint32_t blocks = (n + kBlock - 1) / kBlock;
-  uint32_t maxBlocks = overflowThreads / kBlock;
-  if (blocks > maxBlocks) blocks = maxBlocks;
+  if (slice == 0) return queryBlocks(n);
+  const size_t most = entries / ((size_t)slice * kBlock);
+  if (most == 0) throw std::runtime_error("traversal stack overflow array smaller than one block's");
+  return (uint32_t)std::min<size_t>(queryBlocks(n), most);
+}
+}  // namespace
+
+void launchTraceHits(const DevScene& s, const float* dRays, uint32_t n, HitRecord* dHits, uint2* dOverflow,
+                     size_t entries, uint32_t slice, hipStream_t stream) {
+  const uint32_t blocks = queryGrid(n, entries, slice);
   if (blocks == 0) return;
-  kTraceHits<<<blocks, kBlock, 0, stream>>>(s, dRays, n, dHits, dOverflow);
+  if (s.bvhWidth == 8) kTraceHits<8><<<blocks, kBlock, 0, stream>>>(s, dRays, n, dHits, dOverflow, slice);
+  else kTraceHits<4><<<blocks, kBlock, 0, stream>>>(s, dRays, n, dHits, dOverflow, slice);
+}
+
+void launchTraceClosest(const DevScene& s, const float* dRays, uint32_t n, int32_t* dTri, float* dTuv, uint2* dOverflow,
+                        size_t entries, uint32_t slice, hipStream_t stream) {
+  const uint32_t blocks = queryGrid(n, entries, slice);
+  if (blocks == 0) return;
+  if (s.bvhWidth == 8) kTraceRays<8><<<blocks, kBlock, 0, stream>>>(s, dRays, n, dTri, dTuv, dOverflow, slice);
+  else kTraceRays<4><<<blocks, kBlock, 0, stream>>>(s, dRays, n, dTri, dTuv, dOverflow, slice);
 }
 
 void launchGuidePhotons(const DevScene& s, uint32_t pass, uint32_t count, uint2* dOverflow, uint32_t overflowThreads,
@@ -1269,16 +1300,6 @@ void launchGuidePhotons(const DevScene& s, uint32_t pass, uint32_t count, uint2*
   if (blocks > maxBlocks) blocks = maxBlocks;
   if (blocks == 0) return;
   kGuidePhotons<<<blocks, kBlock, 0, stream>>>(s, pass, count, dOverflow, samples, sampleCount, cap);
-}
-
-void launchTraceClosest(const DevScene& s, const float* dRays, uint32_t n, int32_t* dTri, float* dTuv, uint2* dOverflow,
-                        uint32_t overflowThreads, hipStream_t stream) {
-  if (n >= 0x80000000u) throw std::runtime_error("more than 2^31 - 1 rays in one query");
-  uint32_t blocks = (n + kBlock - 1) / kBlock;
-  uint32_t maxBlocks = overflowThreads / kBlock;
-  if (blocks > maxBlocks) blocks = maxBlocks;
-  if (blocks == 0) return;
-  kTraceRays<<<blocks, kBlock, 0, stream>>>(s, dRays, n, dTri, dTuv, dOverflow);
 }
 
 }  // namespace hasty

@@ -4,9 +4,9 @@
 // The only device memory the query needs beyond its rays and hits is the
 // traversal stack's overflow part (stack entries past the kStackLds kept in
 // LDS).  hasty_trace_hits_device takes it from a buffer the scene allocates on
-// first use; here it is `scratch`, a file-scope device array sized for a
-// fixed grid of kNoAllocBlocks blocks (9 MiB), which every GPU the library runs
-// on holds until the process ends.  Its device address is looked up once per
+// first use; here it is `scratch`, a file-scope device array of 9 MiB (64 blocks
+// with the deepest stack; shallower trees get more blocks), which every GPU the
+// library runs on holds until the process ends.  Its device address is looked up once per
 // device with hipGetSymbolAddress (the array's name is only a host-side
 // stand-in) and passed to the same kernel as hasty_trace_hits_device uses.
 // Stack slices are written before they are read, so nothing needs clearing
@@ -23,9 +23,7 @@
 #include "pt_kernels.h"
 
 namespace {
-constexpr uint32_t kNoAllocBlocks = 64;
-constexpr uint32_t kNoAllocThreads = kNoAllocBlocks * hasty::kBlock;
-constexpr size_t kScratchEntries = (size_t)kNoAllocThreads * hasty::kStackOvf;  // 9 MiB of uint2
+constexpr size_t kScratchEntries = (size_t)64 * hasty::kBlock * hasty::kStackOvf;  // 9 MiB of uint2
 }  // namespace
 
 static __device__ __align__(256) uint2 scratch[kScratchEntries];
@@ -83,7 +81,8 @@ extern "C" int hasty_trace_hits_device_noalloc(HastyScene* scene, const HastyRay
     hipOk(hipSetDevice(v.device), "hipSetDevice");
     uint2* ovf = scratchOn(v.device);
     hasty::launchTraceHits(v.dev, reinterpret_cast<const float*>(d_rays), n,
-                           reinterpret_cast<hasty::HitRecord*>(d_hits), ovf, kNoAllocThreads, v.stream);
+                           reinterpret_cast<hasty::HitRecord*>(d_hits), ovf, kScratchEntries,
+                           hasty::overflowSlice(v.bvhWidth, v.bvhDepth), v.stream);
     hipOk(hipGetLastError(), "kTraceHits launch");
     hipOk(hipStreamSynchronize(v.stream), "hipStreamSynchronize");
     return 0;

@@ -223,7 +223,7 @@ int hasty_trace_hits_device(HastyScene* scene, const HastyRay* d_rays, uint32_t 
  * memory (code under hipGraph capture, tight serving loops, harnesses that
  * forbid hipMalloc): the query of hasty_trace_hits_device with its traversal
  * stack overflow in a static 9 MiB device array of the library instead of a
- * scene buffer, on a fixed grid of 64 blocks.  Allocates nothing (no
+ * scene buffer, on the grid it allows.  Allocates nothing (no
  * hipMalloc / hipFree); n at most 2^31 - 1; hits 16-byte aligned.  Every call
  * on one GPU shares the array: calls that overlap on one GPU race.
  * Synchronous on the scene's stream. */
