@@ -126,6 +126,7 @@ struct JobSet {
   const PassInfo* passes;
   uint32_t nJobs;
   uint32_t paths;  // over all jobs
+  uint32_t finishPaths;  // the last paths are finished one by one from this many (0: never)
   GuideRun g;      // read by the guided kernels only
 };
 
@@ -164,6 +165,7 @@ enum KernelId {
   kKGenerate = 0,
   kKTrace,
   kKShade,
+  kKFinish,
   kKConnect,
   kKAccumulate,
   kKMisc,

@@ -42,6 +42,7 @@ const char* kernelName(int id) {
     case kKGenerate: return "pt_generate";
     case kKTrace: return "pt_trace";
     case kKShade: return "pt_shade";
+    case kKFinish: return "pt_finish";
     case kKConnect: return "pt_connect_late";
     case kKAccumulate: return "pt_accumulate";
     case kKGraph: return "pt_graph_chunk";
@@ -342,7 +343,7 @@ __global__ void __launch_bounds__(kBlock) HASTY_TRACE_ATTR kTrace(JobSet js, Pat
     nodes = tris = rays = 0;
   }
   const uint32_t begin = startCount(pb, c), live = c[kCntA] + begin;
-  if (gtid == 0) {  // the next bounce's counters
+  if (gtid == 0) {  // the next bounce's counters (none alive after kFinish)
     uint32_t* d = pb.counters + (p ^ 1u) * kCntSet;
     d[kCntA] = 0u, d[kCntS] = 0u, d[kCntEnded] = 0u, d[kCntLate] = 0u;
     d[kCntLive] = live;
@@ -385,17 +386,39 @@ __device__ inline bool guideThroughputOk(const GuideRun& g, V3 beta) {
   return fmaxf(beta.x, fmaxf(beta.y, beta.z)) <= g.maxThroughput;
 }
 
-// What a vertex leaves: the path's state where it goes on (o, d, pdf, beta,
-// flags, md, with L up to the vertex's own emission) and its light sample.
-struct Vertex {
+// A path on its way to a vertex: its ray, what it has gathered, and its media
+// stack (txs: the stack's albedo texels, or null).
+struct Path {
   V3 o, d;
   float pdf;
   V3 beta, L;
   uint32_t draws, flags;
-  int32_t tri;
+  int32_t prevTri;
+  uint32_t pid;
   Media md;
-  bool go;  // the path goes on with the ray (o, d)
-  bool cast;  // its light sample needs a shadow ray (record i of pb.sh)
+  uint32_t* txs;
+};
+__device__ inline Path loadPath(const PathSet& ps, uint32_t i, uint4 st) {
+  Path pt;
+  const float4 o = ps.rayO[i], d = ps.rayD[i];
+  pt.o = f4xyz(o), pt.d = f4xyz(d), pt.pdf = d.w;
+  pt.draws = st.x, pt.flags = st.y, pt.prevTri = (int32_t)st.z, pt.pid = st.w;
+  // a path's first vertex starts from throughput 1 and radiance 0 (not
+  // stored by kFill)
+  const bool first = (st.y & 0xFFu) == 0u;
+  pt.beta = first ? v3(1.0f, 1.0f, 1.0f) : f4xyz(ps.beta[i]);
+  pt.L = first ? v3(0.0f, 0.0f, 0.0f) : f4xyz(ps.L[i]);
+  pt.txs = ps.mediaTx ? ps.mediaTx + (size_t)i * kMaxMedia : nullptr;
+  loadMedia(ps, i, st.y, pt.txs, pt.md);
+  return pt;
+}
+// What a vertex did: whether the path goes on (with the state left in it),
+// and the shadow ray of its light sample with the radiance to add if clear.
+struct Vertex {
+  bool go, cast;
+  V3 so, sd, c;
+  float st;  // t of the target triangle (+inf: environment)
+  int32_t target;
 };
 
 // The term of a light sample that nothing blocks, t2 = thr (fD + fC) cos / pL
@@ -424,47 +447,41 @@ __device__ inline V3 lightRadiance(const DevScene& s, int32_t tri, V3 hx, V3 hn,
   return mul(Tb, Le);
 }
 
-// One vertex of path i of the set `in`, whose ray met h4.
+// One vertex of path i, whose ray met h4.
 template <bool GUIDED>
 __device__ inline void shadeVertex(const DevScene& s, const PassInfo& pi, const GuideRun& g, const PathBuffers& pb,
-                                   const PathSet& in, uint32_t i, const uint4 st, Vertex& vx) {
+                                   uint32_t i, Path& pt, float4 h4, Vertex& vx) {
   const bool twoStrategies = s.hasLight && s.useMIS;
-  int depth = (int)(st.y & 0xFFu);
-  int wavelength = (int)((st.y >> 8) & 0x3u) - 1;
+  const uint32_t flags = pt.flags;
+  int depth = (int)(flags & 0xFFu);
+  int wavelength = (int)((flags >> 8) & 0x3u) - 1;
   // per-entry albedo texels of the media stack (albedo-textured scenes)
-  uint32_t* txs = s.texturedMedia ? in.mediaTx + (size_t)i * kMaxMedia : nullptr;
-  Media& md = vx.md;
-  loadMedia(in, i, st.y, txs, md);
-  int32_t prevTri = (int32_t)st.z;
-  const float4 ro4 = in.rayO[i], rd4 = in.rayD[i], h4 = pb.hit[i];
-  V3 ro = f4xyz(ro4), rd = f4xyz(rd4);
+  uint32_t* txs = s.texturedMedia ? pt.txs : nullptr;
+  Media& md = pt.md;
+  const V3 ro = pt.o, rd = pt.d;
   const int32_t tri = __float_as_int(h4.w);
-  // a path's first vertex starts from throughput 1 and radiance 0 (not
-  // stored by kFill)
-  const V3 b0 = depth == 0 ? v3(1.0f, 1.0f, 1.0f) : f4xyz(in.beta[i]);
+  const V3 b0 = pt.beta;
   V3 beta = b0;
-  const float4 L4 = depth == 0 ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : in.L[i];
-  V3& L = vx.L;
-  L = f4xyz(L4);
+  V3& L = pt.L;
   vx.go = vx.cast = false;
-  uint32_t nrec = GUIDED ? (st.y >> kRecShift) & 3u : 0u;
-  if (GUIDED && depth > 0 && nrec > 0 && ((st.y >> (kRecShift + 2)) & 1u)) {
+  uint32_t nrec = GUIDED ? (flags >> kRecShift) & 3u : 0u;
+  if (GUIDED && depth > 0 && nrec > 0 && ((flags >> (kRecShift + 2)) & 1u)) {
     // radiance before the continuation of the last recorded vertex
-    g.rec[(size_t)st.w * 12 + 6 * (nrec - 1) + 5] = L4;
+    g.rec[(size_t)pt.pid * 12 + 6 * (nrec - 1) + 5] = f4(L, 0.0f);
   }
   hrng::Stream rng;
   {
     uint32_t k, pixel;
-    pathPixel(pi, st.w, &pixel, &k);
+    pathPixel(pi, pt.pid, &pixel, &k);
     rng = hrng::make_stream(s.seed, pixel, pi.first + k, hrng::kDomainPath);
-    rng.counter = st.x;
+    rng.counter = pt.draws;
   }
   const EnvUV sky = tri < 0 && s.hasEnv ? envUV(rd) : EnvUV{0.0f, 0.0f, 0.0f};
   const float pSurf = !s.hasEnv ? 1.0f : (s.hasSurfaceLight ? 0.5f : 0.0f);
   // The BSDF sample that produced this ray: self-intersection, then MIS.
   if (depth > 0) {
-    if (tri == prevTri) return;
-    float pB = rd4.w;
+    if (tri == pt.prevTri) return;
+    float pB = pt.pdf;
     float sum = 0.0f;
     if (twoStrategies) {
       float pL;
@@ -481,7 +498,7 @@ __device__ inline void shadeVertex(const DevScene& s, const PassInfo& pi, const 
     float w = powci<2>(pB) / sum;
     beta = beta * w;
   }
-  const uint32_t ri = depth == 0 ? st.w % pb.ringPaths : 0u;
+  const uint32_t ri = depth == 0 ? pt.pid % pb.ringPaths : 0u;
   if (tri < 0) {
     V3 T = beersLaw(mediaTransmittance(s, md), 1e6f);
     V3 Lc = mul(T, s.hasEnv ? envLookup(s, sky.u, sky.v) : v3(s.bg[0], s.bg[1], s.bg[2]));
@@ -587,11 +604,8 @@ __device__ inline void shadeVertex(const DevScene& s, const PassInfo& pi, const 
           pb.sh.lateT[i] = f4(Tc, 0.0f);
         }
       }
-      if (vx.cast) {
-        pb.sh.o[i] = f4(so, tT);
-        pb.sh.d[i] = f4(sd, __int_as_float(target));
-        pb.sh.c[i] = f4(Lt, 0.0f);
-      }
+      vx.so = so, vx.sd = sd, vx.c = Lt;
+      vx.st = tT, vx.target = target;
     }
   }
   // ---- BSDF strategy (MIS.cpp:6-26, Scene.cpp:328-338)
@@ -642,16 +656,16 @@ __device__ inline void shadeVertex(const DevScene& s, const PassInfo& pi, const 
   if (isZero(t2)) return;
   mediaUpdate(md, it, wo, bs.dir, texel, txs);
   vx.go = true;
-  vx.o = offsetOrigin(it, bs.outside);
-  vx.d = bs.dir;
-  vx.pdf = bs.pdf;
-  vx.beta = mul(beta, t2);
-  vx.draws = rng.counter;
-  vx.tri = tri;
+  pt.o = offsetOrigin(it, bs.outside);
+  pt.d = bs.dir;
+  pt.pdf = bs.pdf;
+  pt.beta = mul(beta, t2);
+  pt.draws = rng.counter;
+  pt.prevTri = tri;
   uint32_t recBits = 0u;
   if (GUIDED) {
     if (guided && nrec < 2u && g.sampleCap > 0u) {  // records only when training
-      float4* rr = g.rec + (size_t)st.w * 12 + 6 * nrec;
+      float4* rr = g.rec + (size_t)pt.pid * 12 + 6 * nrec;
       V3 nf = dot(it.ng, wo) >= 0.0f ? it.ng : -it.ng;
       rr[0] = f4(it.x, 0.0f);
       rr[1] = f4(nf, 0.0f);
@@ -664,7 +678,15 @@ __device__ inline void shadeVertex(const DevScene& s, const PassInfo& pi, const 
       recBits = nrec << kRecShift;
     }
   }
-  vx.flags = packFlags(depth + 1, wavelength, md) | recBits | (st.y & ~((1u << kJobShift) - 1u));
+  pt.flags = packFlags(depth + 1, wavelength, md) | recBits | (flags & ~((1u << kJobShift) - 1u));
+}
+
+// The last paths of a render: when none is left to start and so few are alive
+// that launches would only run their longest rays one after another, kFinish
+// runs every path to its end by itself (and the bounce kernels, which test the
+// same counters, find nothing to do).
+__device__ inline bool finishing(const JobSet& js, const uint32_t* c) {
+  return js.finishPaths > 0u && c[kCntNext] >= js.paths && c[kCntLive] <= js.finishPaths;
 }
 
 // Bounce p: every path alive in `in` one vertex further, those that go on
@@ -678,50 +700,126 @@ __global__ void __launch_bounds__(kBlock) HASTY_SHADE_ATTR kShade(JobSet js, Pat
   __shared__ uint2 ldsWave[kBlock / 64];
   __shared__ unsigned long long ldsBase;
   uint32_t* c = pb.counters + p * kCntSet;
+  if (finishing(js, c)) return;
   const uint32_t n = c[kCntLive];
   uint32_t overflowed = 0;
   for (uint32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock) {
     const uint32_t i = base + threadIdx.x;
     Vertex vx;
     vx.go = vx.cast = false;
-    uint4 st = make_uint4(0u, 0u, 0u, 0u);
-    uint32_t job = 0u;
+    Path pt;
+    uint32_t stFlags = 0u;
     if (i < n) {
-      st = in.state[i];
-      job = jobOf<MULTI>(js, st);
+      const uint4 st = in.state[i];
+      stFlags = st.y;
+      const uint32_t job = jobOf<MULTI>(js, st);
+      pt = loadPath(in, i, st);
+      const float4 h4 = pb.hit[i];
       forJob<MULTI>(js, job, [&](const DevScene& s, const PassInfo& pi) {
-        shadeVertex<GUIDED>(s, pi, js.g, pb, in, i, st, vx);
+        shadeVertex<GUIDED>(s, pi, js.g, pb, i, pt, h4, vx);
       });
+      if (vx.cast) {
+        pb.sh.o[i] = f4(vx.so, vx.st);
+        pb.sh.d[i] = f4(vx.sd, __int_as_float(vx.target));
+        pb.sh.c[i] = f4(vx.c, 0.0f);
+        if (MULTI) pb.sh.job[i] = job;
+      }
     }
     uint32_t idxN, idxS;
     blockAppend2((unsigned long long*)(c + kCntA), vx.go, vx.cast, ldsWave, &ldsBase, &idxN, &idxS);
     uint32_t dest = idxN;
     if (vx.go) {
-      out.rayO[idxN] = f4(vx.o, 0.0f);
-      out.rayD[idxN] = f4(vx.d, vx.pdf);
-      out.beta[idxN] = f4(vx.beta, 0.0f);
-      out.L[idxN] = f4(vx.L, 0.0f);
-      out.state[idxN] = make_uint4(vx.draws, vx.flags, (uint32_t)vx.tri, st.w);
-      if (vx.md.n > 0) {
-        storeMedia(out, idxN, vx.md);
+      out.rayO[idxN] = f4(pt.o, 0.0f);
+      out.rayD[idxN] = f4(pt.d, pt.pdf);
+      out.beta[idxN] = f4(pt.beta, 0.0f);
+      out.L[idxN] = f4(pt.L, 0.0f);
+      out.state[idxN] = make_uint4(pt.draws, pt.flags, (uint32_t)pt.prevTri, pt.pid);
+      if (pt.md.n > 0) {
+        storeMedia(out, idxN, pt.md);
         if (in.mediaTx)
-          for (int k = 0; k < vx.md.n; ++k)
+          for (int k = 0; k < pt.md.n; ++k)
             out.mediaTx[(size_t)idxN * kMaxMedia + k] = in.mediaTx[(size_t)i * kMaxMedia + k];
       }
     } else if (i < n) {  // the path ends here (but for its shadow ray, if any)
-      const uint32_t ri = st.w % pb.ringPaths;
+      const uint32_t ri = pt.pid % pb.ringPaths;
       dest = ri | kDestRing;
-      pb.ringL[ri] = f4(vx.L, 0.0f);
-      overflowed += (st.y >> 16) & 1u;
-      const uint32_t nrec = GUIDED ? (st.y >> kRecShift) & 3u : 0u;
-      if (GUIDED && nrec > 0u) pb.ended[atomicAdd(c + kCntEnded, 1u)] = make_uint2(st.w, nrec);
+      pb.ringL[ri] = f4(pt.L, 0.0f);
+      overflowed += (stFlags >> 16) & 1u;
+      const uint32_t nrec = GUIDED ? (stFlags >> kRecShift) & 3u : 0u;
+      if (GUIDED && nrec > 0u) pb.ended[atomicAdd(c + kCntEnded, 1u)] = make_uint2(pt.pid, nrec);
     }
-    if (vx.cast) {
-      pb.sh.q[idxS] = make_uint2(i, dest);
-      if (MULTI) pb.sh.job[i] = job;
-    }
+    if (vx.cast) pb.sh.q[idxS] = make_uint2(i, dest);
   }
   if (count) waveAddStat(&pb.stats[kStatMediaOverflow], overflowed);
+}
+
+// --------------------------------------------------------------- finish ----
+// Every path alive at bounce p to its end, one lane per path: the vertices,
+// shadow rays and extension rays of kShade and kTrace in the same order (so
+// the same bits), with the path in registers.  Few paths are alive, so a wave
+// takes as few of them as keeps every wave of the grid busy: its steps then
+// wait for the longest ray of 8 to 64 lanes instead of all the paths'.
+// Bound by the chain of one path's vertices (instruction and fetch latency).
+// One sample of a 1283x721 GGX grid: 12 further bounces of 290 us became one
+// launch of 0.9 ms, the render 4.07 -> 2.7 ms; 2^18 paths measured best of
+// 2^15 .. 2^19 (2.88, 2.79, 2.76, 2.68, 2.70 ms; caustic box at 720x405: 9.69,
+// 9.54, 9.30, 9.31, 9.66).
+constexpr uint32_t kFinishBlocks = 768;  // 3 waves per SIMD
+#ifndef HASTY_FINISH_PATHS
+#define HASTY_FINISH_PATHS (1u << 18)
+#endif
+constexpr uint32_t kFinishPaths = HASTY_FINISH_PATHS;
+template <bool MULTI, bool COUNT, int W>
+__global__ void __launch_bounds__(kBlock) HASTY_SHADE_ATTR kFinish(JobSet js, PathBuffers pb, PathSet ps, uint32_t p) {
+  __shared__ uint2 stack[kStackLds * kBlock];
+  const uint32_t* c = pb.counters + p * kCntSet;
+  if (!finishing(js, c)) return;
+  const uint32_t n = c[kCntLive];
+  const uint32_t lane = threadIdx.x & 63u, wave = (blockIdx.x * kBlock + threadIdx.x) >> 6;
+  const uint32_t waves = gridDim.x * (kBlock / 64);
+  uint32_t per = 64u;  // paths per wave
+  while (per > 8u && n <= waves * (per / 2u)) per /= 2u;
+  uint2* lds = stack + threadIdx.x;
+  uint2* ovf = pb.stackOverflow + (size_t)(blockIdx.x * kBlock + threadIdx.x) * kStackOvf;
+  uint32_t rays = 0, nodes = 0, tris = 0, shRays = 0, shNodes = 0, shTris = 0, overflowed = 0;
+  for (uint32_t g = wave; g * per < n; g += waves) {
+    const uint32_t i = g * per + lane;
+    if (lane >= per || i >= n) continue;
+    const uint4 st = ps.state[i];
+    const uint32_t job = jobOf<MULTI>(js, st);
+    Path pt = loadPath(ps, i, st);
+    float4 h4 = pb.hit[i];
+    Vertex vx;
+    do {
+      const uint32_t stFlags = pt.flags;
+      forJob<MULTI>(js, job, [&](const DevScene& s, const PassInfo& pi) {
+        shadeVertex<false>(s, pi, js.g, pb, i, pt, h4, vx);
+        if (vx.cast) {
+          const bool clear = findBlocker<kStackLds, kStackOvf, W>(s, prepareRay(vx.so, vx.sd), vx.st,
+                                                                  vx.target >= 0 ? vx.target : 0x7FFFFFFF, lds, kBlock,
+                                                                  ovf, &shNodes, &shTris) < 0;
+          if (clear) pt.L = pt.L + vx.c;
+          shRays++;
+        }
+        if (vx.go) {
+          const Hit h = traceClosest<kStackLds, kStackOvf, W>(s, pt.o, pt.d, lds, kBlock, ovf, &nodes, &tris);
+          h4 = make_float4(h.t, h.u, h.v, __int_as_float(h.tri));
+          rays++;
+        }
+      });
+      if (!vx.go) overflowed += (stFlags >> 16) & 1u;
+    } while (vx.go);
+    pb.ringL[pt.pid % pb.ringPaths] = f4(pt.L, 0.0f);
+  }
+  if (COUNT) {
+    waveAddStat(&pb.stats[kStatExtRays], rays);
+    waveAddStat(&pb.stats[kStatNodes], nodes);
+    waveAddStat(&pb.stats[kStatTris], tris);
+    waveAddStat(&pb.stats[kStatShadowRays], shRays);
+    waveAddStat(&pb.stats[kStatShadowNodes], shNodes);
+    waveAddStat(&pb.stats[kStatShadowTris], shTris);
+    waveAddStat(&pb.stats[kStatMediaOverflow], overflowed);
+  }
 }
 
 // -------------------------------------------------------------- connect ----
@@ -1091,18 +1189,31 @@ struct Bounces {
     if (GUIDED && js.g.sampleCap > 0u)
       timed(kKMisc, [&] { kHarvest<<<blocks(2048, pb.capacity), kBlock, 0, stream>>>(js.g, pb, p); });
   }
-  // `chunk` bounces (even, so every chunk issues identical launches, which is
-  // what a captured graph replays); without `fill` no path starts.
+  // The paths of bounce p to their ends, if they are the render's last and
+  // few (see finishing).
+  void finish(uint32_t p) const {
+    timed(kKFinish, [&] {
+      const uint32_t n = std::min(blocks(kFinishBlocks, 8ull * pb.capacity), pb.traceThreads / kBlock);
+      if (cfg.countStats) kFinish<MULTI, true, W><<<n, kBlock, 0, stream>>>(js, pb, pb.set[p], p);
+      else kFinish<MULTI, false, W><<<n, kBlock, 0, stream>>>(js, pb, pb.set[p], p);
+    });
+  }
+  // `n` bounces (even, so every chunk issues identical launches, which is what
+  // a captured graph replays).  With `fill` paths may start, and the last ones
+  // are left to a later chunk; without, kFinish takes them.
   void chunk(uint32_t n, bool fill) const {
+    JobSet shadeJobs = js;
+    if (fill) shadeJobs.finishPaths = 0u;  // the test kShade shares with kFinish
     for (uint32_t it = 0; it < n; ++it) {
       const uint32_t p = (it & 1u) ^ 1u;
+      if (shadeJobs.finishPaths > 0u) finish(p);
       if (GUIDED)
         timed(kKGuideInfer, [&] {
           kGuideInfer<<<kGuideInferBlocks, kGuideInferThreads, 0, stream>>>(js, pb, pb.set[p], p);
         });
       timed(kKShade, [&] {
         kShade<MULTI, GUIDED><<<blocks(cfg.shadeBlocks, pb.capacity), kBlock, 0, stream>>>(
-            js, pb, pb.set[p], pb.set[p ^ 1u], p, cfg.countStats ? 1u : 0u);
+            shadeJobs, pb, pb.set[p], pb.set[p ^ 1u], p, cfg.countStats ? 1u : 0u);
       });
       fillTrace(p, fill);
     }
@@ -1174,6 +1285,7 @@ void renderJobs(const std::vector<RenderJobDesc>& jobs, const PathBuffers& pb, c
     js.passes = (const PassInfo*)dPasses;
   }
   if (total == 0) return;
+  js.finishPaths = guide || late ? 0u : kFinishPaths;
   if (late && !pb.sh.lateQ) throw std::runtime_error("renderJobs: no buffers for late light samples");
   auto t0 = [&](int k) {
     if (timer) timer->begin(k, stream);
@@ -1218,19 +1330,24 @@ void renderJobs(const std::vector<RenderJobDesc>& jobs, const PathBuffers& pb, c
   std::vector<uint32_t> startedBy;
   uint64_t next = std::min<uint64_t>(limit, pb.capacity);  // paths started so far
   for (uint32_t c = 0;; ++c) {
+    // a small render is all last paths: no bounce kernels
+    const bool finishNow = !exec && total <= js.finishPaths && next >= total;
     if (exec) {
       t0(kKGraph);
       hipOk(hipGraphLaunch(exec, stream), "hipGraphLaunch");
       t1(kKGraph);
     } else {
-      bounces(timer, [&](const auto& b) { b.chunk(chunk, next < total); });
+      bounces(timer, [&](const auto& b) {
+        if (finishNow) b.finish(1u);
+        else b.chunk(chunk, next < total);
+      });
     }
     uint32_t cnt[kNumCounters];
     hipOk(hipMemcpyAsync(cnt, pb.counters, sizeof(cnt), hipMemcpyDeviceToHost, stream), "counter readback");
     hipOk(hipStreamSynchronize(stream), "hipStreamSynchronize");
     // the chunk's last bounce (p = 0) left the next one's counters in set 1
-    const uint32_t live = cnt[kCntSet + kCntLive];
     next = cnt[kCntSet + kCntNext];
+    const uint32_t live = finishNow ? 0u : cnt[kCntSet + kCntLive];
     startedBy.push_back((uint32_t)next);
     uint64_t done = live == 0 ? next : (c >= lag ? startedBy[c - lag] : 0u);
     for (uint32_t j = front; j < nJobs && passes[j].pidBase < done; ++j) {

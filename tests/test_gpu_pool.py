@@ -50,6 +50,20 @@ def test_batch_of_unlike_jobs(tmp_path, cornell_job, slots):
         _same(f.download(), ref)
 
 
+@pytest.mark.parametrize("which", ["cornell", "ggx_small", "caustic_small"])
+@pytest.mark.parametrize("size", [(5, 3), (97, 41), (701, 402)])
+def test_finished_paths_equal_bounce_by_bounce(which, size, request):
+    """The last 2^18 paths of a render run to their ends one by one; a render
+    by captured graphs runs every bounce of every path through the bounce
+    kernels.  15 paths, a partial grid, and more than 2^18."""
+    sc = ha.Scene(request.getfixturevalue(which + "_job"))
+    sc.set_settings(width=size[0], height=size[1])
+    sc.set_launch_ex(use_graph=1)
+    ref = _render(sc, 9, 0, 1)
+    sc.set_launch_ex(use_graph=0)
+    _same(ref, _render(sc, 9, 0, 1))
+
+
 def test_render_longer_than_the_ring(cornell_job):
     """36 samples of a 2048 x 2048 film are more than the ring's 2^27 paths."""
     sc = ha.Scene(cornell_job)
