@@ -153,10 +153,11 @@ struct Builder {
   }
 };
 
-void padBox(const Box& b, float* lo, float* hi) {
+// scene[c]: the largest coordinate magnitude along axis c.
+void padBox(const Box& b, const float* scene, float* lo, float* hi) {
   for (int c = 0; c < 3; ++c) {
     float m = std::max(std::fabs(b.lo[c]), std::fabs(b.hi[c]));
-    float pad = m * 0x1p-18f + 1e-30f;
+    float pad = m * 0x1p-18f + scene[c] * 0x1p-19f + 1e-30f;
     lo[c] = b.lo[c] - pad;
     hi[c] = b.hi[c] + pad;
   }
@@ -176,11 +177,15 @@ Bvh4 buildBvh4(const float* triPos, uint32_t numTris, const BvhBuildOptions& opt
   B.triBox.resize(numTris);
   B.cen.resize((size_t)numTris * 3);
   B.order.resize(numTris);
+  float scene[3] = {0.0f, 0.0f, 0.0f};
   for (uint32_t t = 0; t < numTris; ++t) {
     Box b;
     for (int v = 0; v < 3; ++v) b.growPoint(triPos + (size_t)t * 9 + v * 3);
     B.triBox[t] = b;
-    for (int c = 0; c < 3; ++c) B.cen[(size_t)t * 3 + c] = 0.5f * (b.lo[c] + b.hi[c]);
+    for (int c = 0; c < 3; ++c) {
+      B.cen[(size_t)t * 3 + c] = 0.5f * (b.lo[c] + b.hi[c]);
+      scene[c] = std::max(scene[c], std::max(std::fabs(b.lo[c]), std::fabs(b.hi[c])));
+    }
     B.order[t] = t;
   }
   B.nodes.reserve(numTris > 0 ? 2 * (size_t)numTris : 1);
@@ -257,7 +262,7 @@ Bvh4 buildBvh4(const float* triPos, uint32_t numTris, const BvhBuildOptions& opt
       }
       const BNode& kn = bn[kids[k]];
       float lo[3], hi[3];
-      padBox(kn.box, lo, hi);
+      padBox(kn.box, scene, lo, hi);
       uint32_t ref;
       if (kn.count > 0) {
         uint32_t firstOut = (uint32_t)leafTris.size();

@@ -17,8 +17,9 @@
 // Triangle record (3 x 16 bytes): v0.xyz + global triangle index (bits),
 // v1.xyz + 0, v2.xyz + 0.
 //
-// Boxes are widened by 2^-18 of their magnitude so that conservative slab
-// tests never drop a triangle the watertight test would report.
+// Boxes are widened by 2^-18 of their magnitude plus 2^-19 of the scene's along
+// each axis, so that the traversal's slab tests (with their rounding, see
+// testHalf) never drop a triangle the watertight test would report.
 #pragma once
 #include <stdint.h>
 

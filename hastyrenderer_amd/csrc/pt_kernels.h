@@ -131,11 +131,14 @@ struct JobSet {
 };
 
 // Traversal stack entries kept in LDS per lane (the rest spill to a global
-// slice); a build knob because it trades LDS (occupancy) for spills.
+// slice); a build knob because it trades LDS for spills.  With the row for
+// writes past it, 9 is what 8 blocks of 256 lanes fit in a CU's 160 KB (7, 8,
+// 9 entries: 117.2, 116.0, 115.3 ms on the GGX grid).
 #ifndef HASTY_STACK_LDS
-#define HASTY_STACK_LDS 8
+#define HASTY_STACK_LDS 9
 #endif
 constexpr int kStackLds = HASTY_STACK_LDS;
+constexpr int kStackRows = kStackLds + 1;   // LDS rows (the last for writes past the LDS part)
 constexpr int kStackOvf = 80 - kStackLds;  // 80 entries per lane in all
 constexpr int kBlock = 256;
 

@@ -297,7 +297,7 @@ __global__ void __launch_bounds__(kBlock) kFill(JobSet js, PathBuffers pb, PathS
 // W: node width of the single job's scene (4 or 8), 0 = each job's own.
 template <bool MULTI, bool COUNT, int W, bool LATE>
 __global__ void __launch_bounds__(kBlock) HASTY_TRACE_ATTR kTrace(JobSet js, PathBuffers pb, PathSet ps, uint32_t p) {
-  __shared__ uint2 stack[kStackLds * kBlock];
+  __shared__ uint2 stack[kStackRows * kBlock];
   const uint32_t gtid = xcdBlock() * blockDim.x + threadIdx.x;
   const uint32_t stride = gridDim.x * blockDim.x;
   uint2* lds = stack + threadIdx.x;
@@ -771,7 +771,7 @@ constexpr uint32_t kFinishBlocks = 768;  // 3 waves per SIMD
 constexpr uint32_t kFinishPaths = HASTY_FINISH_PATHS;
 template <bool MULTI, bool COUNT, int W>
 __global__ void __launch_bounds__(kBlock) HASTY_SHADE_ATTR kFinish(JobSet js, PathBuffers pb, PathSet ps, uint32_t p) {
-  __shared__ uint2 stack[kStackLds * kBlock];
+  __shared__ uint2 stack[kStackRows * kBlock];
   const uint32_t* c = pb.counters + p * kCntSet;
   if (!finishing(js, c)) return;
   const uint32_t n = c[kCntLive];
@@ -981,7 +981,7 @@ template <int W>
 __global__ void __launch_bounds__(kBlock) HASTY_TRACE_ATTR kTraceRays(DevScene s, const float* rays, uint32_t n,
                                                                      int32_t* tri, float* tuv, uint2* overflow,
                                                                      uint32_t slice) {
-  __shared__ uint2 stack[kStackLds * kBlock];
+  __shared__ uint2 stack[kStackRows * kBlock];
   uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
   uint32_t stride = gridDim.x * blockDim.x;
   uint2* ovf = overflow + (size_t)gtid * slice;
@@ -1001,7 +1001,7 @@ template <int W>
 __global__ void __launch_bounds__(kBlock) HASTY_TRACE_ATTR kTraceHits(DevScene s, const float* rays, uint32_t n,
                                                                      HitRecord* hits, uint2* overflow,
                                                                      uint32_t slice) {
-  __shared__ uint2 stack[kStackLds * kBlock];
+  __shared__ uint2 stack[kStackRows * kBlock];
   uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
   uint32_t stride = gridDim.x * blockDim.x;
   uint2* ovf = overflow + (size_t)gtid * slice;
@@ -1050,7 +1050,7 @@ __global__ void __launch_bounds__(kBlock) HASTY_TRACE_ATTR kTraceHits(DevScene s
 // (seed, t, p) of its own domain.
 __global__ void __launch_bounds__(kBlock) kGuidePhotons(DevScene s, uint32_t pass, uint32_t count, uint2* overflow,
                                                        float4* samples, uint32_t* sampleCount, uint32_t cap) {
-  __shared__ uint2 stack[kStackLds * kBlock];
+  __shared__ uint2 stack[kStackRows * kBlock];
   const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
   uint2* ovf = overflow + (size_t)gtid * kStackOvf;
   const float minQ = 1.0f - hm::powf_pos(0.1f, 1.0f / (float)s.maxDepth);
@@ -1220,12 +1220,16 @@ struct Bounces {
   }
 };
 
-// f(bounces) with the kernels of a batch (each job's node width read by the
-// kernels) or of one job (its width compiled in).
+// f(bounces) with the kernels of a batch or of one job, the jobs' node width
+// compiled in (0: a batch of both, each job's width read by the kernels; two
+// traversals in one kernel spill at 8 waves per SIMD, 12.4 against 9.0 ms on
+// the cuboid batch).
 template <class F>
 void withBounces(const JobSet& js, const PathBuffers& pb, const LaunchConfig& cfg, hipStream_t stream,
-                 KernelTimer* timer, bool late, bool guided, F&& f) {
-  if (js.nJobs > 1) f(Bounces<true, false, 0>{js, pb, cfg, stream, timer, late});
+                 KernelTimer* timer, bool late, bool guided, int width, F&& f) {
+  if (js.nJobs > 1 && width == 4) f(Bounces<true, false, 4>{js, pb, cfg, stream, timer, late});
+  else if (js.nJobs > 1 && width == 8) f(Bounces<true, false, 8>{js, pb, cfg, stream, timer, late});
+  else if (js.nJobs > 1) f(Bounces<true, false, 0>{js, pb, cfg, stream, timer, late});
   else if (guided && js.s.bvhWidth == 8) f(Bounces<false, true, 8>{js, pb, cfg, stream, timer, late});
   else if (guided) f(Bounces<false, true, 4>{js, pb, cfg, stream, timer, late});
   else if (js.s.bvhWidth == 8) f(Bounces<false, false, 8>{js, pb, cfg, stream, timer, late});
@@ -1248,6 +1252,7 @@ void renderJobs(const std::vector<RenderJobDesc>& jobs, const PathBuffers& pb, c
   uint64_t total = 0;
   int maxDepth = 1;
   bool late = false;
+  int width = 0;  // the jobs' node width, 0 if they differ
   for (uint32_t j = 0; j < nJobs; ++j) {
     const RenderJobDesc& d = jobs[j];
     scenes[j] = d.scene;
@@ -1263,6 +1268,7 @@ void renderJobs(const std::vector<RenderJobDesc>& jobs, const PathBuffers& pb, c
     total += (uint64_t)d.n * pi.pixels;
     maxDepth = std::max(maxDepth, d.scene.maxDepth);
     late = late || (d.scene.hasEnv && d.scene.hasSurfaceLight);
+    width = j == 0 || width == d.scene.bvhWidth ? d.scene.bvhWidth : 0;
   }
   if (total >= (1ull << 31)) throw std::runtime_error("renderJobs: more than 2^31 paths in one call");
   JobSet js{};
@@ -1306,7 +1312,7 @@ void renderJobs(const std::vector<RenderJobDesc>& jobs, const PathBuffers& pb, c
   t0(kKMisc);
   kInitRender<<<1, 64, 0, stream>>>(pb.counters, limit);
   t1(kKMisc);
-  auto bounces = [&](KernelTimer* t, auto&& f) { withBounces(js, pb, cfg, stream, t, late, guide != nullptr, f); };
+  auto bounces = [&](KernelTimer* t, auto&& f) { withBounces(js, pb, cfg, stream, t, late, guide != nullptr, width, f); };
   bounces(timer, [&](const auto& b) { b.fillTrace(0u, true); });
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;

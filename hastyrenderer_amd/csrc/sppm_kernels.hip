@@ -214,7 +214,7 @@ __global__ void __launch_bounds__(kB) kCellFold(const float* partial, int nBlock
 // PhotonMapping.cpp:578-651 (ignoreCosineTerm) times the footprint scale;
 // -1 marks pixels without a usable surface (filled on the host).
 __global__ void __launch_bounds__(kB) kInitRadii(DevScene s, float footprintScale, float* radii, uint2* ovfAll) {
-  __shared__ uint2 stack[kStackLds * kB];
+  __shared__ uint2 stack[kStackRows * kB];
   uint32_t P = s.width * s.height;
   uint32_t gtid = xcdRemap() * kB + threadIdx.x;
   uint2* ovf = ovfAll + (size_t)gtid * kStackOvf;
@@ -285,7 +285,7 @@ __global__ void __launch_bounds__(kB) kInitRadii(DevScene s, float footprintScal
 __global__ void __launch_bounds__(kB) kTracePhotons(DevScene s, SppmDev g, uint32_t first, uint32_t batch,
                                                     uint32_t emitLimit, uint32_t pass, uint32_t cap, float4* slX,
                                                     float4* slWi, float4* slF, uint32_t* slCount) {
-  __shared__ uint2 stack[kStackLds * kB];
+  __shared__ uint2 stack[kStackRows * kB];
   uint32_t gtid = xcdRemap() * kB + threadIdx.x;
   uint2* ovf = g.ovf + (size_t)gtid * kStackOvf;
   const float minQ = 1.0f - hm::powf_pos(0.1f, 1.0f / (float)s.maxDepth);
@@ -868,7 +868,7 @@ __device__ inline V3 gatherQuery(const SppmDev& g, const DevScene& s, bool has, 
 __global__ void __launch_bounds__(kB) HASTY_SPPM_CAMERA_ATTR kSppmCamera(DevScene s, SppmDev g, uint32_t pass, float offX, float offY,
                                                   float alpha, int emittedInt, float* color, float* normalOut,
                                                   float* albedoOut) {
-  __shared__ uint2 stack[kStackLds * kB];
+  __shared__ uint2 stack[kStackRows * kB];
   uint32_t P = s.width * s.height;
   uint32_t gtid = xcdRemap() * kB + threadIdx.x;
   uint2* ovf = g.ovf + (size_t)gtid * kStackOvf;
