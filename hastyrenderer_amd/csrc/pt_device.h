@@ -298,8 +298,8 @@ __device__ inline void cswap(float& ta, uint32_t& ra, float& tb, uint32_t& rb) {
 // global overflow slice.  Children are ordered near-to-far with a sorting
 // network held in registers.
 //
-// The walk is a state (Walk) advanced one step at a time (walkStep: one
-// inner node, or one leaf and the pop after it).  Written this way the
+// The walk is a state (Walk) advanced one step at a time (walkStep: one inner
+// node or one leaf triangle, and the pop after it).  Written this way the
 // compiled loop is shorter than the single-loop form with its break flag
 // (closest-hit launches -5.6 %, occlusion -8 % on the GGX grid).
 struct Walk {
@@ -374,7 +374,44 @@ __device__ inline bool walkStep(const DevScene& s, Walk& w, uint2* ldsGeneric, i
   typedef __attribute__((address_space(3))) unsigned long long LdsEntry;
   LdsEntry* lds = (LdsEntry*)ldsGeneric;
   const RayPre& r = w.r;
-  if ((w.ref & kLeafFlag) == 0) {
+  // Either the lanes at inner nodes or those at leaf triangles take their
+  // step, whichever are more (a choice uniform over the wave); the others
+  // wait, and a leaf's triangles are a step each.  Both codes used to run in
+  // nearly every iteration, the leaf's for a few lanes and as often as the
+  // largest leaf had triangles: 116 -> 109.6 ms on the GGX grid, 9.0 -> 8.1 ms
+  // on the cuboid batch, 1.00 -> 0.88 ms for incoherent queries.  Counting a
+  // lane at a leaf twice or three times: 108.5 and 109.3, 8.2 and 8.3, 0.89 and
+  // 0.91 ms.
+  const bool leaf = (w.ref & kLeafFlag) != 0u;
+  const int leaves = __popcll(__ballot(leaf)), walking = __popcll(__ballot(true));
+  bool pop = false;
+  if (2 * leaves > walking) {
+    if (leaf) {
+      const float4* tr = s.tris + (size_t)(w.ref & 0x00FFFFFFu) * 3;
+      const float4 p0 = ldg4(tr), p1 = ldg4(tr + 1), p2 = ldg4(tr + 2);
+      const int32_t id = (int32_t)__float_as_uint(p0.w);
+      w.nTris++;
+      w.ref += 1u - (1u << 24);  // the leaf's remaining triangles
+      pop = (w.ref & 0x7F000000u) == 0u;
+      float t, u, v;
+      if (intersectTri(r, p0, p1, p2, 1e-6f, &t, &u, &v)) {
+        if (CLOSEST) {
+          if (w.best.tri < 0 || t < w.best.t || (t == w.best.t && id < w.best.tri)) {
+            w.best.t = t;
+            w.best.u = u;
+            w.best.v = v;
+            w.best.tri = id;
+          }
+        } else if (t < w.tBound || (t == w.tBound && id < w.idBound)) {
+          w.best.t = t;
+          w.best.u = u;
+          w.best.v = v;
+          w.best.tri = id;
+          return true;
+        }
+      }
+    }
+  } else if (!leaf) {
     w.nNodes++;
     const float tb = w.best.t * kCullSlack;
     float e[W];
@@ -418,35 +455,11 @@ __device__ inline bool walkStep(const DevScene& s, Walk& w, uint2* ldsGeneric, i
       }
       w.sp = sp;
       w.ref = c[0];
-      return false;
-    }
-  } else if (w.ref != kLeafFlag) {
-    uint32_t count = (w.ref >> 24) & 0x7Fu;
-    uint32_t first = w.ref & 0x00FFFFFFu;
-    for (uint32_t k = 0; k < count; ++k) {
-      const float4* tr = s.tris + (size_t)(first + k) * 3;
-      float4 p0 = ldg4(tr), p1 = ldg4(tr + 1), p2 = ldg4(tr + 2);
-      int32_t id = (int32_t)__float_as_uint(p0.w);
-      w.nTris++;
-      float t, u, v;
-      if (intersectTri(r, p0, p1, p2, 1e-6f, &t, &u, &v)) {
-        if (CLOSEST) {
-          if (w.best.tri < 0 || t < w.best.t || (t == w.best.t && id < w.best.tri)) {
-            w.best.t = t;
-            w.best.u = u;
-            w.best.v = v;
-            w.best.tri = id;
-          }
-        } else if (t < w.tBound || (t == w.tBound && id < w.idBound)) {
-          w.best.t = t;
-          w.best.u = u;
-          w.best.v = v;
-          w.best.tri = id;
-          return true;
-        }
-      }
+    } else {
+      pop = true;
     }
   }
+  if (!pop) return false;
   // pop the nearest remaining entry that can still hold a closer hit
   const float lim = w.best.t * kCullSlack;
   while (w.sp > 0) {
