@@ -165,6 +165,56 @@ void padBox(const Box& b, const float* scene, float* lo, float* hi) {
 
 }  // namespace
 
+std::vector<float> coverBoxes(const float* triPos, uint32_t numTris, const std::vector<uint32_t>& tris, int maxBoxes) {
+  float scene[3] = {0.0f, 0.0f, 0.0f};
+  for (size_t i = 0; i < (size_t)numTris * 9; ++i) scene[i % 3] = std::max(scene[i % 3], std::fabs(triPos[i]));
+  struct Group {
+    Box box;
+    size_t first, last;
+    bool whole;  // not splittable
+  };
+  std::vector<uint32_t> order = tris;
+  auto group = [&](size_t first, size_t last) {
+    Group g{Box(), first, last, last - first < 2};
+    for (size_t i = first; i < last; ++i)
+      for (int v = 0; v < 3; ++v) g.box.growPoint(triPos + (size_t)order[i] * 9 + v * 3);
+    return g;
+  };
+  std::vector<Group> groups;
+  if (!order.empty()) groups.push_back(group(0, order.size()));
+  // split the largest box at the middle of its longest axis until there are enough
+  while (!groups.empty() && (int)groups.size() < maxBoxes) {
+    size_t best = groups.size();
+    for (size_t i = 0; i < groups.size(); ++i)
+      if (!groups[i].whole && (best == groups.size() || groups[i].box.area() > groups[best].box.area())) best = i;
+    if (best == groups.size()) break;
+    Group& g = groups[best];
+    int axis = 0;
+    for (int c = 1; c < 3; ++c)
+      if (g.box.hi[c] - g.box.lo[c] > g.box.hi[axis] - g.box.lo[axis]) axis = c;
+    const float mid = 0.5f * (g.box.lo[axis] + g.box.hi[axis]);
+    auto it = std::partition(order.begin() + g.first, order.begin() + g.last, [&](uint32_t t) {
+      const float* p = triPos + (size_t)t * 9 + axis;
+      return (p[0] + p[3] + p[6]) * (1.0f / 3.0f) < mid;
+    });
+    const size_t cut = (size_t)(it - order.begin());
+    if (cut == g.first || cut == g.last) {
+      g.whole = true;
+      continue;
+    }
+    const size_t last = g.last;
+    groups[best] = group(g.first, cut);
+    groups.push_back(group(cut, last));
+  }
+  std::vector<float> out;
+  for (const Group& g : groups) {
+    float lo[3], hi[3];
+    padBox(g.box, scene, lo, hi);
+    out.insert(out.end(), {lo[0], lo[1], lo[2], 0.0f, hi[0], hi[1], hi[2], 0.0f});
+  }
+  return out;
+}
+
 Bvh4 buildBvh4(const float* triPos, uint32_t numTris, const BvhBuildOptions& opt, int width) {
   if (width != 4 && width != 8) throw std::runtime_error("BVH width must be 4 or 8");
   Bvh4 out;

@@ -48,6 +48,11 @@ struct Bvh4 {
 // triPos: 9 floats per triangle (global order); width 4 or 8.
 Bvh4 buildBvh4(const float* triPos, uint32_t numTris, const BvhBuildOptions& opt, int width = 4);
 
+// At most maxBoxes boxes (lo.xyz 0 hi.xyz 0 each) that together cover the
+// given triangles, widened as the BVH's boxes; few triangles wide where the
+// triangles allow it.
+std::vector<float> coverBoxes(const float* triPos, uint32_t numTris, const std::vector<uint32_t>& tris, int maxBoxes);
+
 constexpr uint32_t kLeafFlag = 0x80000000u;
 inline uint32_t makeLeafRef(uint32_t first, uint32_t count) { return kLeafFlag | (count << 24) | first; }
 

@@ -1652,7 +1652,17 @@ int hasty_sppm_create(HastyScene* s, uint32_t seed, const HastySppmParams* param
     d.seed = seed;
     auto h = std::make_unique<HastySppm>();
     h->scene = s;
-    h->r = std::make_unique<hasty::SppmRenderer>(d, p, s->stream);
+    // surfaces that bounce photons: a concentrated lobe is reflection
+    // (specular or metallic) or transmission (computeProbability)
+    const hasty::Scene& sc = s->job.scene;
+    std::vector<uint32_t> casters;
+    for (uint32_t t = 0; t < sc.numTris; ++t) {
+      const int32_t k = sc.triMaterial[t];
+      const hasty::Material& m = sc.materials[k];
+      if (m.specular != 0.0f || m.metallic != 0.0f || m.transmission != 0.0f) casters.push_back(t);
+    }
+    h->r = std::make_unique<hasty::SppmRenderer>(
+        d, p, hasty::coverBoxes(sc.triPos.data(), sc.numTris, casters, hasty::kSppmCasterBoxes), s->stream);
     *out = h.release();
     return 0;
   } catch (const std::exception& e) {

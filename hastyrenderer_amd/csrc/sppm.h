@@ -23,6 +23,8 @@ struct SppmParams {
   float gatherUnionFactor = 0.0f;      // > 0: union gathers (see kSppmGather); 0: off
 };
 
+constexpr int kSppmCasterBoxes = 32;  // boxes around the surfaces that bounce photons
+
 struct SppmPassInfo {
   uint64_t emitted = 0, stored = 0;
   float cellSize = 0.0f;
@@ -34,7 +36,10 @@ struct SppmPassInfo {
 // (PMRenderJobPixel), the radius image and the per-pass photon map.
 class SppmRenderer {
  public:
-  SppmRenderer(const hdev::DevScene& scene, const SppmParams& params, hipStream_t stream);
+  // casters: boxes (lo.xyz 0 hi.xyz 0 each) that cover every surface with a
+  // concentrated lobe, widened as the BVH's boxes (coverBoxes).
+  SppmRenderer(const hdev::DevScene& scene, const SppmParams& params, const std::vector<float>& casters,
+               hipStream_t stream);
   ~SppmRenderer();
   SppmRenderer(const SppmRenderer&) = delete;
   SppmRenderer& operator=(const SppmRenderer&) = delete;
@@ -85,13 +90,19 @@ class SppmRenderer {
   uint32_t* dCounters_ = nullptr;
   unsigned long long* dGatherStats_ = nullptr;
   uint2* dOverflow_ = nullptr;
-  // photon batches: per-thread slots, batch x cap
-  uint32_t cap_ = 0, batchMax_ = 0;
+  // photon batches: photons emitted per batch at most; slots of those traced
+  // (slots x cap)
+  uint32_t cap_ = 0, batchMax_ = 0, slots_ = 0;
   float4* dSlX_ = nullptr;
   float4* dSlWi_ = nullptr;
   float4* dSlF_ = nullptr;
   uint32_t* dSlCount_ = nullptr;
   uint32_t* dSlOffset_ = nullptr;
+  uint32_t* dSlList_ = nullptr;  // photons of the batch worth tracing
+  float4* dBoxes_ = nullptr;
+  uint32_t nBoxes_ = 0;
+  // shares of the emitted photons that are traced and stored, as last seen
+  double selectRate_ = 0.5, storeRate_ = 0.0;
   void* dScanTmp_ = nullptr;
   size_t scanTmpBytes_ = 0;
   // photons of the pass in emission order and in cell order
