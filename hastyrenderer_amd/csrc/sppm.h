@@ -80,6 +80,7 @@ class SppmRenderer {
   // bytes), queries per pixel, path radiance (3 planes)
   float4* dQuery_ = nullptr;
   uint32_t* dNq_ = nullptr;
+  uint32_t* dTasks_ = nullptr;  // gather tasks of many candidates
   float* dLpath_ = nullptr;
   // cell size reductions
   float* dPartial_ = nullptr;
@@ -121,8 +122,7 @@ class SppmRenderer {
   size_t sortTmpBytes_ = 0;
   // cell table
   uint32_t tableSize_ = 0;
-  unsigned long long* dTableKeys_ = nullptr;
-  uint2* dTableVals_ = nullptr;
+  uint4* dTable_ = nullptr;
 };
 
 }  // namespace hasty

@@ -87,9 +87,8 @@ struct SppmDev {
   float4* sF;
   unsigned long long* keys;
   uint32_t* idx;
-  // cell table
-  unsigned long long* tKeys;
-  uint2* tVals;
+  // cell table: (key, first photon, count) in 16 bytes, so a probe is one load
+  uint4* table;
   uint32_t tMask;
   int* bbox;  // min xyz, max xyz of occupied cells
   const float* cellSize;
@@ -121,6 +120,7 @@ enum Counter {
   kCtrFluxOverflow = 4,  // gathers whose fixed-point flux sum saturated
   kCtrSelected = 5,      // photons of the batch that meet a caster's box
   kCtrTraced = 6,        // the last batch's
+  kCtrShared = 7,        // gather tasks left to kSppmGatherShared
   kNumCtr = 8
 };
 
@@ -505,8 +505,12 @@ __global__ void __launch_bounds__(kB) kCellKeys(SppmDev g, uint32_t n) {
   else if (threadIdx.x < 6) atomicMax(&g.bbox[threadIdx.x], box[threadIdx.x]);
 }
 __global__ void __launch_bounds__(kB) kCellInit(SppmDev g, int clearBox) {
-  for (uint32_t k = blockIdx.x * kB + threadIdx.x; k <= g.tMask; k += gridDim.x * kB) g.tKeys[k] = kEmptyKey;
+  for (uint32_t k = blockIdx.x * kB + threadIdx.x; k <= g.tMask; k += gridDim.x * kB)
+    g.table[k] = make_uint4(~0u, ~0u, 0u, 0u);  // kEmptyKey
   if (clearBox && blockIdx.x == 0 && threadIdx.x < 6) g.bbox[threadIdx.x] = threadIdx.x < 3 ? 0x7FFFFFFF : -0x7FFFFFFF;
+}
+__device__ inline unsigned long long tableKey(uint4 e) {
+  return (unsigned long long)e.x | ((unsigned long long)e.y << 32);
 }
 // Gather the photon records into cell order and insert each cell's first
 // photon into the table; kCellCount then closes each cell at its last photon.
@@ -521,11 +525,11 @@ __global__ void __launch_bounds__(kB) kCellBuild(SppmDev g, const unsigned long 
     if (k == 0 || keysSorted[k - 1] != key) {
       uint32_t h = hashKey(key) & g.tMask;
       while (true) {
-        unsigned long long prev = atomicCAS(&g.tKeys[h], kEmptyKey, key);
+        unsigned long long prev = atomicCAS((unsigned long long*)&g.table[h], kEmptyKey, key);
         if (prev == kEmptyKey) break;
         h = (h + 1) & g.tMask;
       }
-      g.tVals[h] = make_uint2(k, 0u);
+      g.table[h].z = k;
     }
   }
 }
@@ -534,20 +538,25 @@ __global__ void __launch_bounds__(kB) kCellCount(SppmDev g, const unsigned long 
     unsigned long long key = keysSorted[k];
     if (k + 1 == n || keysSorted[k + 1] != key) {
       uint32_t h = hashKey(key) & g.tMask;
-      while (g.tKeys[h] != key) h = (h + 1) & g.tMask;
-      g.tVals[h].y = k + 1 - g.tVals[h].x;
+      while (tableKey(g.table[h]) != key) h = (h + 1) & g.tMask;
+      g.table[h].w = k + 1 - g.table[h].z;
     }
   }
 }
 
-__device__ inline uint2 cellLookup(const SppmDev& g, unsigned long long key) {
-  uint32_t h = hashKey(key) & g.tMask;
+// The photons of a cell (first, count), from its first probe `e` at slot h.
+__device__ inline uint2 cellResolve(const SppmDev& g, unsigned long long key, uint32_t h, uint4 e) {
   while (true) {
-    unsigned long long k = g.tKeys[h];
-    if (k == key) return g.tVals[h];
+    const unsigned long long k = tableKey(e);
+    if (k == key) return make_uint2(e.z, e.w);
     if (k == kEmptyKey) return make_uint2(0u, 0u);
     h = (h + 1) & g.tMask;
+    e = g.table[h];
   }
+}
+__device__ inline uint2 cellLookup(const SppmDev& g, unsigned long long key) {
+  const uint32_t h = hashKey(key) & g.tMask;
+  return cellResolve(g, key, h, g.table[h]);
 }
 
 // photonMapFluxEstimate (PhotonMapping.cpp:271-296) with
@@ -555,17 +564,13 @@ __device__ inline uint2 cellLookup(const SppmDev& g, unsigned long long key) {
 // photons of a cell in emission order, |x - c|^2 <= r^2; the BSDF is the
 // diffuse lobe only with outside IOR 1.
 //
-// When some lane of the wave has many candidate photons (dense maps, large
-// radii), the 64 lanes of the wave serve its queries one owner at a time,
-// every lane testing a share of the owner's photons (rank k of 64 takes
-// photons k, k + 64, ... of each cell, so a cell's run is read in whole
-// cache lines), and the lanes' partial sums are added by a butterfly over
-// the wave.  The set and the count of photons are the reference's; only the
-// FP32 association of the flux sum differs, the same way on every run.
-// Otherwise each lane sums its own photons in the reference's order.  In the
-// shared gather the owner's cell lookups are spread over the lanes (one hash
-// probe each, all in flight together) and the cells' photon runs read back
-// from LDS in cell order; `runs` is this wave's 64-entry LDS scratch.
+// When some query of 64 consecutive pixels has many candidate photons (dense
+// maps, large radii), those queries are gathered one at a time by the 64
+// lanes of a wave (sharedGather), every lane testing a share of the query's
+// photons, and the lanes' partial sums are added by a butterfly over the wave.
+// The set and the count of photons are the reference's; only the FP32
+// association of the flux sum differs, the same way on every run.  Otherwise
+// each lane sums its own photons in the reference's order.
 // The sum of a gather's photon terms.  FloatSum: FP32 in the order the
 // terms arrive (the reference's, for a lane gathering alone).  FixedSum:
 // each term rounded to an integer number of 2^-S units (round to nearest
@@ -661,25 +666,33 @@ __device__ inline void photonTerm(const SppmDev& g, uint32_t q, float4 x4, V3 c,
 #define HASTY_PHOTON_LOADS 4
 #endif
 constexpr uint32_t kPhotonLoads = HASTY_PHOTON_LOADS;
-// Photons first, first + stride, ... below end, in that order, with
-// kPhotonLoads position loads in flight at a time.
+// Photons [first, end) in order, with kPhotonLoads position loads in flight at
+// a time, then the direction and flux loads of those within the radius.
 template <class Sum>
-__device__ inline void photonRun(const SppmDev& g, uint32_t first, uint32_t end, uint32_t stride, V3 c, float r2,
-                                 V3 ns, V3 ng, const DevMaterial& m, Sum* acc, int* found) {
-  uint32_t q = first;
-  for (; q + (kPhotonLoads - 1u) * stride < end; q += kPhotonLoads * stride) {
-    float4 x[kPhotonLoads];
+__device__ inline void photonRun(const SppmDev& g, uint32_t first, uint32_t end, V3 c, float r2, V3 ns, V3 ng,
+                                 const DevMaterial& m, Sum* acc, int* found) {
+  for (uint32_t q = first; q < end; q += kPhotonLoads) {
+    float4 x[kPhotonLoads], wi[kPhotonLoads], fl[kPhotonLoads];
+    bool in[kPhotonLoads];
 #pragma unroll
-    for (uint32_t u = 0; u < kPhotonLoads; ++u) x[u] = g.sX[q + u * stride];
+    for (uint32_t u = 0; u < kPhotonLoads; ++u) x[u] = g.sX[min(q + u, end - 1u)];
 #pragma unroll
-    for (uint32_t u = 0; u < kPhotonLoads; ++u) photonTerm(g, q + u * stride, x[u], c, r2, ns, ng, m, acc, found);
+    for (uint32_t u = 0; u < kPhotonLoads; ++u) {
+      const V3 dlt = f4xyz(x[u]) - c;
+      in[u] = q + u < end && dot(dlt, dlt) <= r2;
+      if (in[u]) wi[u] = g.sWi[q + u], fl[u] = g.sF[q + u];
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < kPhotonLoads; ++u)
+      if (in[u]) photonAdd(g, x[u], wi[u], fl[u], ns, ng, m, acc, found);
   }
-  for (; q < end; q += stride) photonTerm(g, q, g.sX[q], c, r2, ns, ng, m, acc, found);
 }
-// Lanes whose cells hold fewer candidates than g.coopCandidates (default
-// 512) gather on their own (a shared gather costs every lane each owner's
-// cell lookups).
-constexpr uint32_t kCoopCandidatesDefault = 512;
+// Queries with at most g.coopCandidates candidates (default 128) are gathered
+// by a lane each: a longer list is a chain of loads that the other lanes wait
+// for, while a shared gather costs a wave per query.  Passes of the caustic box
+// with 32, 64, 128, 256, 512: 4.94, 4.89, 4.83, 4.84, 4.81 ms (sparse map,
+// 960x540) and 9.68, 9.69, 9.69, 9.97, 10.99 ms (dense map, 640x360).
+constexpr uint32_t kCoopCandidatesDefault = 128;
 // Union gather: the wave visits the cells of the union of its queries'
 // boxes in x -> y -> z order, stages each run of photon positions in LDS 64
 // at a time, and every lane tests them against its own query.  A photon
@@ -755,170 +768,206 @@ __device__ inline void foundTerms(const SppmDev& g, const uint32_t* fq, uint32_t
   __builtin_amdgcn_wave_barrier();  // the slots are refilled afterwards
 }
 
+// Cells a query of radius r around x visits: its box within the occupied one.
+__device__ inline void queryCells(const SppmDev& g, V3 x, float r, float cs, int3* lo, int3* hi) {
+  const int3 l = cellOf(x - v3(r, r, r), cs), h = cellOf(x + v3(r, r, r), cs);
+  *lo = make_int3(max(l.x, g.bbox[0]), max(l.y, g.bbox[1]), max(l.z, g.bbox[2]));
+  *hi = make_int3(min(h.x, g.bbox[3]), min(h.y, g.bbox[4]), min(h.z, g.bbox[5]));
+}
+
+// Cell lookups of a lane's own gather in flight at a time, and the occupied
+// cells it keeps for the gather (more: they are looked up again).
+constexpr int kCellLoads = 4, kOwnRuns = 8;
+// The gathers of a wave's queries, a lane each in the reference's order (or
+// the union gather); false, with nothing gathered, if some query has so many
+// candidates that all of them are left to sharedGather.
 template <class Sum>
-__device__ inline V3 gatherQuery(const SppmDev& g, const DevScene& s, bool has, V3 x, V3 ns, V3 ng, int mat,
-                                 float r, int* M, uint2* runs, float4* staged, uint32_t* fq, uint32_t* candidates) {
+__device__ inline bool ownGather(const SppmDev& g, const DevScene& s, bool has, V3 x, V3 ns, V3 ng, int mat, float r,
+                                 int* M, uint2* runs, float4* staged, uint2* ownRuns, uint32_t* candidates,
+                                 V3* result) {
   const float cs = *g.cellSize;
-  {
-    // candidates of this lane's own query; if no lane of the wave has many,
-    // every lane gathers alone in the reference's order
-    uint32_t cand = 0;
-    int3 lo = make_int3(0, 0, 0), hi = make_int3(-1, -1, -1);
-    if (has) {
-      lo = cellOf(x - v3(r, r, r), cs), hi = cellOf(x + v3(r, r, r), cs);
-      lo = make_int3(max(lo.x, g.bbox[0]), max(lo.y, g.bbox[1]), max(lo.z, g.bbox[2]));
-      hi = make_int3(min(hi.x, g.bbox[3]), min(hi.y, g.bbox[4]), min(hi.z, g.bbox[5]));
-      for (int i = lo.x; i <= hi.x; ++i)
-        for (int j = lo.y; j <= hi.y; ++j)
-          for (int k = lo.z; k <= hi.z; ++k) cand += cellLookup(g, packKey(make_int3(i, j, k))).y;
+  uint32_t cand = 0;
+  int nRuns = 0;  // occupied cells; the first kOwnRuns are at ownRuns[k * kB]
+  int3 lo = make_int3(0, 0, 0), hi = make_int3(-1, -1, -1);
+  if (has) {
+    queryCells(g, x, r, cs, &lo, &hi);
+    int3 c = lo;
+    bool more = lo.x <= hi.x && lo.y <= hi.y && lo.z <= hi.z;
+    while (more) {
+      unsigned long long key[kCellLoads];
+      uint32_t h[kCellLoads];
+      uint4 e[kCellLoads];
+      int n = 0;
+#pragma unroll
+      for (int u = 0; u < kCellLoads; ++u) {
+        if (!more) continue;
+        key[u] = packKey(c);
+        h[u] = hashKey(key[u]) & g.tMask;
+        e[u] = g.table[h[u]];
+        n = u + 1;
+        if (++c.z > hi.z) {
+          c.z = lo.z;
+          if (++c.y > hi.y) {
+            c.y = lo.y;
+            more = ++c.x <= hi.x;
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kCellLoads; ++u) {
+        if (u >= n) continue;
+        const uint2 cell = cellResolve(g, key[u], h[u], e[u]);
+        if (cell.y == 0u) continue;
+        cand += cell.y;
+        if (nRuns < kOwnRuns) ownRuns[nRuns * kB] = cell;
+        nRuns++;
+      }
     }
-    *candidates = cand;
-    if (__ballot(cand > g.coopCandidates) == 0ull) {
-      Sum est;
-      int found = 0;
-      if (has) {
-        const DevMaterial m = ldgStruct(s.mats + mat);
+  }
+  *candidates = cand;
+  if (__ballot(cand > g.coopCandidates) == 0ull) {
+    Sum est;
+    int found = 0;
+    if (has) {
+      const DevMaterial m = ldgStruct(s.mats + mat);
+      if (nRuns <= kOwnRuns) {
+        for (int k = 0; k < nRuns; ++k) {
+          const uint2 cell = ownRuns[k * kB];
+          photonRun(g, cell.x, cell.x + cell.y, x, r * r, ns, ng, m, &est, &found);
+        }
+      } else {
         for (int i = lo.x; i <= hi.x; ++i)
           for (int j = lo.y; j <= hi.y; ++j)
             for (int k = lo.z; k <= hi.z; ++k) {
               const uint2 cell = cellLookup(g, packKey(make_int3(i, j, k)));
-              photonRun(g, cell.x, cell.x + cell.y, 1u, x, r * r, ns, ng, m, &est, &found);
+              photonRun(g, cell.x, cell.x + cell.y, x, r * r, ns, ng, m, &est, &found);
             }
-        if (est.saturated()) atomicAdd(&g.counters[kCtrFluxOverflow], 1u);
       }
-      *M = found;
-      return est.value(g);
+      if (est.saturated()) atomicAdd(&g.counters[kCtrFluxOverflow], 1u);
     }
-    // many candidates: the union gather when the queries' boxes overlap
-    // enough (the union box holds at most unionFactor x their mean cells)
-    if (g.unionFactor > 0.0f) {
-      int3 ulo = make_int3(has ? lo.x : 0x7FFFFFFF, has ? lo.y : 0x7FFFFFFF, has ? lo.z : 0x7FFFFFFF);
-      int3 uhi = make_int3(has ? hi.x : -0x7FFFFFFF, has ? hi.y : -0x7FFFFFFF, has ? hi.z : -0x7FFFFFFF);
-      float own = has ? (float)max(hi.x - lo.x + 1, 0) * (float)max(hi.y - lo.y + 1, 0) *
-                            (float)max(hi.z - lo.z + 1, 0)
-                      : 0.0f;
-      int nHas = has ? 1 : 0;
-      for (int off = 32; off > 0; off >>= 1) {
-        ulo.x = min(ulo.x, __shfl_xor(ulo.x, off));
-        ulo.y = min(ulo.y, __shfl_xor(ulo.y, off));
-        ulo.z = min(ulo.z, __shfl_xor(ulo.z, off));
-        uhi.x = max(uhi.x, __shfl_xor(uhi.x, off));
-        uhi.y = max(uhi.y, __shfl_xor(uhi.y, off));
-        uhi.z = max(uhi.z, __shfl_xor(uhi.z, off));
-        own += __shfl_xor(own, off);
-        nHas += __shfl_xor(nHas, off);
-      }
-      const float unionCells = nHas > 0 ? (float)(uhi.x - ulo.x + 1) * (float)(uhi.y - ulo.y + 1) *
-                                              (float)(uhi.z - ulo.z + 1)
-                                        : 0.0f;
-      const bool nonEmpty = uhi.x >= ulo.x && uhi.y >= ulo.y && uhi.z >= ulo.z;
-      if (nHas > 0 && nonEmpty && unionCells <= g.unionFactor * own / (float)nHas && unionCells < 1.0e6f)
-        return unionGather<Sum>(g, s, has, x, ns, ng, mat, r, lo, hi, ulo, uhi, M, runs, staged);
+    *M = found;
+    *result = est.value(g);
+    return true;
+  }
+  // many candidates: the union gather when the queries' boxes overlap
+  // enough (the union box holds at most unionFactor x their mean cells)
+  if (g.unionFactor > 0.0f) {
+    int3 ulo = make_int3(has ? lo.x : 0x7FFFFFFF, has ? lo.y : 0x7FFFFFFF, has ? lo.z : 0x7FFFFFFF);
+    int3 uhi = make_int3(has ? hi.x : -0x7FFFFFFF, has ? hi.y : -0x7FFFFFFF, has ? hi.z : -0x7FFFFFFF);
+    float own = has ? (float)max(hi.x - lo.x + 1, 0) * (float)max(hi.y - lo.y + 1, 0) *
+                          (float)max(hi.z - lo.z + 1, 0)
+                    : 0.0f;
+    int nHas = has ? 1 : 0;
+    for (int off = 32; off > 0; off >>= 1) {
+      ulo.x = min(ulo.x, __shfl_xor(ulo.x, off));
+      ulo.y = min(ulo.y, __shfl_xor(ulo.y, off));
+      ulo.z = min(ulo.z, __shfl_xor(ulo.z, off));
+      uhi.x = max(uhi.x, __shfl_xor(uhi.x, off));
+      uhi.y = max(uhi.y, __shfl_xor(uhi.y, off));
+      uhi.z = max(uhi.z, __shfl_xor(uhi.z, off));
+      own += __shfl_xor(own, off);
+      nHas += __shfl_xor(nHas, off);
+    }
+    const float unionCells = nHas > 0 ? (float)(uhi.x - ulo.x + 1) * (float)(uhi.y - ulo.y + 1) *
+                                            (float)(uhi.z - ulo.z + 1)
+                                      : 0.0f;
+    const bool nonEmpty = uhi.x >= ulo.x && uhi.y >= ulo.y && uhi.z >= ulo.z;
+    if (nHas > 0 && nonEmpty && unionCells <= g.unionFactor * own / (float)nHas && unionCells < 1.0e6f) {
+      *result = unionGather<Sum>(g, s, has, x, ns, ng, mat, r, lo, hi, ulo, uhi, M, runs, staged);
+      return true;
     }
   }
-  // shared gather, one owner query at a time: the 64 lanes test the owner's
-  // candidate photons, those within the radius are queued in LDS and their
-  // terms taken 64 at a time, and a butterfly adds the lanes' partial sums.
-  // Every lane of the wave takes part (the caller keeps the whole wave
-  // here), so a query's sums do not depend on which other queries share its
-  // wave.
+  return false;
+}
+
+// One query (the same on every lane), by the 64 lanes of the wave: they test
+// its candidate photons, those within the radius are queued in LDS and their
+// terms taken 64 at a time, and a butterfly adds the lanes' partial sums.
+// Every lane of the wave takes part and gets the result.
+template <class Sum>
+__device__ inline V3 sharedGather(const SppmDev& g, const DevScene& s, V3 c, V3 ns, V3 ng, int mat, float rr, int* M,
+                                  uint2* runs, uint32_t* fq, bool* saturated) {
   const uint32_t lane = __lane_id();
   const int rank = (int)lane, nAct = 64;
   const unsigned long long ltMask = (1ull << lane) - 1ull;
-  V3 myEst = v3(0.0f, 0.0f, 0.0f);
-  int myM = 0;
-  uint64_t todo = __ballot(has);
-  while (todo) {
-    const int owner = __ffsll((unsigned long long)todo) - 1;
-    todo &= todo - 1ull;
-    const V3 c = v3(__shfl(x.x, owner), __shfl(x.y, owner), __shfl(x.z, owner));
-    const V3 nso = v3(__shfl(ns.x, owner), __shfl(ns.y, owner), __shfl(ns.z, owner));
-    const V3 ngo = v3(__shfl(ng.x, owner), __shfl(ng.y, owner), __shfl(ng.z, owner));
-    const float rr = __shfl(r, owner);
-    const DevMaterial m = ldgStruct(s.mats + __shfl(mat, owner));
-    const float r2 = rr * rr;
-    int3 lo = cellOf(c - v3(rr, rr, rr), cs), hi = cellOf(c + v3(rr, rr, rr), cs);
-    lo = make_int3(max(lo.x, g.bbox[0]), max(lo.y, g.bbox[1]), max(lo.z, g.bbox[2]));
-    hi = make_int3(min(hi.x, g.bbox[3]), min(hi.y, g.bbox[4]), min(hi.z, g.bbox[5]));
-    Sum acc;
-    int found = 0;
-    uint32_t head = 0u, tail = 0u;  // the queue fq[head .. tail) (mod 128) of photons found
-    // the cells of the box in x -> y -> z order, 64 at a time: lane rank
-    // looks up cell base + rank (all probes in flight together).  Their
-    // photons are then dealt to the lanes as one sequence (cell after cell),
-    // so every lane has work whatever the cells' sizes.
-    const int ny = max(hi.y - lo.y + 1, 0), nz = max(hi.z - lo.z + 1, 0);
-    const int nyz = ny * nz, nc = max(hi.x - lo.x + 1, 0) * nyz;
-    for (int base = 0; base < nc; base += nAct) {
-      const int ci = base + rank;
-      uint2 run = make_uint2(0u, 0u);
-      if (ci < nc) {
-        const int ix = ci / nyz, rem = ci - ix * nyz, iy = rem / nz, iz = rem - iy * nz;
-        run = cellLookup(g, packKey(make_int3(lo.x + ix, lo.y + iy, lo.z + iz)));
-      }
-      // inclusive prefix of the photon counts over the 64 cells
-      uint32_t incl = run.y;
-      for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t t = __shfl_up(incl, off);
-        if (rank >= off) incl += t;
-      }
-      const uint32_t total = __shfl(incl, 63);
-      // sequence index i of this cell's photons maps to photon i + .x
-      // (unsigned arithmetic wraps); .y is where the cell ends
-      runs[rank] = make_uint2(run.x - (incl - run.y), incl);
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      int cur = 0;  // the lane's cell; its sequence indices only grow
-      // the trip count is the same on every lane: foundTerms needs the
-      // whole wave
-      for (uint32_t b0 = 0; b0 < total; b0 += kPhotonLoads * (uint32_t)nAct) {
-        uint32_t q[kPhotonLoads];
-        float4 xp[kPhotonLoads];
+  const DevMaterial m = ldgStruct(s.mats + mat);
+  const float r2 = rr * rr;
+  int3 lo, hi;
+  queryCells(g, c, rr, *g.cellSize, &lo, &hi);
+  Sum acc;
+  int found = 0;
+  uint32_t head = 0u, tail = 0u;  // the queue fq[head .. tail) (mod 128) of photons found
+  // the cells of the box in x -> y -> z order, 64 at a time: lane rank
+  // looks up cell base + rank (all probes in flight together).  Their
+  // photons are then dealt to the lanes as one sequence (cell after cell),
+  // so every lane has work whatever the cells' sizes.
+  const int ny = max(hi.y - lo.y + 1, 0), nz = max(hi.z - lo.z + 1, 0);
+  const int nyz = ny * nz, nc = max(hi.x - lo.x + 1, 0) * nyz;
+  for (int base = 0; base < nc; base += nAct) {
+    const int ci = base + rank;
+    uint2 run = make_uint2(0u, 0u);
+    if (ci < nc) {
+      const int ix = ci / nyz, rem = ci - ix * nyz, iy = rem / nz, iz = rem - iy * nz;
+      run = cellLookup(g, packKey(make_int3(lo.x + ix, lo.y + iy, lo.z + iz)));
+    }
+    // inclusive prefix of the photon counts over the 64 cells
+    uint32_t incl = run.y;
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t t = __shfl_up(incl, off);
+      if (rank >= off) incl += t;
+    }
+    const uint32_t total = __shfl(incl, 63);
+    // sequence index i of this cell's photons maps to photon i + .x
+    // (unsigned arithmetic wraps); .y is where the cell ends
+    runs[rank] = make_uint2(run.x - (incl - run.y), incl);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    int cur = 0;  // the lane's cell; its sequence indices only grow
+    // the trip count is the same on every lane: foundTerms needs the
+    // whole wave
+    for (uint32_t b0 = 0; b0 < total; b0 += kPhotonLoads * (uint32_t)nAct) {
+      uint32_t q[kPhotonLoads];
+      float4 xp[kPhotonLoads];
 #pragma unroll
-        for (uint32_t u = 0; u < kPhotonLoads; ++u) {
-          const uint32_t i = b0 + u * (uint32_t)nAct + (uint32_t)rank;
-          q[u] = ~0u;
-          if (i < total) {
-            while (runs[cur].y <= i) ++cur;
-            q[u] = runs[cur].x + i;
-          }
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < kPhotonLoads; ++u)
-          xp[u] = q[u] != ~0u ? g.sX[q[u]] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        // photons within the radius join the wave's queue; its terms are
-        // taken 64 at a time, one per lane, so the term's arithmetic runs
-        // on full waves instead of on the few lanes that found a photon
-#pragma unroll
-        for (uint32_t u = 0; u < kPhotonLoads; ++u) {
-          const V3 dlt = v3(xp[u].x, xp[u].y, xp[u].z) - c;
-          const bool in = q[u] != ~0u && dot(dlt, dlt) <= r2;
-          const unsigned long long mk = __ballot(in);
-          if (in) fq[(tail + (uint32_t)__popcll(mk & ltMask)) & 127u] = q[u];
-          tail += (uint32_t)__popcll(mk);
-          if (tail - head >= 64u) {
-            foundTerms(g, fq, head, 64u, nso, ngo, m, &acc, &found);
-            head += 64u;
-          }
+      for (uint32_t u = 0; u < kPhotonLoads; ++u) {
+        const uint32_t i = b0 + u * (uint32_t)nAct + (uint32_t)rank;
+        q[u] = ~0u;
+        if (i < total) {
+          while (runs[cur].y <= i) ++cur;
+          q[u] = runs[cur].x + i;
         }
       }
-      __builtin_amdgcn_wave_barrier();  // runs are rewritten for the next cells
+#pragma unroll
+      for (uint32_t u = 0; u < kPhotonLoads; ++u)
+        xp[u] = q[u] != ~0u ? g.sX[q[u]] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      // photons within the radius join the wave's queue; its terms are
+      // taken 64 at a time, one per lane, so the term's arithmetic runs
+      // on full waves instead of on the few lanes that found a photon
+#pragma unroll
+      for (uint32_t u = 0; u < kPhotonLoads; ++u) {
+        const V3 dlt = v3(xp[u].x, xp[u].y, xp[u].z) - c;
+        const bool in = q[u] != ~0u && dot(dlt, dlt) <= r2;
+        const unsigned long long mk = __ballot(in);
+        if (in) fq[(tail + (uint32_t)__popcll(mk & ltMask)) & 127u] = q[u];
+        tail += (uint32_t)__popcll(mk);
+        if (tail - head >= 64u) {
+          foundTerms(g, fq, head, 64u, ns, ng, m, &acc, &found);
+          head += 64u;
+        }
+      }
     }
-    if (tail != head) foundTerms(g, fq, head, tail - head, nso, ngo, m, &acc, &found);
-    // the 64 partial sums by a butterfly: each step adds the same two
-    // operands on both lanes of a pair (in either order), so every lane ends
-    // with the same total
-    acc.reduceWave();
-    for (int off = 32; off > 0; off >>= 1) found += __shfl_xor(found, off);
-    if ((int)lane == owner) {
-      myEst = acc.value(g);
-      myM = found;
-      if (acc.saturated()) atomicAdd(&g.counters[kCtrFluxOverflow], 1u);
-    }
+    __builtin_amdgcn_wave_barrier();  // runs are rewritten for the next cells
   }
-  *M = myM;
-  return myEst;
+  if (tail != head) foundTerms(g, fq, head, tail - head, ns, ng, m, &acc, &found);
+  // the 64 partial sums by a butterfly: each step adds the same two
+  // operands on both lanes of a pair (in either order), so every lane ends
+  // with the same total
+  acc.reduceWave();
+  for (int off = 32; off > 0; off >>= 1) found += __shfl_xor(found, off);
+  *M = found;
+  *saturated = acc.saturated();
+  return acc.value(g);
 }
 
 // Occupancy target of the camera kernel (waves per SIMD; 0: the compiler's
@@ -1125,7 +1174,13 @@ __global__ void __launch_bounds__(kB) HASTY_SPPM_CAMERA_ATTR kSppmCamera(DevScen
   }
 }
 
-// Occupancy target of the gather kernel (waves per SIMD; 0: the compiler's
+// The radius a pixel gathers with: its own once it has one.
+__device__ inline float pixelRadius(const SppmDev& g, uint32_t p) {
+  const float r = g.radius[p];
+  return r == -1.0f ? g.radii[p] : r;
+}
+
+// Occupancy target of the gather kernels (waves per SIMD; 0: the compiler's
 // choice, 146 VGPRs and 3 waves).  At 4 (128 VGPRs, 40 B of spills) the
 // 4M-photon gathers take 67 ms against 69 and the sparse ones 2.7 ms against
 // 3.2 on the 1920x1080 caustic box; 5 loses on the dense maps.
@@ -1139,55 +1194,113 @@ __global__ void __launch_bounds__(kB) HASTY_SPPM_CAMERA_ATTR kSppmCamera(DevScen
 #endif
 // The photon gathers of the pass's camera paths (photonMapFluxEstimate,
 // PhotonMapping.cpp:271-296, at each diffuse vertex of
-// pathTraceWithCausticsMap) and the pixel statistics update.  A wave holds 64
-// consecutive pixels; round v gathers every pixel's v-th query, and all 64
-// lanes stay in the loop so that the shared gather always has 64 ranks.
-// F_R = sum over the vertices in path order of W_R (Tb est), as the camera
-// path would have summed it.
+// pathTraceWithCausticsMap): task (v, k) is the v-th queries of the 64 pixels
+// from 64 k on, a wave each.  A gather's estimate and count of photons replace
+// the position and material in its query record.  Tasks with a query of many
+// candidates are listed for kSppmGatherShared.
+// One wave used to run all the rounds v of its pixels one after another and
+// shared gathers within, so a launch lasted as long as its heaviest 64 pixels:
+// 9.7 ms for the dense map's 833,000 queries and 273M candidates in the fifth
+// pass, 5.4 ms in tasks.  Bound by the latency of cell probes and photon loads.
 template <class Sum>
-__global__ void __launch_bounds__(kB) HASTY_SPPM_GATHER_ATTR kSppmGather(DevScene s, SppmDev g, float alpha,
-                                                                        int emittedInt, float* color) {
+__global__ void __launch_bounds__(kB) HASTY_SPPM_GATHER_ATTR kSppmGather(DevScene s, SppmDev g, uint32_t* tasks) {
   __shared__ uint2 gatherRuns[kB];
   __shared__ float4 gatherStaged[kB];
-  __shared__ uint32_t gatherFound[2 * kB];
-  const uint32_t P = s.width * s.height;
+  __shared__ uint2 gatherOwn[kOwnRuns * kB];
+  const uint32_t P = s.width * s.height, groups = (P + 63u) / 64u, lane = threadIdx.x & 63u;
+  const uint32_t waves = gridDim.x * (kB / 64), total = groups * (uint32_t)max(1, s.maxDepth);
   unsigned long long nQueries = 0, nCand = 0, nFound = 0;
-  for (uint32_t base = blockIdx.x * kB; base < P; base += gridDim.x * kB) {
-    const uint32_t p = base + threadIdx.x;
-    const bool valid = p < P;
-    float pxRadius = 0.0f;
-    uint32_t nq = 0;
-    if (valid) {
-      pxRadius = g.radius[p];
-      if (pxRadius == -1.0f) pxRadius = g.radii[p];
-      nq = g.nq[p];
+  for (uint32_t t = (blockIdx.x * kB + threadIdx.x) >> 6; t < total; t += waves) {
+    const uint32_t v = t / groups, p = (t - v * groups) * 64u + lane;
+    const bool has = p < P && v < g.nq[p];
+    if (__ballot(has) == 0ull) continue;
+    float4 q0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), q1 = q0, q2 = q0;
+    float radius = 0.0f;
+    float4* qr = g.query + 4 * ((size_t)v * P + p);
+    if (has) {
+      q0 = qr[0], q1 = qr[1], q2 = qr[2];
+      radius = pixelRadius(g, p);
     }
+    int M = 0;
+    uint32_t cand = 0;
+    V3 est;
+    const bool done = ownGather<Sum>(g, s, has, f4xyz(q0), f4xyz(q1), f4xyz(q2), __float_as_int(q0.w), radius, &M,
+                                     gatherRuns + (threadIdx.x & ~63u), gatherStaged + (threadIdx.x & ~63u),
+                                     gatherOwn + threadIdx.x, &cand, &est);
+    if (has) {
+      nQueries += 1;
+      nCand += cand;
+      if (done) {
+        nFound += (unsigned long long)M;
+        qr[0] = f4(est, __int_as_float(M));
+      }
+    }
+    if (!done && lane == 0) tasks[atomicAdd(&g.counters[kCtrShared], 1u)] = t;
+  }
+  // one atomic per wave and statistic
+  for (int off = 32; off > 0; off >>= 1) {
+    nQueries += __shfl_xor(nQueries, off);
+    nCand += __shfl_xor(nCand, off);
+    nFound += __shfl_xor(nFound, off);
+  }
+  if (lane == 0 && nQueries) {
+    atomicAdd(&g.gatherStats[0], nQueries);
+    atomicAdd(&g.gatherStats[1], nCand);
+    atomicAdd(&g.gatherStats[2], nFound);
+  }
+}
+
+// The listed tasks, kShareQueries queries to a wave: small pieces, since a
+// query of a caustic has thousands of candidates and one beside it none (1, 2,
+// 4, 8, 16: 10.67, 10.74, 10.85, 11.20, 11.42 ms a pass of the dense map).
+constexpr uint32_t kShareQueries = 1;
+template <class Sum>
+__global__ void __launch_bounds__(kB) HASTY_SPPM_GATHER_ATTR kSppmGatherShared(DevScene s, SppmDev g,
+                                                                              const uint32_t* tasks) {
+  __shared__ uint2 gatherRuns[kB];
+  __shared__ uint32_t gatherFound[2 * kB];
+  const uint32_t P = s.width * s.height, groups = (P + 63u) / 64u;
+  const uint32_t parts = 64u / kShareQueries, n = g.counters[kCtrShared] * parts;
+  const uint32_t waves = gridDim.x * (kB / 64);
+  unsigned long long nFound = 0;
+  for (uint32_t k = __builtin_amdgcn_readfirstlane((blockIdx.x * kB + threadIdx.x) >> 6); k < n; k += waves) {
+    const uint32_t t = tasks[k / parts], v = t / groups;
+    const uint32_t first = (t - v * groups) * 64u + (k % parts) * kShareQueries;
+    for (uint32_t p = first; p < min(first + kShareQueries, P); ++p) {
+      if (v >= g.nq[p]) continue;
+      float4* qr = g.query + 4 * ((size_t)v * P + p);
+      const float4 q0 = qr[0], q1 = qr[1], q2 = qr[2];
+      int M = 0;
+      bool saturated;
+      const V3 est = sharedGather<Sum>(g, s, f4xyz(q0), f4xyz(q1), f4xyz(q2), __float_as_int(q0.w), pixelRadius(g, p),
+                                       &M, gatherRuns + (threadIdx.x & ~63u), gatherFound + 2u * (threadIdx.x & ~63u),
+                                       &saturated);
+      if ((threadIdx.x & 63u) == 0) {
+        qr[0] = f4(est, __int_as_float(M));
+        if (saturated) atomicAdd(&g.counters[kCtrFluxOverflow], 1u);
+      }
+      nFound += (unsigned long long)M;
+    }
+  }
+  if ((threadIdx.x & 63u) == 0 && nFound) atomicAdd(&g.gatherStats[2], nFound);
+}
+
+// The pixels' statistics: F_R = sum over the vertices in path order of
+// W_R (Tb est), as the camera path would have summed it, then the update.
+__global__ void __launch_bounds__(kB) kSppmUpdate(DevScene s, SppmDev g, float alpha, int emittedInt, float* color) {
+  const uint32_t P = s.width * s.height;
+  for (uint32_t p = blockIdx.x * kB + threadIdx.x; p < P; p += gridDim.x * kB) {
+    float pxRadius = pixelRadius(g, p);
+    const uint32_t nq = g.nq[p];
     float radius = pxRadius;
-    uint32_t rounds = nq;
-    for (int off = 32; off > 0; off >>= 1) rounds = max(rounds, (uint32_t)__shfl_xor((int)rounds, off));
     V3 F0 = v3(0.0f, 0.0f, 0.0f);
     int Mtot = 0;
-    for (uint32_t v = 0; v < rounds; ++v) {
-      uint32_t cand = 0;
-      const bool has = v < nq;
-      float4 q0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), q1 = q0, q2 = q0, q3 = q0;
-      if (has) {
-        const float4* qr = g.query + 4 * ((size_t)v * P + p);
-        q0 = qr[0], q1 = qr[1], q2 = qr[2], q3 = qr[3];
-      }
-      int M = 0;
-      const V3 est = gatherQuery<Sum>(g, s, has, f4xyz(q0), f4xyz(q1), f4xyz(q2), __float_as_int(q0.w), radius,
-                                      &M, gatherRuns + (threadIdx.x & ~63u), gatherStaged + (threadIdx.x & ~63u),
-                                      gatherFound + 2u * (threadIdx.x & ~63u), &cand);
-      if (has) {
-        nQueries += 1;
-        nCand += cand;
-        nFound += (unsigned long long)M;
-        Mtot += M;
-        F0 = F0 + mul(f4xyz(q3), mul(v3(q1.w, q2.w, q3.w), est));
-      }
+    for (uint32_t v = 0; v < nq; ++v) {
+      const float4* qr = g.query + 4 * ((size_t)v * P + p);
+      const float4 q0 = qr[0], q3 = qr[3];
+      Mtot += __float_as_int(q0.w);
+      F0 = F0 + mul(f4xyz(q3), mul(v3(qr[1].w, qr[2].w, q3.w), f4xyz(q0)));
     }
-    if (!valid) continue;
     // PMRenderJob::unlockAndUpdateStatistic (PhotonMapping.h:63-105)
     const V3 L = v3(g.Lpath[p], g.Lpath[P + p], g.Lpath[2 * P + p]);
     bool bad = L.x != L.x || L.y != L.y || L.z != L.z || F0.x != F0.x || F0.y != F0.y || F0.z != F0.z;
@@ -1231,17 +1344,6 @@ __global__ void __launch_bounds__(kB) HASTY_SPPM_GATHER_ATTR kSppmGather(DevScen
     }
     g.radii[p] = radius;
     color[p * 3] = Lnew.x, color[p * 3 + 1] = Lnew.y, color[p * 3 + 2] = Lnew.z;
-  }
-  // one atomic per wave and statistic
-  for (int off = 32; off > 0; off >>= 1) {
-    nQueries += __shfl_xor(nQueries, off);
-    nCand += __shfl_xor(nCand, off);
-    nFound += __shfl_xor(nFound, off);
-  }
-  if ((threadIdx.x & 63u) == 0) {
-    atomicAdd(&g.gatherStats[0], nQueries);
-    atomicAdd(&g.gatherStats[1], nCand);
-    atomicAdd(&g.gatherStats[2], nFound);
   }
 }
 
@@ -1289,6 +1391,7 @@ SppmRenderer::SppmRenderer(const DevScene& scene, const SppmParams& params, cons
   // gather queries: at most one per path depth and pixel
   dQuery_ = alloc<float4>((size_t)4 * std::max(1, s_.maxDepth) * P);
   dNq_ = alloc<uint32_t>(P);
+  dTasks_ = alloc<uint32_t>((P + 63) / 64 * (size_t)std::max(1, s_.maxDepth));
   dLpath_ = alloc<float>(3 * P);
   dCounters_ = alloc<uint32_t>(8);
   dGatherStats_ = alloc<unsigned long long>(3);
@@ -1338,8 +1441,7 @@ SppmRenderer::SppmRenderer(const DevScene& scene, const SppmParams& params, cons
   uint32_t ts = 1024;
   while (ts < 2 * photonCap_) ts <<= 1;
   tableSize_ = ts;
-  dTableKeys_ = alloc<unsigned long long>(tableSize_);
-  dTableVals_ = alloc<uint2>(tableSize_);
+  dTable_ = alloc<uint4>(tableSize_);
   hipLaunchKernelGGL(kPixelInit, dim3(1024), dim3(kB), 0, stream_,
                      SppmDev{dPixel_, dPixel_ + P, dPixel_ + 2 * P, dPixel_ + 3 * P, dPixel_ + 6 * P,
                              (int*)(dPixel_ + 9 * P), dRadii_},
@@ -1431,8 +1533,7 @@ void SppmRenderer::pass(uint32_t passIndex, float offX, float offY, float* dColo
   g.sX = dSX_, g.sWi = dSWi_, g.sF = dSF_;
   g.keys = dKeys_;
   g.idx = dIdx_;
-  g.tKeys = dTableKeys_;
-  g.tVals = dTableVals_;
+  g.table = dTable_;
   g.tMask = tableSize_ - 1;
   g.bbox = dBox_;
   g.cellSize = dCellSize_;
@@ -1562,11 +1663,17 @@ void SppmRenderer::pass(uint32_t passIndex, float offX, float offY, float* dColo
   HC(hipGetLastError());
   if (timer) timer->end(kKSppmCamera, stream_);
   if (timer) timer->begin(kKSppmGather, stream_);
-  const dim3 gatherGrid((uint32_t)std::min<size_t>((P + kB - 1) / kB, 16384));
-  if (p_.fixedPointFlux)
-    hipLaunchKernelGGL(kSppmGather<FixedSum>, gatherGrid, dim3(kB), 0, stream_, s_, g, p_.alpha, (int)emitted, dColor);
-  else
-    hipLaunchKernelGGL(kSppmGather<FloatSum>, gatherGrid, dim3(kB), 0, stream_, s_, g, p_.alpha, (int)emitted, dColor);
+  const size_t gatherTasks = (P + 63) / 64 * (size_t)std::max(1, s_.maxDepth);
+  const dim3 gatherGrid((uint32_t)std::min<size_t>((gatherTasks + 3) / 4, 4096));
+  if (p_.fixedPointFlux) {
+    hipLaunchKernelGGL(kSppmGather<FixedSum>, gatherGrid, dim3(kB), 0, stream_, s_, g, dTasks_);
+    hipLaunchKernelGGL(kSppmGatherShared<FixedSum>, dim3(4096), dim3(kB), 0, stream_, s_, g, (const uint32_t*)dTasks_);
+  } else {
+    hipLaunchKernelGGL(kSppmGather<FloatSum>, gatherGrid, dim3(kB), 0, stream_, s_, g, dTasks_);
+    hipLaunchKernelGGL(kSppmGatherShared<FloatSum>, dim3(4096), dim3(kB), 0, stream_, s_, g, (const uint32_t*)dTasks_);
+  }
+  hipLaunchKernelGGL(kSppmUpdate, dim3((uint32_t)std::min<size_t>((P + kB - 1) / kB, 16384)), dim3(kB), 0, stream_, s_,
+                     g, p_.alpha, (int)emitted, dColor);
   HC(hipGetLastError());
   if (timer) timer->end(kKSppmGather, stream_);
   uint32_t c[kNumCtr];

@@ -396,7 +396,7 @@ typedef struct HastySppmParams {
    * is counted in HastySppmInfo.flux_overflows.  Default 0 (FP32). */
   int32_t fixed_point_flux;
   int32_t flux_frac_bits;            /* 0: 24; at most 40 */
-  uint32_t gather_share_candidates;  /* 0: 512; a wave gathers its queries together when one of them has
+  uint32_t gather_share_candidates;  /* 0: 128; a wave gathers its queries together when one of them has
                                         more candidate photons than this (no effect on the result with
                                         fixed-point flux) */
   float gather_union_factor;         /* > 0: such a wave reads the union of its queries' cells once, each
