@@ -71,7 +71,7 @@ class SppmRenderer {
   uint32_t passes_ = 0;
   SppmPassInfo info_;
   std::vector<void*> allocs_;
-  uint32_t traceBlocks_ = 0, partialBlocks_ = 0;
+  uint32_t traceBlocks_ = 0, cameraBlocks_ = 0, partialBlocks_ = 0;
   uint32_t emitLimit_ = 0, storeLimit_ = 0;
   // per pixel
   float* dPixel_ = nullptr;  // 10 planes
@@ -80,6 +80,7 @@ class SppmRenderer {
   // bytes), queries per pixel, path radiance (3 planes)
   float4* dQuery_ = nullptr;
   uint32_t* dNq_ = nullptr;
+  float4* dCamera_ = nullptr;   // two sets of camera paths between segments
   uint32_t* dTasks_ = nullptr;  // gather tasks of many candidates
   float* dLpath_ = nullptr;
   // cell size reductions

@@ -121,8 +121,11 @@ enum Counter {
   kCtrSelected = 5,      // photons of the batch that meet a caster's box
   kCtrTraced = 6,        // the last batch's
   kCtrShared = 7,        // gather tasks left to kSppmGatherShared
-  kNumCtr = 8
+  kNumCtr = 8            // then the paths alive at the end of each camera segment
 };
+// Vertices at which the camera paths are packed anew (see kSppmCamera).
+constexpr int kCameraCuts[] = {3, 7};
+constexpr int kCameraSegments = (int)(sizeof(kCameraCuts) / sizeof(int)) + 1;
 
 // ------------------------------------------------------------ cell size ----
 // PhotonMapping.cpp:522-576 as three reductions.  Each block writes its
@@ -971,8 +974,8 @@ __device__ inline V3 sharedGather(const SppmDev& g, const DevScene& s, V3 c, V3 
 }
 
 // Occupancy target of the camera kernel (waves per SIMD; 0: the compiler's
-// choice).  At 4 waves it spills ~200 B per lane and is still the fastest
-// on the 1920x1080 caustic box (3, 5 and 6 measured slower).
+// choice).  At 4 waves it spills ~300 B per lane and is still the fastest (the
+// caustic box's pass at 960x540: 4.37 ms, 5.01 with 3 waves).
 #ifndef HASTY_SPPM_CAMERA_WAVES
 #define HASTY_SPPM_CAMERA_WAVES 4
 #endif
@@ -982,43 +985,104 @@ __device__ inline V3 sharedGather(const SppmDev& g, const DevScene& s, V3 c, V3 
 #define HASTY_SPPM_CAMERA_ATTR
 #endif
 // --------------------------------------------------------------- camera ----
+__device__ inline void storeAux(float* normalOut, float* albedoOut, uint32_t p, V3 n, V3 a) {
+  normalOut[p * 3] = n.x, normalOut[p * 3 + 1] = n.y, normalOut[p * 3 + 2] = n.z;
+  albedoOut[p * 3] = a.x, albedoOut[p * 3 + 1] = a.y, albedoOut[p * 3 + 2] = a.z;
+}
 // renderPhotonThread's pixel loop (PhotonMapping.cpp:874-925) with
 // pathTraceWithCausticsMap (PhotonMapping.cpp:404-503) unrolled into one
 // path.  A node's result (photon flux F, light LL, rest LR, specular LS)
 // enters the pixel through per-node weights: W_R for F and LR, W_S for LS,
 // and a light hit reached through an edge (tD, tC) counts W_S(parent) tC +
 // W_R(parent) tD.  Children: W_S' = W_S tC, W_R' = W_R (tD + tC).
-__global__ void __launch_bounds__(kB) HASTY_SPPM_CAMERA_ATTR kSppmCamera(DevScene s, SppmDev g, uint32_t pass, float offX, float offY,
-                                                  float alpha, int emittedInt, float* color, float* normalOut,
-                                                  float* albedoOut) {
+// The paths run in segments of vertices [d0, d1): those still alive at d1 are
+// packed into `out`, and the next segment takes them from there with full
+// waves (and, once few are left, with few paths per wave, as kFinish does).
+// One launch over all vertices lasted as long as the longest of all paths, with
+// waves mostly of ended ones: 2.9 ms a pass of the caustic box at 960x540 and
+// 2.75 ms at 640x360, 2.1 and 1.7 ms in segments cut at vertices 3 and 7 (passes
+// with cuts 1 2 4 7; 2 4 8; 2 5; 3 7; every vertex: 4.36, 4.32, 4.26, 4.07, 4.56
+// ms).  Bound by the latency of a path's vertices; the kernel spills 300 B a
+// lane at 4 waves per SIMD and is slower at 3.  Which segment runs a vertex
+// changes nothing.
+struct CameraPaths {
+  float4* a;    // origin; w = media entries | wavelength + 1 << 4 | queries << 8 (bits)
+  float4* b;    // direction; w = random numbers drawn (bits)
+  float4* hit;  // t, u, v, triangle (bits)
+  float4* ws;   // W_S; w = pixel (bits)
+  float4* wr;   // W_R; w = LR.x
+  float4* wlr;  // W_LR; w = LR.y
+  float4* ls;   // LS; w = LR.z
+  uint4* media; // two per path
+};
+template <int W>
+__global__ void __launch_bounds__(kB) HASTY_SPPM_CAMERA_ATTR kSppmCamera(DevScene s, SppmDev g, uint32_t pass,
+                                                                        float offX, float offY, int d0, int d1,
+                                                                        CameraPaths in, const uint32_t* inCount,
+                                                                        CameraPaths out, uint32_t* outCount,
+                                                                        float* normalOut, float* albedoOut) {
   __shared__ uint2 stack[kStackRows * kB];
-  uint32_t P = s.width * s.height;
-  uint32_t gtid = xcdRemap() * kB + threadIdx.x;
-  uint2* ovf = g.ovf + (size_t)gtid * kStackOvf;
+  __shared__ uint32_t waveCount[kB / 64];
+  __shared__ uint32_t blockBase;
+  const uint32_t P = s.width * s.height;
+  const uint32_t n = d0 == 0 ? P : *inCount;
+  const uint32_t block = xcdRemap(), lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const uint32_t waves = gridDim.x * (kB / 64);
+  uint32_t per = 64u;  // paths per wave
+  while (per > 8u && n <= waves * (per / 2u)) per /= 2u;
+  uint2* ovf = g.ovf + (size_t)(block * kB + threadIdx.x) * kStackOvf;
   const bool twoStrategies = s.hasLight && s.useMIS;
-  for (uint32_t p = gtid; p < P; p += gridDim.x * kB) {
-    uint32_t i = p % s.width, j = p / s.width;
-    hrng::Stream rng = hrng::make_stream(s.seed, p, pass, hrng::kDomainPath);
-    V3 ro, rd;
-    cameraRay(s, rng, (float)i + offX, (float)j + offY, &ro, &rd);
-    V3 nrm = v3(0.0f, 0.0f, 0.0f), alb = v3(0.0f, 0.0f, 0.0f);
-    V3 LL0 = v3(0.0f, 0.0f, 0.0f), LR0 = v3(0.0f, 0.0f, 0.0f), LS0 = v3(0.0f, 0.0f, 0.0f);
-    V3 WS = v3(1.0f, 1.0f, 1.0f), WR = v3(1.0f, 1.0f, 1.0f), WLR = v3(0.0f, 0.0f, 0.0f);
+  for (uint32_t base = block * (kB / 64) * per; base < n; base += waves * per) {  // uniform over the block
+    const uint32_t at = base + wave * per + lane;
+    const bool mine = lane < per && at < n;
+    bool alive = false;  // at d1
+    uint32_t p = 0;
+    hrng::Stream rng = hrng::make_stream(s.seed, 0u, pass, hrng::kDomainPath);
+    V3 ro = v3(0.0f, 0.0f, 0.0f), rd = ro, LL0 = ro, LR0 = ro, LS0 = ro, WLR = ro;
+    V3 WS = v3(1.0f, 1.0f, 1.0f), WR = WS;
     uint32_t nq = 0;
     Media md;
     md.n = 0;
     md.overflow = false;
     md.tx0 = 0u;
     int wavelength = -1;
-    Hit h = traceClosest<kStackLds, kStackOvf>(s, ro, rd, stack + threadIdx.x, kB, ovf, nullptr, nullptr);
-    for (int depth = 0; depth < s.maxDepth; ++depth) {
+    Hit h;
+    h.t = h.u = h.v = 0.0f, h.tri = -1;
+    if (mine && d0 == 0) {
+      p = at;
+      rng.stream = p;
+      cameraRay(s, rng, (float)(p % s.width) + offX, (float)(p / s.width) + offY, &ro, &rd);
+      h = traceClosest<kStackLds, kStackOvf, W>(s, ro, rd, stack + threadIdx.x, kB, ovf, nullptr, nullptr);
+    } else if (mine) {
+      const float4 a = in.a[at], b = in.b[at], hh = in.hit[at], ws = in.ws[at], wr = in.wr[at], wlr = in.wlr[at],
+                   ls = in.ls[at];
+      const uint32_t bits = __float_as_uint(a.w);
+      ro = f4xyz(a), rd = f4xyz(b), WS = f4xyz(ws), WR = f4xyz(wr), WLR = f4xyz(wlr), LS0 = f4xyz(ls);
+      LR0 = v3(wr.w, wlr.w, ls.w);
+      rng.counter = __float_as_uint(b.w);
+      h.t = hh.x, h.u = hh.y, h.v = hh.z, h.tri = __float_as_int(hh.w);
+      p = __float_as_uint(ws.w);
+      rng.stream = p;
+      md.n = (int)(bits & 15u);
+      wavelength = (int)((bits >> 4) & 15u) - 1;
+      nq = bits >> 8;
+      const uint4 m0 = in.media[2 * (size_t)at], m1 = in.media[2 * (size_t)at + 1];
+      md.e[0] = m0.x, md.e[1] = m0.y, md.e[2] = m0.z, md.e[3] = m0.w;
+      md.e[4] = m1.x, md.e[5] = m1.y, md.e[6] = m1.z, md.e[7] = m1.w;
+    }
+    // no vertices: not even the first one's normal and albedo
+    if (mine && s.maxDepth <= 0) storeAux(normalOut, albedoOut, p, v3(0.0f, 0.0f, 0.0f), v3(0.0f, 0.0f, 0.0f));
+    for (int depth = mine ? d0 : s.maxDepth; depth < s.maxDepth; ++depth) {
+      if (depth == d1) {
+        alive = true;
+        break;
+      }
       if (h.tri < 0) {
         V3 T = beersLaw(mediaTransmittance(s, md), 1e6f);
         V3 LR = mul(T, evalEnvironment(s, rd));
         if (depth == 0) {
           LR0 = LR;
-          nrm = v3(0.0f, 0.0f, 0.0f);
-          alb = LR;
+          storeAux(normalOut, albedoOut, p, v3(0.0f, 0.0f, 0.0f), LR);
         } else {
           LR0 = LR0 + mul(WR, LR);
         }
@@ -1026,10 +1090,7 @@ __global__ void __launch_bounds__(kB) HASTY_SPPM_CAMERA_ATTR kSppmCamera(DevScen
       }
       Interaction it = makeInteraction(s, h.tri, h.u, h.v);
       const DevMaterial& m = s.mats[it.mat];
-      if (depth == 0) {
-        nrm = it.ns;
-        alb = albedoOf(m);
-      }
+      if (depth == 0) storeAux(normalOut, albedoOut, p, it.ns, albedoOf(m));
       V3 Tb = beersLaw(mediaTransmittance(s, md), norm(it.x - ro));
       V3 wo = -rd;
       if (m.isLight) {
@@ -1092,7 +1153,7 @@ __global__ void __launch_bounds__(kB) HASTY_SPPM_CAMERA_ATTR kSppmCamera(DevScen
         Hit hl;
         hl.tri = -2;  // not traced
         if (lit && !isZero(ev.fD + ev.fC))
-          hl = traceClosest<kStackLds, kStackOvf>(s, so, sd, stack + threadIdx.x, kB, ovf, nullptr, nullptr);
+          hl = traceClosest<kStackLds, kStackOvf, W>(s, so, sd, stack + threadIdx.x, kB, ovf, nullptr, nullptr);
         bool visible = hl.tri != -2 && (target >= 0 ? hl.tri == target
                                                      : (hl.tri < 0 || s.mats[s.triMat[hl.tri]].isLight));
         if (visible) {
@@ -1141,7 +1202,7 @@ __global__ void __launch_bounds__(kB) HASTY_SPPM_CAMERA_ATTR kSppmCamera(DevScen
       // zero throughput (including pdf 0) ends the path before any trace
       if (bs.pdf == 0.0f || isZero(bs.tD + bs.tC)) break;
       V3 no = offsetOrigin(it, bs.outside);
-      Hit h2 = traceClosest<kStackLds, kStackOvf>(s, no, bs.dir, stack + threadIdx.x, kB, ovf, nullptr, nullptr);
+      Hit h2 = traceClosest<kStackLds, kStackOvf, W>(s, no, bs.dir, stack + threadIdx.x, kB, ovf, nullptr, nullptr);
       if (h2.tri == it.tri) break;
       float w;
       {
@@ -1166,11 +1227,37 @@ __global__ void __launch_bounds__(kB) HASTY_SPPM_CAMERA_ATTR kSppmCamera(DevScen
       rd = bs.dir;
       h = h2;
     }
-    const V3 L = LL0 + LR0 + LS0;
-    g.Lpath[p] = L.x, g.Lpath[P + p] = L.y, g.Lpath[2 * P + p] = L.z;
-    g.nq[p] = nq;
-    normalOut[p * 3] = nrm.x, normalOut[p * 3 + 1] = nrm.y, normalOut[p * 3 + 2] = nrm.z;
-    albedoOut[p * 3] = alb.x, albedoOut[p * 3 + 1] = alb.y, albedoOut[p * 3 + 2] = alb.z;
+    if (mine && !alive) {
+      const V3 L = LL0 + LR0 + LS0;
+      g.Lpath[p] = L.x, g.Lpath[P + p] = L.y, g.Lpath[2 * P + p] = L.z;
+      g.nq[p] = nq;
+    }
+    const unsigned long long mask = __ballot(alive);
+    if (lane == 0) waveCount[wave] = (uint32_t)__popcll(mask);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      uint32_t sum = 0;
+      for (uint32_t w = 0; w < kB / 64; ++w) {
+        const uint32_t c = waveCount[w];
+        waveCount[w] = sum;
+        sum += c;
+      }
+      blockBase = sum ? atomicAdd(outCount, sum) : 0u;
+    }
+    __syncthreads();
+    if (alive) {  // LL is zero: only the first vertex sets it, and such a path ends there
+      const uint32_t k = blockBase + waveCount[wave] + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+      out.a[k] = f4(ro, __uint_as_float((uint32_t)md.n | ((uint32_t)(wavelength + 1) << 4) | (nq << 8)));
+      out.b[k] = f4(rd, __uint_as_float(rng.counter));
+      out.hit[k] = make_float4(h.t, h.u, h.v, __int_as_float(h.tri));
+      out.ws[k] = f4(WS, __uint_as_float(p));
+      out.wr[k] = f4(WR, LR0.x);
+      out.wlr[k] = f4(WLR, LR0.y);
+      out.ls[k] = f4(LS0, LR0.z);
+      out.media[2 * (size_t)k] = make_uint4(md.e[0], md.e[1], md.e[2], md.e[3]);
+      out.media[2 * (size_t)k + 1] = make_uint4(md.e[4], md.e[5], md.e[6], md.e[7]);
+    }
+    __syncthreads();
   }
 }
 
@@ -1393,13 +1480,15 @@ SppmRenderer::SppmRenderer(const DevScene& scene, const SppmParams& params, cons
   dNq_ = alloc<uint32_t>(P);
   dTasks_ = alloc<uint32_t>((P + 63) / 64 * (size_t)std::max(1, s_.maxDepth));
   dLpath_ = alloc<float>(3 * P);
-  dCounters_ = alloc<uint32_t>(8);
+  dCounters_ = alloc<uint32_t>(kNumCtr + kCameraSegments);
+  dCamera_ = alloc<float4>(2 * 9 * P);
   dGatherStats_ = alloc<unsigned long long>(3);
   dCellSize_ = alloc<float>(4);
   dCand_ = alloc<float>(16);
   dState_ = alloc<float>(4);
   dBox_ = alloc<int>(8);
   traceBlocks_ = 2048;
+  cameraBlocks_ = 1024;  // the kernel's 4 waves per SIMD
   dOverflow_ = alloc<uint2>((size_t)traceBlocks_ * kB * kStackOvf);
   partialBlocks_ = 512;
   dPartial_ = alloc<float>((size_t)partialBlocks_ * kCandidates);
@@ -1566,7 +1655,7 @@ void SppmRenderer::pass(uint32_t passIndex, float offX, float offY, float* dColo
   if (timer) timer->end(kKSppmCellSize, stream_);
 
   // 2. photons
-  hipLaunchKernelGGL(kZeroU32, dim3(1), dim3(64), 0, stream_, dCounters_, 8u);
+  hipLaunchKernelGGL(kZeroU32, dim3(1), dim3(64), 0, stream_, dCounters_, (uint32_t)(kNumCtr + kCameraSegments));
   hipLaunchKernelGGL(kZeroU64, dim3(1), dim3(64), 0, stream_, dGatherStats_, 3u);
   uint32_t stored = 0, emitted = 0, next = 0;
   if (s_.hasSurfaceLight) {
@@ -1658,8 +1747,29 @@ void SppmRenderer::pass(uint32_t passIndex, float offX, float offY, float* dColo
   // 4. camera paths (recording their gathers), then the gathers and the
   // statistics
   if (timer) timer->begin(kKSppmCamera, stream_);
-  hipLaunchKernelGGL(kSppmCamera, dim3(traceBlocks_), dim3(kB), 0, stream_, s_, g, passIndex, offX, offY, p_.alpha,
-                     (int)emitted, dColor, dNormal, dAlbedo);
+  {
+    const size_t P16 = P * 16;
+    CameraPaths sets[2];
+    for (int k = 0; k < 2; ++k) {
+      char* m = (char*)dCamera_ + (size_t)k * 9 * P16;
+      sets[k] = CameraPaths{(float4*)m, (float4*)(m + P16), (float4*)(m + 2 * P16), (float4*)(m + 3 * P16),
+                            (float4*)(m + 4 * P16), (float4*)(m + 5 * P16), (float4*)(m + 6 * P16),
+                            (uint4*)(m + 7 * P16)};
+    }
+    const dim3 grid(std::min<uint32_t>(cameraBlocks_, (uint32_t)(((P + 8 * (kB / 64) - 1) / (8 * (kB / 64)) + 7) & ~(size_t)7)));
+    int seg = 0;
+    for (int d0 = 0; d0 < std::max(1, s_.maxDepth); ++seg) {
+      const int d1 = seg < kCameraSegments - 1 ? kCameraCuts[seg] : 0x7FFFFFFF;
+      const uint32_t* inCount = dCounters_ + kNumCtr + seg - 1;
+      if (s_.bvhWidth == 8)
+        hipLaunchKernelGGL(kSppmCamera<8>, grid, dim3(kB), 0, stream_, s_, g, passIndex, offX, offY, d0, d1,
+                           sets[seg & 1], inCount, sets[(seg & 1) ^ 1], dCounters_ + kNumCtr + seg, dNormal, dAlbedo);
+      else
+        hipLaunchKernelGGL(kSppmCamera<4>, grid, dim3(kB), 0, stream_, s_, g, passIndex, offX, offY, d0, d1,
+                           sets[seg & 1], inCount, sets[(seg & 1) ^ 1], dCounters_ + kNumCtr + seg, dNormal, dAlbedo);
+      d0 = d1;
+    }
+  }
   HC(hipGetLastError());
   if (timer) timer->end(kKSppmCamera, stream_);
   if (timer) timer->begin(kKSppmGather, stream_);
