@@ -28,13 +28,13 @@ struct V3 {
   float x, y, z;
 };
 __host__ __device__ inline V3 v3(float x, float y, float z) { return V3{x, y, z}; }
-__device__ inline V3 operator+(V3 a, V3 b) { return V3{a.x + b.x, a.y + b.y, a.z + b.z}; }
-__device__ inline V3 operator-(V3 a, V3 b) { return V3{a.x - b.x, a.y - b.y, a.z - b.z}; }
+__host__ __device__ inline V3 operator+(V3 a, V3 b) { return V3{a.x + b.x, a.y + b.y, a.z + b.z}; }
+__host__ __device__ inline V3 operator-(V3 a, V3 b) { return V3{a.x - b.x, a.y - b.y, a.z - b.z}; }
 __device__ inline V3 operator-(V3 a) { return V3{-a.x, -a.y, -a.z}; }
 __device__ inline V3 operator*(V3 a, float s) { return V3{a.x * s, a.y * s, a.z * s}; }
 __device__ inline V3 operator*(float s, V3 a) { return V3{a.x * s, a.y * s, a.z * s}; }
 __device__ inline V3 operator/(V3 a, float s) { return V3{a.x / s, a.y / s, a.z / s}; }
-__device__ inline V3 mul(V3 a, V3 b) { return V3{a.x * b.x, a.y * b.y, a.z * b.z}; }
+__host__ __device__ inline V3 mul(V3 a, V3 b) { return V3{a.x * b.x, a.y * b.y, a.z * b.z}; }
 __device__ inline float dot(V3 a, V3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 __device__ inline V3 cross(V3 a, V3 b) {
   return V3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
@@ -59,9 +59,13 @@ template <class T>
 __device__ inline T ldg(const T* p) {
   return *(const __attribute__((address_space(1))) T*)p;
 }
-__device__ inline float4 ldg4(const float4* p) {
+__host__ __device__ inline float4 ldg4(const float4* p) {
+#ifdef __HIP_DEVICE_COMPILE__
   const HNf4 v = *(const __attribute__((address_space(1))) HNf4*)p;
   return make_float4(v.x, v.y, v.z, v.w);
+#else
+  return *p;
+#endif
 }
 __device__ inline V3 load3g(const float* p) { return V3{ldg(p), ldg(p + 1), ldg(p + 2)}; }
 // Copy of a plain struct in global memory, by words.
@@ -76,7 +80,7 @@ __device__ inline T ldgStruct(const T* p) {
   __builtin_memcpy(&out, w, sizeof(T));
   return out;
 }
-__device__ inline V3 f4xyz(float4 a) { return V3{a.x, a.y, a.z}; }
+__host__ __device__ inline V3 f4xyz(float4 a) { return V3{a.x, a.y, a.z}; }
 __device__ inline float4 f4(V3 a, float w) { return make_float4(a.x, a.y, a.z, w); }
 
 // VMath.h:461-488
@@ -205,14 +209,24 @@ struct RayPre {
   V3 binv, ob;
   uint32_t nearX, nearY, nearZ;
 };
-__device__ inline float c3(V3 a, int i) { return i == 0 ? a.x : (i == 1 ? a.y : a.z); }
-__device__ inline RayPre prepareRay(V3 o, V3 d) {
+__host__ __device__ inline float c3(V3 a, int i) { return i == 0 ? a.x : (i == 1 ? a.y : a.z); }
+__host__ __device__ inline RayPre prepareRay(V3 o, V3 d) {
   RayPre r;
   r.o = o;
   r.binv = v3(1.0f / copysignf(fmaxf(__builtin_fabsf(d.x), 1e-20f), d.x),
               1.0f / copysignf(fmaxf(__builtin_fabsf(d.y), 1e-20f), d.y),
               1.0f / copysignf(fmaxf(__builtin_fabsf(d.z), 1e-20f), d.z));
   r.ob = mul(o, r.binv);
+  // A ray that is not finite hits nothing.  Its planes may be NaN on every
+  // axis, and the slab test's maxima and minima drop a NaN, so it would enter
+  // every box and every empty slot (whose ref leads out of the tree).  Instead
+  // every plane across x, +inf ones too, is at t = +inf: no child is entered.
+  // (A product with zero is NaN for NaN and infinities.)
+  const float zero = 0.0f * o.x + 0.0f * o.y + 0.0f * o.z + 0.0f * d.x + 0.0f * d.y + 0.0f * d.z;
+  if (!(zero == 0.0f)) {
+    r.binv.x = 1.0f;
+    r.ob.x = -__builtin_inff();
+  }
   r.nearX = r.binv.x >= 0.0f ? 0u : 16u;
   r.nearY = r.binv.y >= 0.0f ? 32u : 48u;
   r.nearZ = r.binv.z >= 0.0f ? 64u : 80u;
@@ -238,7 +252,7 @@ struct Hit {
 };
 
 // Watertight ray/triangle test (Woop, Benthin, Wald, JCGT 2013), t > tnear.
-__device__ inline bool intersectTri(const RayPre& r, float4 p0, float4 p1, float4 p2, float tnear, float* tOut,
+__host__ __device__ inline bool intersectTri(const RayPre& r, float4 p0, float4 p1, float4 p2, float tnear, float* tOut,
                                     float* uOut, float* vOut) {
   V3 A = f4xyz(p0) - r.o, B = f4xyz(p1) - r.o, C = f4xyz(p2) - r.o;
   float Akz = c3(A, r.kz), Bkz = c3(B, r.kz), Ckz = c3(C, r.kz);
@@ -311,7 +325,7 @@ struct Walk {
   int sp;        // stack depth
   uint32_t nNodes, nTris;
 };
-__device__ inline void walkInit(Walk& w, const RayPre& r, float tBound, int32_t idBound) {
+__host__ __device__ inline void walkInit(Walk& w, const RayPre& r, float tBound, int32_t idBound) {
   w.r = r;
   w.tBound = tBound;
   w.idBound = idBound;
@@ -332,12 +346,13 @@ __device__ inline void walkInit(Walk& w, const RayPre& r, float tBound, int32_t 
 // rounded binv and ob, the computed t is ((L - o) - o e1) (1 + e2) / d with
 // |e1| <= u, |e2| <= 2.1 u: the exact t of a plane moved by at most u |o| +
 // 2.1 u |L - o|, or a relative error.  Let M be the scene's largest coordinate
-// along the axis.  If |o| <= 2 M the move is below 2^-21 M, and the builder has
-// widened every box by 2^-19 M; else |L - o| >= |o| / 2 and the relative error
-// is below 5 u, twice which the exit's factor 1 + 16 u covers.
+// along the axis.  If |o| <= 2 M then |L - o| <= 3 M and the move is at most
+// 8.3 u M, below 2^-20 M, and the builder has widened every box by 2^-19 M; else
+// |L - o| >= |o| / 2 and the relative error is below 5 u, twice which the exit's
+// factor 1 + 16 u covers.  (Rays that are not finite enter nothing: prepareRay.)
 //
 // An empty slot's planes are all +inf, so its entry is +inf or its exit -inf.
-__device__ inline void testHalf(const DevScene& s, const RayPre& r, uint32_t half, float tb, float* e, uint32_t* ref) {
+__host__ __device__ inline void testHalf(const DevScene& s, const RayPre& r, uint32_t half, float tb, float* e, uint32_t* ref) {
   // 32-bit byte offsets from the node array (< 4 GiB of nodes)
   const char* nb = reinterpret_cast<const char*>(s.nodes);
   const uint32_t no = half * 128u;
@@ -352,13 +367,20 @@ __device__ inline void testHalf(const DevScene& s, const RayPre& r, uint32_t hal
     const float t1 = fminf(fminf(__builtin_fmaf(fx.C, r.binv.x, -r.ob.x), __builtin_fmaf(fy.C, r.binv.y, -r.ob.y)), \
                            __builtin_fmaf(fz.C, r.binv.z, -r.ob.z));                                            \
     e[K] = t0 <= fminf(t1 * kTmaxScale, tb) ? t0 : __builtin_inff();                                           \
-    ref[K] = __float_as_uint(rf.C);                                                                            \
+    ref[K] = __builtin_bit_cast(uint32_t, rf.C);                                                                         \
   }
   HDEV_SLAB(x, 0)
   HDEV_SLAB(y, 1)
   HDEV_SLAB(z, 2)
   HDEV_SLAB(w, 3)
 #undef HDEV_SLAB
+}
+
+// Leaf ref past its first triangle; true when no triangle is left (an empty
+// slot, which has none, loses its flag here and ends as well).
+__host__ __device__ inline bool leafNext(uint32_t& ref) {
+  ref += 1u - (1u << 24);
+  return ref < kLeafFlag + (1u << 24);
 }
 
 // One step; true when the walk has ended (w.best then holds the result,
@@ -391,8 +413,7 @@ __device__ inline bool walkStep(const DevScene& s, Walk& w, uint2* ldsGeneric, i
       const float4 p0 = ldg4(tr), p1 = ldg4(tr + 1), p2 = ldg4(tr + 2);
       const int32_t id = (int32_t)__float_as_uint(p0.w);
       w.nTris++;
-      w.ref += 1u - (1u << 24);  // the leaf's remaining triangles
-      pop = (w.ref & 0x7F000000u) == 0u;
+      pop = leafNext(w.ref);
       float t, u, v;
       if (intersectTri(r, p0, p1, p2, 1e-6f, &t, &u, &v)) {
         if (CLOSEST) {
