@@ -203,19 +203,26 @@ struct RayPre {
   int kx, ky, kz;
   float Sx, Sy, Sz;
   // box tests: t of plane L along an axis = fma(L, binv, -ob) with binv = 1 / d
-  // (components of d clamped to |d| >= 1e-20, so that no t is NaN) and ob =
+  // (components of d clamped, see boxReciprocal, so that no t is NaN) and ob =
   // o binv; near* = byte offset in a node of the float4 holding each axis'
   // near planes (lo when binv >= 0).
   V3 binv, ob;
   uint32_t nearX, nearY, nearZ;
 };
 __host__ __device__ inline float c3(V3 a, int i) { return i == 0 ? a.x : (i == 1 ? a.y : a.z); }
+// 1 / d with |d| at least 1e-20, and at least 2^-126 |o|, from |o| = 8.5e17 on the
+// larger: o / d then is at most 2^126.  Were it infinite, the t of every plane
+// along the axis would be -inf, or NaN at an empty slot.  The second clamp moves
+// the ray along the axis by less than the boxes' widening (2^-18 of where it is)
+// within t = 2^107.
+__host__ __device__ inline float boxReciprocal(float o, float d) {
+  const float least = fmaxf(1e-20f, __builtin_fabsf(o) * 0x1p-126f);
+  return 1.0f / copysignf(fmaxf(__builtin_fabsf(d), least), d);
+}
 __host__ __device__ inline RayPre prepareRay(V3 o, V3 d) {
   RayPre r;
   r.o = o;
-  r.binv = v3(1.0f / copysignf(fmaxf(__builtin_fabsf(d.x), 1e-20f), d.x),
-              1.0f / copysignf(fmaxf(__builtin_fabsf(d.y), 1e-20f), d.y),
-              1.0f / copysignf(fmaxf(__builtin_fabsf(d.z), 1e-20f), d.z));
+  r.binv = v3(boxReciprocal(o.x, d.x), boxReciprocal(o.y, d.y), boxReciprocal(o.z, d.z));
   r.ob = mul(o, r.binv);
   // A ray that is not finite hits nothing.  Its planes may be NaN on every
   // axis, and the slab test's maxima and minima drop a NaN, so it would enter

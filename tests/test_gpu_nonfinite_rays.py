@@ -1,12 +1,13 @@
-"""Rays that are not finite (masked-out entries of a host program's arrays) miss
-in every query form, and the ordinary rays that share a wave with them keep
+"""Rays that are not finite (masked-out entries of a host program's arrays) and
+rays from so far out that origin / direction overflows miss in every query form,
+and the ordinary rays that share a wave with them keep
 their hits.  tests/test_walk_cpu.py walks the same rays on the host with every
 index checked."""
 import numpy as np
 import pytest
 
 import hastyrenderer_amd as ha
-from test_walk_cpu import nonfinite_rays
+from test_walk_cpu import nonfinite_rays, overflowing_rays
 from test_zz_no_alloc import _Dev, _noalloc
 
 pytestmark = pytest.mark.gpu
@@ -17,7 +18,7 @@ RECORD = np.dtype([("geom_id", "<u4"), ("prim_id", "<u4"), ("t", "<f4"), ("u", "
 
 def _mixed(every):
     """Ordinary rays with every `every`-th one replaced."""
-    bad = nonfinite_rays()
+    bad = np.concatenate([nonfinite_rays(), overflowing_rays()])
     rng = np.random.default_rng(every)
     n = every * len(bad)
     d = rng.normal(size=(n, 3))
@@ -30,7 +31,7 @@ def _mixed(every):
 
 @pytest.mark.parametrize("width", [4, 8])
 @pytest.mark.parametrize("every", [1, 2, 7])
-def test_nonfinite_rays_miss(cornell_job, ggx_small_job, every, width):
+def test_unusable_rays_miss(cornell_job, ggx_small_job, every, width):
     rays, mixed, bad = _mixed(every)
     for job in (cornell_job, ggx_small_job):
         sc = ha.Scene(job)

@@ -1,7 +1,8 @@
 """The BVH walk on the host (tests/csrc/walk_host.hip: the renderer's own slab
 test, leaf step and triangle test, every index checked): rays that are not
-finite stay inside the tree and miss, and every other ray's hit is the one the
-triangle test finds over all triangles.  Trees with empty slots, both node widths."""
+finite and rays whose slab arithmetic overflows stay inside the tree and miss,
+and every other ray's hit is the one the triangle test finds over all
+triangles.  Trees with empty slots, both node widths."""
 import ctypes as C
 import itertools
 
@@ -50,6 +51,13 @@ def nonfinite_rays():
     return np.array(rays, np.float32)
 
 
+def overflowing_rays():
+    """Finite rays for which origin / direction exceeds the largest float."""
+    return np.array([(s * b,) * 3 + (x, y, z) for b in (1e19, 1e30, 3e38) for s in (-1.0, 1.0)
+                     for x, y, z in itertools.product((0.0, -0.0, 1e-20, -1e-20, 1e-38, 1.0, 3e38), repeat=3)],
+                    np.float32)
+
+
 @pytest.mark.parametrize("width", [4, 8])
 @pytest.mark.parametrize("ntris", [0, 1, 2, 5, 21, 300])
 def test_nonfinite_rays_miss(ntris, width):
@@ -59,13 +67,28 @@ def test_nonfinite_rays_miss(ntris, width):
 
 
 @pytest.mark.parametrize("width", [4, 8])
+@pytest.mark.parametrize("ntris", [1, 2, 5, 21])
+def test_overflowing_slabs_stay_in_the_tree(ntris, width):
+    rays = overflowing_rays()
+    tris = _soup(ntris)
+    tri, _, status = _walk(tris, width, rays)
+    assert (status == 0).all()
+    assert np.array_equal(tri, _walk(tris, 0, rays)[0])
+
+
+@pytest.mark.parametrize("width", [4, 8])
 @pytest.mark.parametrize("ntris", [1, 2, 5, 21, 300])
-@pytest.mark.parametrize("offset", [0.0, 1e5])
+@pytest.mark.parametrize("offset", [0.0, 1e5, 1e20])
 def test_finite_rays_hit_what_the_triangle_test_finds(ntris, width, offset):
-    """Scattered and axis-parallel rays, also where the scene lies far out."""
+    """Scattered and axis-parallel rays, also where the scene lies so far out
+    along x that an axis-parallel ray's origin / direction overflows."""
     tris = _soup(ntris)
     rays = _rays(3000)
     rays[::3, 3:] = np.eye(3)[np.arange(1000) % 3] * np.where(np.arange(1000) % 2, 1.0, -1.0)[:, None]
+    if offset == 1e20:  # slabs in x: the spacing of floats at 1e20 is 8.8e12
+        tris[:, :, 0] *= 1e14
+        rays[:, 0] *= 1e14
+        rays[:, 3:] = [0.0, 0.0, 1.0]
     tris[:, :, 0] += np.float32(offset)
     rays = rays.astype(np.float32)
     rays[:, 0] += np.float32(offset)
