@@ -17,6 +17,7 @@
 
 #include "bvh.h"
 #include "capi_internal.h"
+#include "pool_plan.h"
 #include "pt_kernels.h"
 #include "rng.h"
 #include "image_io.h"
@@ -187,7 +188,6 @@ struct HastyScene {
   std::vector<void*> pathAllocs;
   uint32_t poolCapacity = 0, poolRing = 0;  // allocated paths and ring entries
   uint32_t poolMost = 0xFFFFFFFFu, ringMost = 0xFFFFFFFFu;  // what an allocation failed above
-  static constexpr uint32_t kDefaultSlots = 1u << 24;
   uint32_t slotsWanted = 0;  // 0 = automatic
   uint32_t* dTileOrder = nullptr;
   uint32_t tileW = 0, tileH = 0;
@@ -281,32 +281,14 @@ struct HastyScene {
     dev.height = st.height;
   }
 
-  // Paths in flight (a path that ends makes room for the next) of a render of
-  // `paths` paths: the wanted pool (default 2^24), but no more than the
-  // render needs (at least 2^16).  Larger pools spread a bounce's fixed costs
-  // (the tail of its longest rays) over more rays: 132 ms at 2^22, 129 at
-  // 2^23, 125 at 2^24, 122 at 2^25 for 128 samples of the 1024x1024 GGX grid.
-  uint32_t slotCount(uint64_t paths) const {
-    uint64_t want = slotsWanted ? slotsWanted : kDefaultSlots;
-    return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(want, std::max<uint64_t>(paths, 1ull << 16)));
-  }
-  // Results ring: the whole render if it is no more than about 2^27 paths
-  // (finished paths wait in the ring for the oldest one in flight, so a ring
-  // much longer than a pool x depth never holds a path's start up), else
-  // whole samples of this scene's film.
-  uint32_t ringPathsWanted(uint64_t paths) const {
-    const uint64_t P = (uint64_t)dev.width * dev.height, most = 1ull << 27;
-    if (paths <= std::max(P, most)) return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(paths, 1), 0x7FFFFFFFull);
-    return (uint32_t)std::min<uint64_t>(std::max(P, most / P * P), 0x7FFFFFFFull / P * P);
-  }
-
   // Buffers of a render call; grown when a call needs more, else kept (a call
   // that needs less uses a part).  A pool or ring that does not fit the free
   // memory is halved until it does.
-  void ensurePathBuffers(uint64_t paths, bool late, bool textured) {
-    const uint32_t need = std::min(slotCount(paths), poolMost);
-    const uint64_t P = (uint64_t)dev.width * dev.height;
-    const uint32_t ring = (uint32_t)std::min<uint64_t>(ringPathsWanted(paths), std::max<uint64_t>(ringMost, P));
+  void ensurePathBuffers(const hasty::PoolNeed& call) {
+    bool late = call.late, textured = call.textured;
+    const uint64_t P = call.film;
+    const uint32_t need = std::min(hasty::poolPaths(call, slotsWanted), poolMost);
+    const uint32_t ring = (uint32_t)std::min<uint64_t>(hasty::ringPaths(call), std::max<uint64_t>(ringMost, P));
     const uint32_t traceThreads = launch.traceBlocks * hasty::kBlock;
     const bool fits = need <= poolCapacity && ring <= poolRing && traceThreads <= pb.traceThreads &&
                       (!late || pb.sh.lateQ) && (!textured || pb.set[0].mediaTx);
@@ -452,15 +434,14 @@ static void renderBatch(HastyScene* owner, const BatchItem* items, uint32_t nIte
     renderGuided(owner, items[0]);
     return;
   }
-  uint64_t allPaths = 0;
-  bool late = false, textured = false;
+  hasty::PoolNeed need;
   for (uint32_t i = 0; i < nItems; ++i) {
     const hdev::DevScene& d = items[i].scene->dev;
-    allPaths += (uint64_t)items[i].n * d.width * d.height;
-    late = late || (d.hasEnv && d.hasSurfaceLight);
-    textured = textured || d.texturedMedia;
+    need.add(items[i].n, (uint64_t)d.width * d.height);
+    need.late = need.late || (d.hasEnv && d.hasSurfaceLight);
+    need.textured = need.textured || d.texturedMedia;
   }
-  owner->ensurePathBuffers(allPaths, late, textured);
+  owner->ensurePathBuffers(need);
   // Split every item into calls of < 2^31 paths and lay out all Halton
   // offsets in one upload to the owner's offset buffer.
   struct Piece {
@@ -572,7 +553,11 @@ static void renderGuided(HastyScene* s, const BatchItem& it) {
   const bool training = s->guideLr > 0.0f;
   const uint64_t groupPaths = training ? HastyScene::kGuideTrainPaths : 0x7FFFFFFFull;
   const uint32_t perCall = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(it.n, groupPaths / P));
-  s->ensurePathBuffers(perCall * P, s->dev.hasEnv && s->dev.hasSurfaceLight, s->dev.texturedMedia != 0);
+  hasty::PoolNeed need;
+  need.add(perCall, P);
+  need.late = s->dev.hasEnv && s->dev.hasSurfaceLight;
+  need.textured = s->dev.texturedMedia != 0;
+  s->ensurePathBuffers(need);
   s->ensureTileOrder();
   const size_t slots = s->pb.capacity;
   float4* raw = (float4*)s->guideRaw.ensure(sizeof(float4) * 10 * slots);
@@ -1445,7 +1430,7 @@ int hasty_get_launch(const HastyScene* s, HastyLaunch* out) {
     g_lastError = "null argument";
     return 1;
   }
-  out->path_slots = s->slotsWanted ? s->slotsWanted : HastyScene::kDefaultSlots;
+  out->path_slots = s->slotsWanted ? s->slotsWanted : hasty::kDefaultSlots;
   out->trace_blocks = s->launch.traceBlocks;
   out->shade_blocks = s->launch.shadeBlocks;
   out->chunk = s->launch.chunk;

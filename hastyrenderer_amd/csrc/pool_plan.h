@@ -1,0 +1,44 @@
+// Sizes of a render call's path pool and results ring (host only).
+#pragma once
+#include <stdint.h>
+
+#include <algorithm>
+
+namespace hasty {
+
+constexpr uint32_t kDefaultSlots = 1u << 24;
+
+// What the jobs of a call add up to.
+struct PoolNeed {
+  uint64_t paths = 0;  // of all jobs
+  uint64_t film = 0;   // pixels of the largest job
+  bool late = false;      // some job has both a sky and emissive triangles
+  bool textured = false;  // some job has textured media
+  void add(uint32_t samples, uint64_t pixels) {
+    paths += samples * pixels;
+    film = std::max(film, pixels);
+  }
+};
+
+// Paths in flight (a path that ends makes room for the next): the wanted pool
+// (0: the default), but no more than the call needs (at least 2^16).  Larger
+// pools spread a bounce's fixed costs (the tail of its longest rays) over more
+// rays: 132 ms at 2^22, 129 at 2^23, 125 at 2^24, 122 at 2^25 for 128 samples of
+// the 1024x1024 GGX grid.
+inline uint32_t poolPaths(const PoolNeed& need, uint32_t wanted) {
+  const uint64_t most = wanted ? wanted : kDefaultSlots;
+  return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(most, std::max<uint64_t>(need.paths, 1ull << 16)));
+}
+
+// Results ring: the whole call if it is no more than about 2^27 paths
+// (finished paths wait in the ring for the oldest one in flight, so a ring
+// much longer than a pool x depth never holds a path's start up), else whole
+// samples of the largest film; never less than one, which renderJobs needs.
+inline uint32_t ringPaths(const PoolNeed& need) {
+  const uint64_t P = std::max<uint64_t>(need.film, 1), most = 1ull << 27;
+  if (need.paths <= std::max(P, most))
+    return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(need.paths, 1), 0x7FFFFFFFull);
+  return (uint32_t)std::min<uint64_t>(std::max(P, most / P * P), 0x7FFFFFFFull / P * P);
+}
+
+}  // namespace hasty

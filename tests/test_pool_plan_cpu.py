@@ -1,0 +1,37 @@
+"""Sizes of the path pool and the results ring."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from conftest import load_testkernels
+
+RING = 1 << 27
+
+
+def _sizes(jobs, wanted=0):
+    L = load_testkernels()
+    n = np.array([j[0] for j in jobs], np.uint32)
+    px = np.array([j[1] for j in jobs], np.uint64)
+    out = np.zeros(2, np.uint32)
+    L.tk_pool_sizes(n.ctypes.data_as(C.c_void_p), px.ctypes.data_as(C.c_void_p), C.c_uint32(len(jobs)),
+                    C.c_uint32(wanted), out.ctypes.data_as(C.c_void_p))
+    return int(out[0]), int(out[1])
+
+
+@pytest.mark.parametrize("first", [1, 64, 1000003, RING // 2 + 1, RING + 5])
+@pytest.mark.parametrize("other", [1, 999983, RING // 3, RING + 77, 0x7FFFFFFF])
+@pytest.mark.parametrize("samples", [1, 3, 200])
+def test_ring_holds_a_sample_of_every_job(first, other, samples):
+    """A batch that starts with a small film and holds a large one: renderJobs
+    refuses a ring smaller than one sample of any job."""
+    paths, ring = _sizes([(samples, first), (1, other)])
+    assert ring >= max(first, other)
+    total = samples * first + other
+    assert ring <= max(total, 1) and ring <= max(RING, first, other)
+    assert paths == min(1 << 24, max(total, 1 << 16))
+
+
+def test_pool_wanted_is_an_upper_limit():
+    assert _sizes([(1, 100)], wanted=7) == (7, 100)
+    assert _sizes([(64, 1 << 20)], wanted=1 << 10)[0] == 1 << 10
