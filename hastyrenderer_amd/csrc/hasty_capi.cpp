@@ -246,7 +246,12 @@ struct HastyScene {
   template <class T>
   T* allocPath(size_t count) {
     void* p = nullptr;
-    HIPCHECK(hipMalloc(&p, count * sizeof(T)));
+    const hipError_t e = hipMalloc(&p, count * sizeof(T));
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();  // this call's; the caller asks for less
+      throw hasty::OutOfMemory(std::string("hipMalloc(&p, count * sizeof(T)): ") + hipGetErrorString(e));
+    }
+    HIPCHECK(e);
     pathAllocs.push_back(p);
     return (T*)p;
   }
@@ -293,22 +298,20 @@ struct HastyScene {
     const bool fits = need <= poolCapacity && ring <= poolRing && traceThreads <= pb.traceThreads &&
                       (!late || pb.sh.lateQ) && (!textured || pb.set[0].mediaTx);
     if (!fits) {
-      uint32_t n = std::max(need, poolCapacity), r = std::max(ring, poolRing);
+      const hasty::PoolSize want{std::max(need, poolCapacity), std::max(ring, poolRing)};
       late = late || pb.sh.lateQ;
       textured = textured || pb.set[0].mediaTx;
       const uint32_t tt = std::max(traceThreads, pb.traceThreads);
-      for (;;) {
+      const hasty::PoolSize got = hasty::allocHalving(want, P, [&](hasty::PoolSize n) {
         try {
-          allocPool(n, r, tt, late, textured);
-          break;
-        } catch (const std::exception&) {
+          allocPool(n.paths, n.ring, tt, late, textured);
+        } catch (...) {
           freePath();
-          (void)hipGetLastError();  // the failed allocation's
-          if (n <= (1u << 20) && r <= std::max<uint64_t>(P, 1u << 20)) throw;
-          if (n > (1u << 20)) poolMost = n = n / 2;
-          if (r > std::max<uint64_t>(P, 1u << 20)) ringMost = r = (uint32_t)std::max<uint64_t>(P, r / 2);
+          throw;
         }
-      }
+      });
+      if (got.paths < want.paths) poolMost = got.paths;
+      if (got.ring < want.ring) ringMost = got.ring;
     }
     pb.capacity = std::min(need, poolCapacity);
     pb.ringPaths = std::min(ring, poolRing);

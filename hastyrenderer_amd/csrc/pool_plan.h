@@ -3,6 +3,8 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <stdexcept>
+#include <string>
 
 namespace hasty {
 
@@ -39,6 +41,34 @@ inline uint32_t ringPaths(const PoolNeed& need) {
   if (need.paths <= std::max(P, most))
     return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(need.paths, 1), 0x7FFFFFFFull);
   return (uint32_t)std::min<uint64_t>(std::max(P, most / P * P), 0x7FFFFFFFull / P * P);
+}
+
+struct PoolSize {
+  uint32_t paths, ring;
+};
+
+// Thrown by a device allocation that the free memory cannot serve.
+struct OutOfMemory : std::runtime_error {
+  using std::runtime_error::runtime_error;
+};
+
+// The largest of `want`, and of its halvings, that `alloc` can serve: the pool
+// down to 2^20 paths, the ring down to 2^20 entries or one sample of the largest
+// film.  Errors other than OutOfMemory are the caller's.
+template <class Alloc>
+PoolSize allocHalving(PoolSize want, uint64_t film, Alloc&& alloc) {
+  constexpr uint32_t least = 1u << 20;
+  const uint32_t leastRing = (uint32_t)std::max<uint64_t>(film, least);
+  for (;;) {
+    try {
+      alloc(want);
+      return want;
+    } catch (const OutOfMemory&) {
+      if (want.paths <= least && want.ring <= leastRing) throw;
+      if (want.paths > least) want.paths /= 2;
+      if (want.ring > leastRing) want.ring = std::max(leastRing, want.ring / 2);
+    }
+  }
 }
 
 }  // namespace hasty

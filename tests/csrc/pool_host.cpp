@@ -2,6 +2,10 @@
 // (pool_plan.h).
 #include "../../hastyrenderer_amd/csrc/pool_plan.h"
 
+namespace {
+constexpr uint64_t kPathBytes = 300, kRingBytes = 48;
+}  // namespace
+
 extern "C" {
 
 // Paths and ring entries of a call of n jobs (samples and pixels of each).
@@ -10,6 +14,29 @@ void tk_pool_sizes(const uint32_t* samples, const uint64_t* pixels, uint32_t n, 
   for (uint32_t i = 0; i < n; ++i) need.add(samples[i], pixels[i]);
   out2[0] = hasty::poolPaths(need, wanted);
   out2[1] = hasty::ringPaths(need);
+}
+
+// allocHalving on a device with `freeBytes` free, whose allocation number
+// `errorAt` (from 1; 0: none) fails with another error.  Returns 0, 1 when out
+// of memory, 2 for the other error; out: paths, ring, allocations asked for.
+int tk_alloc_halving(uint32_t paths, uint32_t ring, uint64_t film, uint64_t freeBytes, uint32_t errorAt,
+                     uint32_t* out3) {
+  uint32_t tries = 0;
+  int rc = 0;
+  out3[0] = out3[1] = 0;
+  try {
+    const hasty::PoolSize got = hasty::allocHalving({paths, ring}, film, [&](hasty::PoolSize n) {
+      if (++tries == errorAt) throw std::runtime_error("unspecified launch failure");
+      if (n.paths * kPathBytes + n.ring * kRingBytes > freeBytes) throw hasty::OutOfMemory("out of memory");
+    });
+    out3[0] = got.paths, out3[1] = got.ring;
+  } catch (const hasty::OutOfMemory&) {
+    rc = 1;
+  } catch (const std::exception&) {
+    rc = 2;
+  }
+  out3[2] = tries;
+  return rc;
 }
 
 }  // extern "C"

@@ -35,3 +35,29 @@ def test_ring_holds_a_sample_of_every_job(first, other, samples):
 def test_pool_wanted_is_an_upper_limit():
     assert _sizes([(1, 100)], wanted=7) == (7, 100)
     assert _sizes([(64, 1 << 20)], wanted=1 << 10)[0] == 1 << 10
+
+
+def _halving(paths, ring, film, free, error_at=0):
+    L = load_testkernels()
+    out = np.zeros(3, np.uint32)
+    rc = L.tk_alloc_halving(C.c_uint32(paths), C.c_uint32(ring), C.c_uint64(film), C.c_uint64(free),
+                            C.c_uint32(error_at), out.ctypes.data_as(C.c_void_p))
+    return rc, tuple(int(x) for x in out)
+
+
+def test_pool_is_halved_until_it_fits():
+    M = 1 << 20
+    assert _halving(16 * M, 128 * M, 5 * M, 1 << 40) == (0, (16 * M, 128 * M, 1))
+    assert _halving(16 * M, 128 * M, 5 * M, 300 * 4 * M + 48 * 32 * M) == (0, (4 * M, 32 * M, 3))
+    # not below 2^20 paths and one sample of the largest film
+    assert _halving(16 * M, 128 * M, 5 * M, 300 * M + 48 * 5 * M) == (0, (M, 5 * M, 6))
+    assert _halving(16 * M, 128 * M, 5 * M, 300 * M + 48 * 5 * M - 1) == (1, (0, 0, 6))
+    assert _halving(100, 7, 7, 1000) == (1, (0, 0, 1))
+
+
+@pytest.mark.parametrize("error_at", [1, 2, 3])
+def test_other_errors_are_not_a_shortage(error_at):
+    """A lost device or a failed launch is reported, not answered by asking
+    for less."""
+    M = 1 << 20
+    assert _halving(16 * M, 128 * M, M, 300 * M + 48 * M, error_at) == (2, (0, 0, error_at))
