@@ -186,8 +186,7 @@ struct HastyScene {
   // path buffers
   hasty::PathBuffers pb{};
   std::vector<void*> pathAllocs;
-  uint32_t poolCapacity = 0, poolRing = 0;  // allocated paths and ring entries
-  uint32_t poolMost = 0xFFFFFFFFu, ringMost = 0xFFFFFFFFu;  // what an allocation failed above
+  hasty::PoolFit pool;
   uint32_t slotsWanted = 0;  // 0 = automatic
   uint32_t* dTileOrder = nullptr;
   uint32_t tileW = 0, tileH = 0;
@@ -259,7 +258,6 @@ struct HastyScene {
     for (void* p : pathAllocs) (void)hipFree(p);
     pathAllocs.clear();
     pb = hasty::PathBuffers{};
-    poolCapacity = poolRing = 0;
   }
   ~HastyScene() {
     if (timer) timer->collect();
@@ -290,31 +288,27 @@ struct HastyScene {
   // that needs less uses a part).  A pool or ring that does not fit the free
   // memory is halved until it does.
   void ensurePathBuffers(const hasty::PoolNeed& call) {
-    bool late = call.late, textured = call.textured;
-    const uint64_t P = call.film;
-    const uint32_t need = std::min(hasty::poolPaths(call, slotsWanted), poolMost);
-    const uint32_t ring = (uint32_t)std::min<uint64_t>(hasty::ringPaths(call), std::max<uint64_t>(ringMost, P));
-    const uint32_t traceThreads = launch.traceBlocks * hasty::kBlock;
-    const bool fits = need <= poolCapacity && ring <= poolRing && traceThreads <= pb.traceThreads &&
-                      (!late || pb.sh.lateQ) && (!textured || pb.set[0].mediaTx);
-    if (!fits) {
-      const hasty::PoolSize want{std::max(need, poolCapacity), std::max(ring, poolRing)};
-      late = late || pb.sh.lateQ;
-      textured = textured || pb.set[0].mediaTx;
-      const uint32_t tt = std::max(traceThreads, pb.traceThreads);
-      const hasty::PoolSize got = hasty::allocHalving(want, P, [&](hasty::PoolSize n) {
-        try {
-          allocPool(n.paths, n.ring, tt, late, textured);
-        } catch (...) {
-          freePath();
-          throw;
-        }
-      });
-      if (got.paths < want.paths) poolMost = got.paths;
-      if (got.ring < want.ring) ringMost = got.ring;
-    }
-    pb.capacity = std::min(need, poolCapacity);
-    pb.ringPaths = std::min(ring, poolRing);
+    const hasty::PoolSize want{hasty::poolPaths(call, slotsWanted), hasty::ringPaths(call)};
+    const uint32_t traceThreads = std::max(launch.traceBlocks * hasty::kBlock, pb.traceThreads);
+    const bool late = call.late || pb.sh.lateQ, textured = call.textured || pb.set[0].mediaTx;
+    const bool regrow = traceThreads > pb.traceThreads || (late && !pb.sh.lateQ) || (textured && !pb.set[0].mediaTx);
+    pool.fit(
+        want, call.film, regrow, [&](hasty::PoolSize n) { return hasty::poolBytes(n, late, textured); },
+        [] {
+          size_t free = 0, total = 0;
+          HIPCHECK(hipMemGetInfo(&free, &total));
+          return (uint64_t)free;
+        },
+        [&](hasty::PoolSize n) {
+          try {
+            allocPool(n.paths, n.ring, traceThreads, late, textured);
+          } catch (...) {
+            freePath();
+            throw;
+          }
+        });
+    pb.capacity = std::min(want.paths, pool.have.paths);
+    pb.ringPaths = std::min(want.ring, pool.have.ring);
   }
   void allocPool(uint32_t n, uint32_t r, uint32_t traceThreads, bool late, bool textured) {
     freePath();
@@ -346,8 +340,6 @@ struct HastyScene {
     pb.ringA = allocPath<float4>(r);
     pb.traceThreads = traceThreads;
     HIPCHECK(hipMemset(pb.stats, 0, sizeof(unsigned long long) * hasty::kNumStats));
-    poolCapacity = n;
-    poolRing = r;
   }
 
   void ensureTileOrder() {

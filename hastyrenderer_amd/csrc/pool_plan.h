@@ -46,6 +46,12 @@ inline uint32_t ringPaths(const PoolNeed& need) {
 struct PoolSize {
   uint32_t paths, ring;
 };
+// Device memory of a pool (the traversal's overflow slices aside): two sets of
+// path records (112 B, and 32 B of media texels), hits, shadow rays (60 B, and
+// 104 B where they may be late), and 48 B a ring entry.
+inline uint64_t poolBytes(PoolSize n, bool late, bool textured) {
+  return (uint64_t)n.paths * (2 * (112 + (textured ? 32 : 0)) + 16 + 60 + (late ? 104 : 0)) + (uint64_t)n.ring * 48;
+}
 
 // Thrown by a device allocation that the free memory cannot serve.
 struct OutOfMemory : std::runtime_error {
@@ -70,5 +76,35 @@ PoolSize allocHalving(PoolSize want, uint64_t film, Alloc&& alloc) {
     }
   }
 }
+
+// The pool a scene holds, kept from call to call and grown when a call needs
+// more.  After a shortage the smaller pool stays in use, and the wanted size is
+// tried again once the memory for it is there; until then a call that wants more
+// than the pool asks for the free memory and allocates nothing.
+class PoolFit {
+ public:
+  PoolSize have{0, 0};
+  // Makes `have` at least `want`, or what memory allows.  regrow: the buffers
+  // have to be allocated again whatever their size.  bytes(size): memory of a
+  // pool; freeBytes(): the device's free memory; alloc as for allocHalving,
+  // giving back the former pool first.
+  template <class Bytes, class Free, class Alloc>
+  void fit(PoolSize want, uint64_t film, bool regrow, Bytes&& bytes, Free&& freeBytes, Alloc&& alloc) {
+    if (!regrow && want.paths <= have.paths && want.ring <= have.ring) return;
+    want.paths = std::max(want.paths, have.paths), want.ring = std::max(want.ring, have.ring);
+    if (!regrow && shortAt_ && have.ring >= std::min<uint64_t>(film, want.ring)) {
+      const uint64_t room = freeBytes() + bytes(have);
+      if (room < bytes(want) || room <= shortAt_) return;
+    }
+    have = PoolSize{0, 0};
+    shortAt_ = 0;
+    const PoolSize got = allocHalving(want, film, alloc);
+    if (got.paths < want.paths || got.ring < want.ring) shortAt_ = freeBytes() + bytes(got);
+    have = got;
+  }
+
+ private:
+  uint64_t shortAt_ = 0;  // memory for a pool when one last came out smaller (0: none did)
+};
 
 }  // namespace hasty

@@ -39,4 +39,29 @@ int tk_alloc_halving(uint32_t paths, uint32_t ring, uint64_t film, uint64_t free
   return rc;
 }
 
+// A scene's pool over n calls on a device of which call k leaves freeBytes[k] to
+// the pool: paths and ring held after each, and allocations asked for in it (0
+// paths: the call was refused).
+void tk_pool_fit(const uint32_t* paths, const uint32_t* ring, const uint64_t* film, const uint64_t* freeBytes,
+                 const uint32_t* regrow, uint32_t n, uint32_t* out3) {
+  hasty::PoolFit pool;
+  auto bytes = [](hasty::PoolSize s) { return hasty::poolBytes(s, false, false); };
+  for (uint32_t k = 0; k < n; ++k) {
+    uint32_t tries = 0;
+    uint64_t held = bytes(pool.have);
+    try {
+      pool.fit({paths[k], ring[k]}, film[k], regrow[k] != 0, bytes,
+               [&] { return freeBytes[k] - std::min(freeBytes[k], held); },
+               [&](hasty::PoolSize s) {
+                 ++tries;
+                 held = 0;
+                 if (bytes(s) > freeBytes[k]) throw hasty::OutOfMemory("out of memory");
+                 held = bytes(s);
+               });
+    } catch (const hasty::OutOfMemory&) {
+    }
+    out3[3 * k] = pool.have.paths, out3[3 * k + 1] = pool.have.ring, out3[3 * k + 2] = tries;
+  }
+}
+
 }  // extern "C"

@@ -61,3 +61,47 @@ def test_other_errors_are_not_a_shortage(error_at):
     for less."""
     M = 1 << 20
     assert _halving(16 * M, 128 * M, M, 300 * M + 48 * M, error_at) == (2, (0, 0, error_at))
+
+
+def _fit(calls):
+    """calls: (paths, ring, film, bytes left to the pool, regrow)."""
+    L = load_testkernels()
+    cols = [np.array([c[k] for c in calls], t) for k, t in enumerate((np.uint32, np.uint32, np.uint64, np.uint64,
+                                                                      np.uint32))]
+    out = np.zeros((len(calls), 3), np.uint32)
+    L.tk_pool_fit(*(a.ctypes.data_as(C.c_void_p) for a in cols), C.c_uint32(len(calls)),
+                  out.ctypes.data_as(C.c_void_p))
+    return [tuple(int(x) for x in r) for r in out]
+
+
+def test_a_passing_shortage_passes():
+    M, G = 1 << 20, 1 << 30
+    whole = (16 * M, 128 * M, M)
+    # short, still short, a little more free, enough again, then kept
+    got = _fit([whole + (4 * G, 0), whole + (4 * G, 0), whole + (5 * G, 0), whole + (20 * G, 0), whole + (4 * G, 0)])
+    assert got[0] == (4 * M, 32 * M, 3)
+    assert got[1] == got[2] == (4 * M, 32 * M, 0)
+    assert got[3] == (16 * M, 128 * M, 1)
+    assert got[4] == (16 * M, 128 * M, 0)
+
+
+def test_pool_grows_and_is_kept():
+    M, G = 1 << 20, 1 << 30
+    got = _fit([(M, M, 100, 100 * G, 0), (M // 2, M, 100, 100 * G, 0), (2 * M, M // 2, 100, 100 * G, 0),
+                (M, M, 100, 100 * G, 1)])
+    assert got == [(M, M, 1), (M, M, 0), (2 * M, M, 1), (2 * M, M, 1)]
+
+
+def test_short_pool_still_serves_what_it_must():
+    """A larger film than the short ring holds, and buffers of another kind,
+    are allocated again whatever is free; a call that cannot be served at all
+    leaves no pool behind, and the next one starts afresh."""
+    M, G = 1 << 20, 1 << 30
+    whole = (16 * M, 128 * M, M)
+    got = _fit([whole + (4 * G, 0), (16 * M, 128 * M, 40 * M, 4 * G, 0), whole + (4 * G, 1), whole + (M, 1),
+                whole + (20 * G, 0)])
+    assert got[0] == (4 * M, 32 * M, 3)
+    assert got[1] == (4 * M, 40 * M, 3)
+    assert got[2] == (4 * M, 32 * M, 3)
+    assert got[3][:2] == (0, 0)
+    assert got[4] == (16 * M, 128 * M, 1)
