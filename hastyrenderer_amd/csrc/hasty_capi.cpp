@@ -218,7 +218,7 @@ struct HastyScene {
   uint32_t lastGuidePhotonSamples = 0;
   DevBuf guideRaw;    // mixture tables of the paths alive
   DevBuf guideSel;    // their learned selection probabilities
-  DevBuf guideRec;    // training records by path of a call
+  DevBuf guideRec;    // training records of the paths from the oldest in flight on
   DevBuf guideEnded;  // paths that ended at a bounce with records
   float4* guideSamples = nullptr;
   uint32_t* guideCount = nullptr;
@@ -557,7 +557,8 @@ static void renderGuided(HastyScene* s, const BatchItem& it) {
   const size_t slots = s->pb.capacity;
   float4* raw = (float4*)s->guideRaw.ensure(sizeof(float4) * 10 * slots);
   float* sel = s->guide->g->learnedSelection() ? (float*)s->guideSel.ensure(sizeof(float) * slots) : nullptr;
-  float4* rec = training ? (float4*)s->guideRec.ensure(sizeof(float4) * 12 * (size_t)perCall * P) : nullptr;
+  const uint32_t recPaths = hasty::recordPaths(need, s->slotsWanted);
+  float4* rec = training ? (float4*)s->guideRec.ensure(sizeof(float4) * 12 * (size_t)recPaths) : nullptr;
   s->pb.ended = training ? (uint2*)s->guideEnded.ensure(sizeof(uint2) * slots) : nullptr;
   if (!s->guideSamples) {
     HIPCHECK(hipMalloc(&s->guideSamples, sizeof(float4) * 4 * (size_t)HastyScene::kGuideSampleCap));
@@ -567,6 +568,7 @@ static void renderGuided(HastyScene* s, const BatchItem& it) {
   gr.net = s->guide->g->net();
   gr.raw = raw;
   gr.rec = rec;
+  gr.recPaths = recPaths;
   gr.samples = s->guideSamples;
   gr.sampleCount = s->guideCount;
   gr.sampleCap = training ? HastyScene::kGuideSampleCap : 0u;

@@ -43,6 +43,14 @@ inline uint32_t ringPaths(const PoolNeed& need) {
   return (uint32_t)std::min<uint64_t>(std::max(P, most / P * P), 0x7FFFFFFFull / P * P);
 }
 
+// Paths with room for the guide's training records (192 B each): those of the
+// call, but for a film of more than four pools only that many from the oldest
+// in flight on (a call trains on about 2^20 paths, or one sample of the film).
+inline uint32_t recordPaths(const PoolNeed& need, uint32_t wanted) {
+  const uint64_t most = std::max<uint64_t>(4ull * (wanted ? wanted : kDefaultSlots), 1ull << 20);
+  return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(need.paths, most));
+}
+
 struct PoolSize {
   uint32_t paths, ring;
 };

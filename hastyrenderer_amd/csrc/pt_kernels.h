@@ -99,7 +99,7 @@ struct PassInfo {
 };
 
 // Guided rendering (single job): guide outputs of the paths alive, training
-// records by path id (2 x {position, normal, wo + the density wi was drawn
+// records by path id modulo recPaths (2 x {position, normal, wo + the density wi was drawn
 // with, wi + the BSDF density of wi, throughput before the sample, radiance
 // before the continuation}) and the training samples harvested when paths
 // end (4 float4 each: position + weight, normal, wo + drawing density,
@@ -107,7 +107,8 @@ struct PassInfo {
 struct GuideRun {
   guide::Net net;
   float4* raw;      // 10 float4 per path alive
-  float4* rec;      // 12 float4 per path of the call (training)
+  float4* rec;      // 12 float4 for each of recPaths paths (training)
+  uint32_t recPaths;  // paths from the oldest in flight on that may have records
   float4* samples;  // sampleCap x 4 float4
   uint32_t* sampleCount;
   uint32_t sampleCap;

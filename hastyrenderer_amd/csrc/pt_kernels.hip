@@ -467,7 +467,7 @@ __device__ inline void shadeVertex(const DevScene& s, const PassInfo& pi, const 
   uint32_t nrec = GUIDED ? (flags >> kRecShift) & 3u : 0u;
   if (GUIDED && depth > 0 && nrec > 0 && ((flags >> (kRecShift + 2)) & 1u)) {
     // radiance before the continuation of the last recorded vertex
-    g.rec[(size_t)pt.pid * 12 + 6 * (nrec - 1) + 5] = f4(L, 0.0f);
+    g.rec[(size_t)(pt.pid % g.recPaths) * 12 + 6 * (nrec - 1) + 5] = f4(L, 0.0f);
   }
   hrng::Stream rng;
   {
@@ -665,7 +665,7 @@ __device__ inline void shadeVertex(const DevScene& s, const PassInfo& pi, const 
   uint32_t recBits = 0u;
   if (GUIDED) {
     if (guided && nrec < 2u && g.sampleCap > 0u) {  // records only when training
-      float4* rr = g.rec + (size_t)pt.pid * 12 + 6 * nrec;
+      float4* rr = g.rec + (size_t)(pt.pid % g.recPaths) * 12 + 6 * nrec;
       V3 nf = dot(it.ng, wo) >= 0.0f ? it.ng : -it.ng;
       rr[0] = f4(it.x, 0.0f);
       rr[1] = f4(nf, 0.0f);
@@ -859,7 +859,7 @@ __global__ void __launch_bounds__(kBlock) kHarvest(GuideRun g, PathBuffers pb, u
     const uint2 e = pb.ended[q];
     const float4 Lf = pb.ringL[e.x % pb.ringPaths];
     for (uint32_t r = 0; r < e.y; ++r) {
-      const float4* rr = g.rec + (size_t)e.x * 12 + 6 * r;
+      const float4* rr = g.rec + (size_t)(e.x % g.recPaths) * 12 + 6 * r;
       float4 b = rr[4], ls = rr[5];
       float cx = b.x > 0.0f ? (Lf.x - ls.x) / b.x : 0.0f;
       float cy = b.y > 0.0f ? (Lf.y - ls.y) / b.y : 0.0f;
@@ -1308,7 +1308,14 @@ void renderJobs(const std::vector<RenderJobDesc>& jobs, const PathBuffers& pb, c
   auto accPid = [&]() -> uint64_t {
     return front < nJobs ? (uint64_t)passes[front].pidBase + (uint64_t)acc[front] * passes[front].pixels : total;
   };
-  uint32_t limit = (uint32_t)std::min<uint64_t>(total, accPid() + pb.ringPaths);
+  // Paths that may have started when all below `done` have finished: those with
+  // a place in the ring, and (training) one for their records.
+  auto startLimit = [&](uint64_t done) {
+    uint64_t most = std::min<uint64_t>(total, accPid() + pb.ringPaths);
+    if (guide && guide->sampleCap > 0u) most = std::min<uint64_t>(most, done + guide->recPaths);
+    return (uint32_t)most;
+  };
+  uint32_t limit = startLimit(0);
   t0(kKMisc);
   kInitRender<<<1, 64, 0, stream>>>(pb.counters, limit);
   t1(kKMisc);
@@ -1370,7 +1377,7 @@ void renderJobs(const std::vector<RenderJobDesc>& jobs, const PathBuffers& pb, c
       }
     }
     while (front < nJobs && acc[front] * (uint64_t)passes[front].pixels == passes[front].paths) ++front;
-    uint32_t newLimit = (uint32_t)std::min<uint64_t>(total, accPid() + pb.ringPaths);
+    const uint32_t newLimit = startLimit(done);
     if (newLimit != limit) {
       t0(kKMisc);
       kSetLimit<<<1, 64, 0, stream>>>(pb.counters, newLimit);

@@ -8,12 +8,14 @@ constexpr uint64_t kPathBytes = 300, kRingBytes = 48;
 
 extern "C" {
 
-// Paths and ring entries of a call of n jobs (samples and pixels of each).
-void tk_pool_sizes(const uint32_t* samples, const uint64_t* pixels, uint32_t n, uint32_t wanted, uint32_t* out2) {
+// Paths, ring entries and paths with training records of a call of n jobs
+// (samples and pixels of each).
+void tk_pool_sizes(const uint32_t* samples, const uint64_t* pixels, uint32_t n, uint32_t wanted, uint32_t* out3) {
   hasty::PoolNeed need;
   for (uint32_t i = 0; i < n; ++i) need.add(samples[i], pixels[i]);
-  out2[0] = hasty::poolPaths(need, wanted);
-  out2[1] = hasty::ringPaths(need);
+  out3[0] = hasty::poolPaths(need, wanted);
+  out3[1] = hasty::ringPaths(need);
+  out3[2] = hasty::recordPaths(need, wanted);
 }
 
 // allocHalving on a device with `freeBytes` free, whose allocation number

@@ -191,3 +191,28 @@ def test_photon_trained_guide_unbiased_and_gains(ring_job, ring_reference, selec
     print("trimmed relMSE at %d spp: plain %.5f, guided %.5f, guided without photons %.5f" % (
         batches * spp, pe, ge, ne), flush=True)
     assert ge < 0.8 * pe and ge < ne
+
+
+def test_training_records_in_a_window(tmp_path):
+    """A film with more pixels than there are training records (2^20 with a
+    pool this small): paths take the places of the oldest that have finished, and
+    the samples harvested and the film are those of records for every path.
+    One minibatch holds all samples, so that the loss does not depend on the
+    order in which they arrived but for its FP32 sum over some 2^14 partial
+    sums (2^14 u = 1e-3 at most)."""
+    job = scenes.write_cornell(str(tmp_path / "w"), width=1250, height=1000, spp=1, max_depth=4)
+    got = []
+    for slots in (0, 1 << 15):
+        sc = ha.Scene(job)
+        if slots:
+            sc.set_launch(path_slots=slots)
+        g = ha.Guide(sc, seed=0)
+        sc.set_guide_training(minibatch=1 << 21)
+        sc.set_guide(g, fraction=0.5, train_lr=1e-3)
+        films = sc.render_pt(seed=3, first_sample=0, num_samples=1)
+        got.append((sc.guide_stats(), films))
+    (loss, n), films = got[1]
+    assert 0 < n < 1 << 21 and n == got[0][0][1]
+    assert abs(loss - got[0][0][0]) <= 1e-3 * abs(loss)
+    for a, b in zip(films, got[0][1]):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))

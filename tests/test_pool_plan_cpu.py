@@ -13,10 +13,10 @@ def _sizes(jobs, wanted=0):
     L = load_testkernels()
     n = np.array([j[0] for j in jobs], np.uint32)
     px = np.array([j[1] for j in jobs], np.uint64)
-    out = np.zeros(2, np.uint32)
+    out = np.zeros(3, np.uint32)
     L.tk_pool_sizes(n.ctypes.data_as(C.c_void_p), px.ctypes.data_as(C.c_void_p), C.c_uint32(len(jobs)),
                     C.c_uint32(wanted), out.ctypes.data_as(C.c_void_p))
-    return int(out[0]), int(out[1])
+    return tuple(int(x) for x in out)
 
 
 @pytest.mark.parametrize("first", [1, 64, 1000003, RING // 2 + 1, RING + 5])
@@ -25,7 +25,7 @@ def _sizes(jobs, wanted=0):
 def test_ring_holds_a_sample_of_every_job(first, other, samples):
     """A batch that starts with a small film and holds a large one: renderJobs
     refuses a ring smaller than one sample of any job."""
-    paths, ring = _sizes([(samples, first), (1, other)])
+    paths, ring, _ = _sizes([(samples, first), (1, other)])
     assert ring >= max(first, other)
     total = samples * first + other
     assert ring <= max(total, 1) and ring <= max(RING, first, other)
@@ -33,8 +33,20 @@ def test_ring_holds_a_sample_of_every_job(first, other, samples):
 
 
 def test_pool_wanted_is_an_upper_limit():
-    assert _sizes([(1, 100)], wanted=7) == (7, 100)
+    assert _sizes([(1, 100)], wanted=7)[:2] == (7, 100)
     assert _sizes([(64, 1 << 20)], wanted=1 << 10)[0] == 1 << 10
+
+
+def test_training_records_are_bounded():
+    """192 B each: a call trains on 2^20 paths or one sample of the film, and a
+    film of 2^30 pixels must not take 200 GB for them."""
+    M = 1 << 20
+    assert _sizes([(7, 150000)])[2] == 1050000
+    assert _sizes([(1, 64 * M)])[2] == 64 * M
+    assert _sizes([(1, 1024 * M)])[2] == 64 * M
+    assert _sizes([(1, 8 * M)], wanted=M)[2] == 4 * M
+    assert _sizes([(1, 8 * M)], wanted=7)[2] == M
+    assert _sizes([(1, 5)], wanted=7)[2] == 5
 
 
 def _halving(paths, ring, film, free, error_at=0):
