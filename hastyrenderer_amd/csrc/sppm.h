@@ -81,7 +81,7 @@ class SppmRenderer {
   float4* dQuery_ = nullptr;
   uint32_t* dNq_ = nullptr;
   float4* dCamera_ = nullptr;   // two sets of camera paths between segments
-  uint32_t* dTasks_ = nullptr;  // gather tasks of many candidates
+  uint32_t* dHeavy_ = nullptr;  // gather queries of many candidates
   float* dLpath_ = nullptr;
   // cell size reductions
   float* dPartial_ = nullptr;

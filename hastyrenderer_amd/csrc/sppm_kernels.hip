@@ -120,7 +120,7 @@ enum Counter {
   kCtrFluxOverflow = 4,  // gathers whose fixed-point flux sum saturated
   kCtrSelected = 5,      // photons of the batch that meet a caster's box
   kCtrTraced = 6,        // the last batch's
-  kCtrShared = 7,        // gather tasks left to kSppmGatherShared
+  kCtrShared = 7,        // queries left to kSppmGatherShared
   kNumCtr = 8            // then the paths alive at the end of each camera segment
 };
 // Vertices at which the camera paths are packed anew (see kSppmCamera).
@@ -696,6 +696,13 @@ __device__ inline void photonRun(const SppmDev& g, uint32_t first, uint32_t end,
 // with 32, 64, 128, 256, 512: 4.94, 4.89, 4.83, 4.84, 4.81 ms (sparse map,
 // 960x540) and 9.68, 9.69, 9.69, 9.97, 10.99 ms (dense map, 640x360).
 constexpr uint32_t kCoopCandidatesDefault = 128;
+// Where a query of the wave is over that limit, those over a third of it are left
+// as well: few lanes would walk their lists while the others, whose queries are
+// left, idle.  Passes 2-6, 7-12, 13-24, 25-48 of the dense map with the limit
+// itself, 1/2, 1/3, 1/4, 1/8 of it and every query left: 10.20 9.28 8.68 7.60; 9.52
+// 8.79 8.34 7.49; 9.58 8.60 8.28 7.55; 9.58 8.56 8.24 7.61; 9.61 8.65 8.24 7.80; 9.58
+// 8.72 8.33 7.92 ms; of the sparse map (13-24) 4.02, 4.05, 4.06, 4.08, 4.09, 4.12.
+constexpr uint32_t kMixedShare = 3;
 // Union gather: the wave visits the cells of the union of its queries'
 // boxes in x -> y -> z order, stages each run of photon positions in LDS 64
 // at a time, and every lane tests them against its own query.  A photon
@@ -782,8 +789,9 @@ __device__ inline void queryCells(const SppmDev& g, V3 x, float r, float cs, int
 // cells it keeps for the gather (more: they are looked up again).
 constexpr int kCellLoads = 4, kOwnRuns = 8;
 // The gathers of a wave's queries, a lane each in the reference's order (or
-// the union gather); false, with nothing gathered, if some query has so many
-// candidates that all of them are left to sharedGather.
+// the union gather); false, with nothing gathered, on the lanes whose query has
+// so many candidates that it is left to sharedGather.  A lane over the limit looks
+// up no further cells (unless the union gather's choice needs all boxes).
 template <class Sum>
 __device__ inline bool ownGather(const SppmDev& g, const DevScene& s, bool has, V3 x, V3 ns, V3 ng, int mat, float r,
                                  int* M, uint2* runs, float4* staged, uint2* ownRuns, uint32_t* candidates,
@@ -796,7 +804,7 @@ __device__ inline bool ownGather(const SppmDev& g, const DevScene& s, bool has, 
     queryCells(g, x, r, cs, &lo, &hi);
     int3 c = lo;
     bool more = lo.x <= hi.x && lo.y <= hi.y && lo.z <= hi.z;
-    while (more) {
+    while (more && (cand <= g.coopCandidates || g.unionFactor > 0.0f)) {
       unsigned long long key[kCellLoads];
       uint32_t h[kCellLoads];
       uint4 e[kCellLoads];
@@ -828,33 +836,11 @@ __device__ inline bool ownGather(const SppmDev& g, const DevScene& s, bool has, 
     }
   }
   *candidates = cand;
-  if (__ballot(cand > g.coopCandidates) == 0ull) {
-    Sum est;
-    int found = 0;
-    if (has) {
-      const DevMaterial m = ldgStruct(s.mats + mat);
-      if (nRuns <= kOwnRuns) {
-        for (int k = 0; k < nRuns; ++k) {
-          const uint2 cell = ownRuns[k * kB];
-          photonRun(g, cell.x, cell.x + cell.y, x, r * r, ns, ng, m, &est, &found);
-        }
-      } else {
-        for (int i = lo.x; i <= hi.x; ++i)
-          for (int j = lo.y; j <= hi.y; ++j)
-            for (int k = lo.z; k <= hi.z; ++k) {
-              const uint2 cell = cellLookup(g, packKey(make_int3(i, j, k)));
-              photonRun(g, cell.x, cell.x + cell.y, x, r * r, ns, ng, m, &est, &found);
-            }
-      }
-      if (est.saturated()) atomicAdd(&g.counters[kCtrFluxOverflow], 1u);
-    }
-    *M = found;
-    *result = est.value(g);
-    return true;
-  }
+  const bool anyHeavy = __ballot(cand > g.coopCandidates) != 0ull;
+  const bool heavy = cand > (anyHeavy ? g.coopCandidates / kMixedShare : g.coopCandidates);
   // many candidates: the union gather when the queries' boxes overlap
   // enough (the union box holds at most unionFactor x their mean cells)
-  if (g.unionFactor > 0.0f) {
+  if (g.unionFactor > 0.0f && anyHeavy) {
     int3 ulo = make_int3(has ? lo.x : 0x7FFFFFFF, has ? lo.y : 0x7FFFFFFF, has ? lo.z : 0x7FFFFFFF);
     int3 uhi = make_int3(has ? hi.x : -0x7FFFFFFF, has ? hi.y : -0x7FFFFFFF, has ? hi.z : -0x7FFFFFFF);
     float own = has ? (float)max(hi.x - lo.x + 1, 0) * (float)max(hi.y - lo.y + 1, 0) *
@@ -880,7 +866,28 @@ __device__ inline bool ownGather(const SppmDev& g, const DevScene& s, bool has, 
       return true;
     }
   }
-  return false;
+  Sum est;
+  int found = 0;
+  if (has && !heavy) {
+    const DevMaterial m = ldgStruct(s.mats + mat);
+    if (nRuns <= kOwnRuns) {
+      for (int k = 0; k < nRuns; ++k) {
+        const uint2 cell = ownRuns[k * kB];
+        photonRun(g, cell.x, cell.x + cell.y, x, r * r, ns, ng, m, &est, &found);
+      }
+    } else {
+      for (int i = lo.x; i <= hi.x; ++i)
+        for (int j = lo.y; j <= hi.y; ++j)
+          for (int k = lo.z; k <= hi.z; ++k) {
+            const uint2 cell = cellLookup(g, packKey(make_int3(i, j, k)));
+            photonRun(g, cell.x, cell.x + cell.y, x, r * r, ns, ng, m, &est, &found);
+          }
+    }
+    if (est.saturated()) atomicAdd(&g.counters[kCtrFluxOverflow], 1u);
+  }
+  *M = found;
+  *result = est.value(g);
+  return !heavy;
 }
 
 // One query (the same on every lane), by the 64 lanes of the wave: they test
@@ -889,7 +896,7 @@ __device__ inline bool ownGather(const SppmDev& g, const DevScene& s, bool has, 
 // Every lane of the wave takes part and gets the result.
 template <class Sum>
 __device__ inline V3 sharedGather(const SppmDev& g, const DevScene& s, V3 c, V3 ns, V3 ng, int mat, float rr, int* M,
-                                  uint2* runs, uint32_t* fq, bool* saturated) {
+                                  uint2* runs, uint32_t* fq, bool* saturated, uint32_t* candidates) {
   const uint32_t lane = __lane_id();
   const int rank = (int)lane, nAct = 64;
   const unsigned long long ltMask = (1ull << lane) - 1ull;
@@ -900,6 +907,7 @@ __device__ inline V3 sharedGather(const SppmDev& g, const DevScene& s, V3 c, V3 
   Sum acc;
   int found = 0;
   uint32_t head = 0u, tail = 0u;  // the queue fq[head .. tail) (mod 128) of photons found
+  uint32_t cand = 0u;
   // the cells of the box in x -> y -> z order, 64 at a time: lane rank
   // looks up cell base + rank (all probes in flight together).  Their
   // photons are then dealt to the lanes as one sequence (cell after cell),
@@ -920,6 +928,7 @@ __device__ inline V3 sharedGather(const SppmDev& g, const DevScene& s, V3 c, V3 
       if (rank >= off) incl += t;
     }
     const uint32_t total = __shfl(incl, 63);
+    cand += total;
     // sequence index i of this cell's photons maps to photon i + .x
     // (unsigned arithmetic wraps); .y is where the cell ends
     runs[rank] = make_uint2(run.x - (incl - run.y), incl);
@@ -970,6 +979,7 @@ __device__ inline V3 sharedGather(const SppmDev& g, const DevScene& s, V3 c, V3 
   for (int off = 32; off > 0; off >>= 1) found += __shfl_xor(found, off);
   *M = found;
   *saturated = acc.saturated();
+  *candidates = cand;
   return acc.value(g);
 }
 
@@ -1283,14 +1293,14 @@ __device__ inline float pixelRadius(const SppmDev& g, uint32_t p) {
 // PhotonMapping.cpp:271-296, at each diffuse vertex of
 // pathTraceWithCausticsMap): task (v, k) is the v-th queries of the 64 pixels
 // from 64 k on, a wave each.  A gather's estimate and count of photons replace
-// the position and material in its query record.  Tasks with a query of many
-// candidates are listed for kSppmGatherShared.
+// the position and material in its query record.  Queries of many candidates
+// are listed for kSppmGatherShared.
 // One wave used to run all the rounds v of its pixels one after another and
 // shared gathers within, so a launch lasted as long as its heaviest 64 pixels:
 // 9.7 ms for the dense map's 833,000 queries and 273M candidates in the fifth
 // pass, 5.4 ms in tasks.  Bound by the latency of cell probes and photon loads.
 template <class Sum>
-__global__ void __launch_bounds__(kB) HASTY_SPPM_GATHER_ATTR kSppmGather(DevScene s, SppmDev g, uint32_t* tasks) {
+__global__ void __launch_bounds__(kB) HASTY_SPPM_GATHER_ATTR kSppmGather(DevScene s, SppmDev g, uint32_t* heavy) {
   __shared__ uint2 gatherRuns[kB];
   __shared__ float4 gatherStaged[kB];
   __shared__ uint2 gatherOwn[kOwnRuns * kB];
@@ -1314,15 +1324,19 @@ __global__ void __launch_bounds__(kB) HASTY_SPPM_GATHER_ATTR kSppmGather(DevScen
     const bool done = ownGather<Sum>(g, s, has, f4xyz(q0), f4xyz(q1), f4xyz(q2), __float_as_int(q0.w), radius, &M,
                                      gatherRuns + (threadIdx.x & ~63u), gatherStaged + (threadIdx.x & ~63u),
                                      gatherOwn + threadIdx.x, &cand, &est);
-    if (has) {
-      nQueries += 1;
+    if (has) nQueries += 1;
+    if (has && done) {
       nCand += cand;
-      if (done) {
-        nFound += (unsigned long long)M;
-        qr[0] = f4(est, __int_as_float(M));
-      }
+      nFound += (unsigned long long)M;
+      qr[0] = f4(est, __int_as_float(M));
     }
-    if (!done && lane == 0) tasks[atomicAdd(&g.counters[kCtrShared], 1u)] = t;
+    const unsigned long long left = __ballot(has && !done);
+    if (left != 0ull) {
+      uint32_t at = 0;
+      if (lane == 0) at = atomicAdd(&g.counters[kCtrShared], (uint32_t)__popcll(left));
+      at = __shfl(at, 0) + (uint32_t)__popcll(left & ((1ull << lane) - 1ull));
+      if (has && !done) heavy[at] = v * P + p;
+    }
   }
   // one atomic per wave and statistic
   for (int off = 32; off > 0; off >>= 1) {
@@ -1337,39 +1351,43 @@ __global__ void __launch_bounds__(kB) HASTY_SPPM_GATHER_ATTR kSppmGather(DevScen
   }
 }
 
-// The listed tasks, kShareQueries queries to a wave: small pieces, since a
-// query of a caustic has thousands of candidates and one beside it none (1, 2,
-// 4, 8, 16: 10.67, 10.74, 10.85, 11.20, 11.42 ms a pass of the dense map).
-constexpr uint32_t kShareQueries = 1;
+// The listed queries, one to a wave.  Bound by the VALU (the tests and the BSDF
+// terms) as long as the photons, which neighbouring queries share, stay in the
+// caches: so exactly 4 waves per SIMD, all of the grid resident, each XCD's share of
+// the list contiguous.  Nine passes of 4M photons on the 1920x1080 caustic box
+// (7.5M queries of 1,100 candidates), first and last, this kernel: 5 waves 123.2 ..
+// 46.2 ms, 6 waves 126.7 .. 48.9, 4 waves and 4096 blocks in launch order 118.2 ..
+// 44.3, as here 113.2 .. 43.6.  With kSppmGather 597 ms in all, 641 when one kernel
+// ran all the queries of its 64 pixels, 650 with whole tasks left and 5 waves.
+constexpr uint32_t kSharedWaves = 4, kSharedBlocks = 256 * kSharedWaves;
 template <class Sum>
-__global__ void __launch_bounds__(kB) HASTY_SPPM_GATHER_ATTR kSppmGatherShared(DevScene s, SppmDev g,
-                                                                              const uint32_t* tasks) {
+__global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(kSharedWaves, kSharedWaves)))
+    kSppmGatherShared(DevScene s, SppmDev g, const uint32_t* heavy) {
   __shared__ uint2 gatherRuns[kB];
   __shared__ uint32_t gatherFound[2 * kB];
-  const uint32_t P = s.width * s.height, groups = (P + 63u) / 64u;
-  const uint32_t parts = 64u / kShareQueries, n = g.counters[kCtrShared] * parts;
-  const uint32_t waves = gridDim.x * (kB / 64);
-  unsigned long long nFound = 0;
-  for (uint32_t k = __builtin_amdgcn_readfirstlane((blockIdx.x * kB + threadIdx.x) >> 6); k < n; k += waves) {
-    const uint32_t t = tasks[k / parts], v = t / groups;
-    const uint32_t first = (t - v * groups) * 64u + (k % parts) * kShareQueries;
-    for (uint32_t p = first; p < min(first + kShareQueries, P); ++p) {
-      if (v >= g.nq[p]) continue;
-      float4* qr = g.query + 4 * ((size_t)v * P + p);
-      const float4 q0 = qr[0], q1 = qr[1], q2 = qr[2];
-      int M = 0;
-      bool saturated;
-      const V3 est = sharedGather<Sum>(g, s, f4xyz(q0), f4xyz(q1), f4xyz(q2), __float_as_int(q0.w), pixelRadius(g, p),
-                                       &M, gatherRuns + (threadIdx.x & ~63u), gatherFound + 2u * (threadIdx.x & ~63u),
-                                       &saturated);
-      if ((threadIdx.x & 63u) == 0) {
-        qr[0] = f4(est, __int_as_float(M));
-        if (saturated) atomicAdd(&g.counters[kCtrFluxOverflow], 1u);
-      }
-      nFound += (unsigned long long)M;
+  const uint32_t P = s.width * s.height, n = g.counters[kCtrShared], waves = gridDim.x * (kB / 64);
+  unsigned long long nCand = 0, nFound = 0;
+  for (uint32_t k = __builtin_amdgcn_readfirstlane((xcdRemap() * kB + threadIdx.x) >> 6); k < n; k += waves) {
+    const uint32_t q = heavy[k];
+    float4* qr = g.query + 4 * (size_t)q;
+    const float4 q0 = qr[0], q1 = qr[1], q2 = qr[2];
+    int M = 0;
+    bool saturated;
+    uint32_t cand;
+    const V3 est = sharedGather<Sum>(g, s, f4xyz(q0), f4xyz(q1), f4xyz(q2), __float_as_int(q0.w),
+                                     pixelRadius(g, q % P), &M, gatherRuns + (threadIdx.x & ~63u),
+                                     gatherFound + 2u * (threadIdx.x & ~63u), &saturated, &cand);
+    if ((threadIdx.x & 63u) == 0) {
+      qr[0] = f4(est, __int_as_float(M));
+      if (saturated) atomicAdd(&g.counters[kCtrFluxOverflow], 1u);
     }
+    nCand += cand;
+    nFound += (unsigned long long)M;
   }
-  if ((threadIdx.x & 63u) == 0 && nFound) atomicAdd(&g.gatherStats[2], nFound);
+  if ((threadIdx.x & 63u) == 0 && nCand) {
+    atomicAdd(&g.gatherStats[1], nCand);
+    atomicAdd(&g.gatherStats[2], nFound);
+  }
 }
 
 // The pixels' statistics: F_R = sum over the vertices in path order of
@@ -1478,7 +1496,8 @@ SppmRenderer::SppmRenderer(const DevScene& scene, const SppmParams& params, cons
   // gather queries: at most one per path depth and pixel
   dQuery_ = alloc<float4>((size_t)4 * std::max(1, s_.maxDepth) * P);
   dNq_ = alloc<uint32_t>(P);
-  dTasks_ = alloc<uint32_t>((P + 63) / 64 * (size_t)std::max(1, s_.maxDepth));
+  // (each query has 64 B of its own: fewer than 2^32 fit the device)
+  dHeavy_ = alloc<uint32_t>((size_t)std::max(1, s_.maxDepth) * P);
   dLpath_ = alloc<float>(3 * P);
   dCounters_ = alloc<uint32_t>(kNumCtr + kCameraSegments);
   dCamera_ = alloc<float4>(2 * 9 * P);
@@ -1776,11 +1795,13 @@ void SppmRenderer::pass(uint32_t passIndex, float offX, float offY, float* dColo
   const size_t gatherTasks = (P + 63) / 64 * (size_t)std::max(1, s_.maxDepth);
   const dim3 gatherGrid((uint32_t)std::min<size_t>((gatherTasks + 3) / 4, 4096));
   if (p_.fixedPointFlux) {
-    hipLaunchKernelGGL(kSppmGather<FixedSum>, gatherGrid, dim3(kB), 0, stream_, s_, g, dTasks_);
-    hipLaunchKernelGGL(kSppmGatherShared<FixedSum>, dim3(4096), dim3(kB), 0, stream_, s_, g, (const uint32_t*)dTasks_);
+    hipLaunchKernelGGL(kSppmGather<FixedSum>, gatherGrid, dim3(kB), 0, stream_, s_, g, dHeavy_);
+    hipLaunchKernelGGL(kSppmGatherShared<FixedSum>, dim3(kSharedBlocks), dim3(kB), 0, stream_, s_, g,
+                       (const uint32_t*)dHeavy_);
   } else {
-    hipLaunchKernelGGL(kSppmGather<FloatSum>, gatherGrid, dim3(kB), 0, stream_, s_, g, dTasks_);
-    hipLaunchKernelGGL(kSppmGatherShared<FloatSum>, dim3(4096), dim3(kB), 0, stream_, s_, g, (const uint32_t*)dTasks_);
+    hipLaunchKernelGGL(kSppmGather<FloatSum>, gatherGrid, dim3(kB), 0, stream_, s_, g, dHeavy_);
+    hipLaunchKernelGGL(kSppmGatherShared<FloatSum>, dim3(kSharedBlocks), dim3(kB), 0, stream_, s_, g,
+                       (const uint32_t*)dHeavy_);
   }
   hipLaunchKernelGGL(kSppmUpdate, dim3((uint32_t)std::min<size_t>((P + kB - 1) / kB, 16384)), dim3(kB), 0, stream_, s_,
                      g, p_.alpha, (int)emitted, dColor);

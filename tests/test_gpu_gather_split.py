@@ -37,3 +37,29 @@ def test_gather_forms_agree(size, fixed):
                 assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
             else:
                 np.testing.assert_allclose(a, b, rtol=1e-4, atol=1e-6)
+
+
+@pytest.mark.parametrize("fixed", [True, False])
+@pytest.mark.parametrize("limit", [0, 3, 40, 1000])
+def test_light_and_heavy_queries_of_one_wave(limit, fixed):
+    """Where some of a wave's 64 queries have more candidates than the limit and
+    some have not, the wave gathers the light ones and leaves the heavy ones:
+    counts are those of every query gathered by its lane, and so is the flux
+    (to FP32 summation error, as above)."""
+    d = scenes.write_caustic_scene("", width=97, height=61, n_major=60, n_minor=24, max_depth=8, as_desc=True)
+    sc = ha.Scene.create(**d)
+    outs = []
+    for share in (1 << 30, limit):
+        sp = ha.Sppm(sc, 4, initial_radius=0.25, store_fraction=2.0, emit_fraction=80.0, fixed_point_flux=fixed,
+                     gather_share_candidates=share)
+        films = [sp.pass_(k)[0].copy() for k in range(3)]
+        i = sp.info()
+        outs.append((films, (i["gather_queries"], i["gather_candidates"], i["gather_found"]), sp.pixels()["N"]))
+    (ref, counts, n_ref), (got, counts2, n_got) = outs
+    assert counts == counts2 and counts[2] > 0
+    assert np.array_equal(n_ref, n_got)
+    for a, b in zip(ref, got):
+        if fixed:
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+        else:
+            np.testing.assert_allclose(a, b, rtol=1e-4, atol=1e-6)
