@@ -1521,7 +1521,7 @@ static int autotuneItems(std::vector<BatchItem> items, uint32_t trialSamples, Ha
     hasty_set_launch_ex(owner, &best);
     timeIt();  // warm-up (allocations)
     double bestT = timeIt();
-    const std::vector<uint32_t> slots = {1u << 20, 1u << 21, 1u << 22, 1u << 23};
+    const std::vector<uint32_t> slots(std::begin(hasty::kTunedSlots), std::end(hasty::kTunedSlots));
     const std::vector<uint32_t> trace = {1024, 2048, 4096};
     const std::vector<uint32_t> shade = {2048, 4096, 8192};
     const std::vector<uint32_t> chunks = {4, 8, 16};

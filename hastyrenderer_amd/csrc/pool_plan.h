@@ -9,6 +9,9 @@
 namespace hasty {
 
 constexpr uint32_t kDefaultSlots = 1u << 24;
+// Pools the autotuner tries, up to the default (a larger one is faster still,
+// see poolPaths, but a pool is kept once it is allocated, 5 GB at 2^24).
+constexpr uint32_t kTunedSlots[] = {1u << 20, 1u << 21, 1u << 22, 1u << 23, kDefaultSlots};
 
 // What the jobs of a call add up to.
 struct PoolNeed {

@@ -18,6 +18,13 @@ void tk_pool_sizes(const uint32_t* samples, const uint64_t* pixels, uint32_t n, 
   out3[2] = hasty::recordPaths(need, wanted);
 }
 
+// The pools the autotuner tries; returns how many.
+uint32_t tk_tuned_slots(uint32_t* out8) {
+  uint32_t n = 0;
+  for (uint32_t s : hasty::kTunedSlots) out8[n++] = s;
+  return n;
+}
+
 // allocHalving on a device with `freeBytes` free, whose allocation number
 // `errorAt` (from 1; 0: none) fails with another error.  Returns 0, 1 when out
 // of memory, 2 for the other error; out: paths, ring, allocations asked for.

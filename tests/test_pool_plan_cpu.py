@@ -49,6 +49,15 @@ def test_training_records_are_bounded():
     assert _sizes([(1, 5)], wanted=7)[2] == 5
 
 
+def test_autotuner_tries_the_default_pool():
+    """A scene whose pool was set smaller can be tuned back to what an untuned
+    scene has."""
+    out = np.zeros(8, np.uint32)
+    n = load_testkernels().tk_tuned_slots(out.ctypes.data_as(C.c_void_p))
+    tried = [int(x) for x in out[:n]]
+    assert _sizes([(1, 1 << 30)])[0] in tried and tried == sorted(tried)
+
+
 def _halving(paths, ring, film, free, error_at=0):
     L = load_testkernels()
     out = np.zeros(3, np.uint32)
