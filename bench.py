@@ -17,7 +17,9 @@ extension and shadow rays): its algorithmic bytes per launch are the canonical
 per-ray bytes (64 B per BVH2 node visit + 48 B per triangle test, counted by
 the CPU oracle's binned-SAH BVH2 over 2^16 paths) plus the 48 B of ray and hit
 records each ray moves, times the rays one launch processes; divided by the
-launch's average duration from HIP events on the library's stream.
+launch's average duration from HIP events on the library's stream.  (A shadow
+ray is charged as an extension ray: most go to the sky, find no blocker and walk
+10.2 nodes against 9.1, see "traversal".)
 
 cpu_baseline: the oracle (the project's C++ restatement of the reference path
 tracer) timed on the host on 48 passes (48 spp) of the same 1024x1024 workload.
@@ -25,7 +27,10 @@ tracer) timed on the host on 48 passes (48 spp) of the same 1024x1024 workload.
 roofline.traffic: HBM bytes per pt_trace launch measured by rocprofv3
 FETCH_SIZE and WRITE_SIZE runs, scaled by the factor the same counters read
 for a plain copy of known size (--copy-calibration); read from the committed
-summary in profiles/ when present.
+summary in profiles/ when present.  traffic_frac is that traffic over the launch's
+average duration, as a share of the peak.  The caches serve most of the
+algorithmic bytes, so frac may pass 1; traffic_frac is what says how far the HBM
+is from its limit.
 
 Other workloads (not the headline line): --workload sppm times photon-mapping
 passes on the caustic box (prism + 2M-triangle torus, 1920x1080);
@@ -704,13 +709,15 @@ def main():
         bytes_per_launch = rays_per_launch * (b_ray + STATE_BYTES_PER_RAY)
         avg_s = trace_ms / launches / 1e3
         achieved = bytes_per_launch / avg_s / 1e9
+        traffic = measured_traffic()
         roofline = {
             "bound": "hbm",
             "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
-            "traffic": measured_traffic(),
+            "traffic": traffic,
+            "traffic_frac": round(traffic / avg_s / 1e9 / HBM_PEAK_GBS, 4) if traffic else None,
             "traffic_source": "rocprofv3 FETCH_SIZE/WRITE_SIZE of an earlier run of this command, read from "
                               "profiles/pt_trace_ggx_grid_1024_traffic.md (not measured in this run)",
             "kernel": "pt_trace",
