@@ -23,7 +23,10 @@ struct SppmParams {
   float gatherUnionFactor = 0.0f;      // > 0: union gathers (see kSppmGather); 0: off
 };
 
-constexpr int kSppmCasterBoxes = 32;  // boxes around the surfaces that bounce photons
+// Boxes around the surfaces that bounce photons: more select fewer photons and
+// take longer to test.  8, 16, 32, 64, 128 on the 960x540 caustic box: 12, 8, 7, 6,
+// 6 % selected, 1.08, 0.79, 0.83, 0.97, 1.28 ms of photon tracing a pass.
+constexpr int kSppmCasterBoxes = 32;
 
 struct SppmPassInfo {
   uint64_t emitted = 0, stored = 0;

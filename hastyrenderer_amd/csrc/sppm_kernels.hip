@@ -6,16 +6,20 @@
 // One pass:
 //   1. cell size: three deterministic reductions over the radius image
 //      (mean; eleven growing candidates; ten shrinking candidates);
-//   2. photons: batches of photon indices traced in parallel, each thread
-//      keeping its stored photons in private slots; a scan of the per-thread
-//      counts decides where the sequential emission loop of the reference
-//      stops (fewer than storeLimit stored, fewer than emitLimit emitted)
-//      and compacts the emitted photons in emission order;
+//   2. photons: in batches of photon indices, the photons whose ray meets a box
+//      around the surfaces that bounce photons are listed (all of them where
+//      that would be most) and traced, each into slots of its own; a scan of
+//      the photons' stored counts decides where the sequential emission loop of
+//      the reference stops (fewer than storeLimit stored, fewer than emitLimit
+//      emitted) and compacts the emitted photons in emission order;
 //   3. cells: 63-bit packed cell keys, stable radix sort (key, emission
 //      index), cell table (open addressing, key -> first, count);
-//   4. camera: one thread per pixel runs the whole MIS path with gathers in
-//      the reference's cell order (x, then y, then z; photons of a cell in
-//      emission order) and applies the pixel statistics update.
+//   4. camera: MIS paths in segments of vertices, packed between them, that
+//      record a query at every diffuse vertex;
+//   5. gathers: a lane per query in the reference's cell order (x, then y, then
+//      z; photons of a cell in emission order), a wave per query where many
+//      photons are near;
+//   6. the pixels' statistics update, from their gathers in path order.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -693,8 +697,8 @@ __device__ inline void photonRun(const SppmDev& g, uint32_t first, uint32_t end,
 // Queries with at most g.coopCandidates candidates (default 128) are gathered
 // by a lane each: a longer list is a chain of loads that the other lanes wait
 // for, while a shared gather costs a wave per query.  Passes of the caustic box
-// with 32, 64, 128, 256, 512: 4.94, 4.89, 4.83, 4.84, 4.81 ms (sparse map,
-// 960x540) and 9.68, 9.69, 9.69, 9.97, 10.99 ms (dense map, 640x360).
+// with 32, 64, 128, 256, 512: 4.18, 4.17, 4.13, 4.08, 4.08 ms (sparse map,
+// 960x540) and 8.22, 8.11, 8.41, 8.90, 9.87 ms (dense map, 640x360).
 constexpr uint32_t kCoopCandidatesDefault = 128;
 // Where a query of the wave is over that limit, those over a third of it are left
 // as well: few lanes would walk their lists while the others, whose queries are
@@ -1680,16 +1684,21 @@ void SppmRenderer::pass(uint32_t passIndex, float offX, float offY, float* dColo
   if (s_.hasSurfaceLight) {
     // Photons to emit for what is still to be stored, at the store rate seen
     // so far (this pass's, else the last one's), with a margin for its spread:
-    // one batch a pass as a rule, since each ends with the tail of its longest
-    // light paths (0.3 to 0.5 ms).  Before any photon is stored, one for each to
-    // store, then four times those emitted.
+    // one batch a pass where it emits no more than batchMax_ (2^25) photons,
+    // since each ends with the tail of its longest light paths (0.3 to 0.5 ms).
+    // Before any photon is stored, one for each to store, then four times those
+    // emitted.
     double rate = storeRate_;
     while (stored < storeLimit_ && next < emitLimit_) {
       const double left = (double)(storeLimit_ - stored);
       const double want = rate > 0.0 ? 1.01 * (left + 4.0 * std::sqrt(left) + 64.0) / rate
                                      : std::max(left, 4.0 * (double)emitted);
       uint32_t batch = (uint32_t)std::min<double>(emitLimit_ - next, std::max(65536.0, want));
-      const bool select = selectRate_ < 0.75;  // above, selecting costs what it saves
+      // Selecting saves what it leaves untraced and costs the emission twice:
+      // where 7 % of the photons are selected 0.83 ms against 1.98 for tracing all,
+      // 49 % 1.07 against 1.21, all of them 0.61 against 0.57 (960x540 caustic
+      // box, more of its surfaces glossy each time); even at about four fifths.
+      const bool select = selectRate_ < 0.75;
       // what the list of photons to trace may take, with a margin
       batch = (uint32_t)std::min<double>(batch, select ? std::min<double>(batchMax_, 0.9 * slots_ / selectRate_)
                                                        : (double)slots_);

@@ -254,7 +254,14 @@ int hasty_counters_ex(HastyScene* scene, uint64_t* out, uint32_t n);
 /* Launch-shape knobs: path slots in flight (paths are regenerated into
  * freed slots; default 2^24, at least 2^16 unless the film is smaller) and
  * the grid sizes of the traversal and shading kernels.  0 keeps the current
- * value.  Images do not depend on these. */
+ * value.  Images do not depend on these.
+ *
+ * The slots are an upper limit: no more are allocated than a render has paths,
+ * and fewer where the device is short of memory.  A scene holds about 300 B a
+ * slot (404 with both a sky and light triangles, 64 more with textured media)
+ * and, whatever the slots, 48 B for each of up to 2^27 finished paths (at least
+ * one sample of the film): 11.5 GB for a large render at the default, until it is
+ * destroyed. */
 int hasty_set_launch(HastyScene* scene, uint32_t path_slots, uint32_t trace_blocks, uint32_t shade_blocks);
 
 /* Launch configuration of a scene's path pool (also used for batches whose
@@ -264,7 +271,7 @@ int hasty_set_launch(HastyScene* scene, uint32_t path_slots, uint32_t trace_bloc
  * uploaded the first time it is asked for; images do not depend on it).
  * Fields that are 0 keep their value (except use_graph). */
 typedef struct HastyLaunch {
-  uint32_t path_slots;
+  uint32_t path_slots; /* hasty_get_launch: as set, or the default */
   uint32_t trace_blocks;
   uint32_t shade_blocks;
   uint32_t chunk;
@@ -396,10 +403,10 @@ typedef struct HastySppmParams {
    * is counted in HastySppmInfo.flux_overflows.  Default 0 (FP32). */
   int32_t fixed_point_flux;
   int32_t flux_frac_bits;            /* 0: 24; at most 40 */
-  uint32_t gather_share_candidates;  /* 0: 128; a wave gathers its queries together when one of them has
-                                        more candidate photons than this (no effect on the result with
-                                        fixed-point flux) */
-  float gather_union_factor;         /* > 0: such a wave reads the union of its queries' cells once, each
+  uint32_t gather_share_candidates;  /* 0: 128; a query with more candidate photons than this is gathered
+                                        by a whole wave, and so are those of its 64 pixels with more than a
+                                        third of it (no effect on the result with fixed-point flux) */
+  float gather_union_factor;         /* > 0: a wave with such a query reads the union of its queries' cells once, each
                                         lane summing its own photons in the reference's order (FP32 results
                                         of the per-lane gather), when the union box holds at most this x the
                                         queries' mean cells; 0 (default): the shared gather, faster on dense
