@@ -571,10 +571,10 @@ __device__ inline uint2 cellLookup(const SppmDev& g, unsigned long long key) {
 // photons of a cell in emission order, |x - c|^2 <= r^2; the BSDF is the
 // diffuse lobe only with outside IOR 1.
 //
-// When some query of 64 consecutive pixels has many candidate photons (dense
-// maps, large radii), those queries are gathered one at a time by the 64
-// lanes of a wave (sharedGather), every lane testing a share of the query's
-// photons, and the lanes' partial sums are added by a butterfly over the wave.
+// A query with many candidate photons (dense maps, large radii) is gathered by
+// the 64 lanes of a wave (sharedGather), every lane testing a share of the
+// query's photons, and the lanes' partial sums are added by a butterfly over the
+// wave.
 // The set and the count of photons are the reference's; only the FP32
 // association of the flux sum differs, the same way on every run.  Otherwise
 // each lane sums its own photons in the reference's order.
